@@ -2542,7 +2542,7 @@ int band_factor (sx_msys* s, hipStream_t st, int* d_status)
   return SX_OK;
 }
 
-int band_solve (const sx_msys* s, int nr, hipStream_t st, int moves)
+static int band_sweeps (const sx_msys* s, int nr, hipStream_t st, int moves)
 {
   if (s->sw_panel) {
     // right-hand sides per workgroup: SX_PANEL_NR in the environment, else
@@ -2655,6 +2655,15 @@ int band_solve (const sx_msys* s, int nr, hipStream_t st, int moves)
   set_error ("band solver: band width " + std::to_string (s->m->nband) +
              " outside the instantiated range (nband <= 768)");
   return SX_ERR_LIMIT;
+}
+
+int band_solve (const sx_msys* s, int nr, hipStream_t st, int moves)
+{
+  if (s->use_tree) return tree_solve (s, nr, st);
+  if (!s->sing) return band_sweeps (s, nr, st, moves);
+  int rc;
+  if ((rc = sing_keep (s, nr, st)) || (rc = band_sweeps (s, nr, st, 3))) return rc;
+  return sing_refine (s, nr, st);
 }
 
 // ---------------------------------------------------------------------------

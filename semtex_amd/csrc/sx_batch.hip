@@ -263,6 +263,9 @@ extern "C" int sx_batch_create (int n, const sx_msys_t* systems, const int* nz,
       return SX_ERR_ARG;
     }
   *out = nullptr;
+  // the recorded solves are band sweeps: so are the systems' own from here
+  for (int i = 0; i < n; i++)
+    if (int rc = msys_use_band (systems[i])) return rc;
   sx_batch* b = new sx_batch;
   b->n = n;
   auto fail = [&] (int r) { sx_batch_destroy (b); return r; };

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -38,8 +39,30 @@ void side_area (int np, const double* x, const double* y, int side,
 
 }  // namespace sx
 
+struct sx_mesh;
 struct sx_msys;
 namespace sx {
+// Dissection solve of the condensed systems -- sx_tree.hip.  tree_prepare:
+// the mesh's plan for a mode count (kept with the mesh), null when the band
+// solve is to be used; tree_factor: from the condensed element matrices;
+// tree_solve: from the assembled right-hand sides in rhs_in (s) to d_rhs.
+struct TreeDev;
+struct TreeSing;
+int    tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always = false);
+void   tree_free (TreeDev* t);
+void   tree_sing_free (TreeSing* g);
+int    tree_workspace (sx_msys* s, int nr);
+int    tree_factor (sx_msys* s, const double* Sel, hipStream_t st, int* d_status);
+int    tree_solve (const sx_msys* s, int nr, hipStream_t st);
+// A singular mode's refinement: its set-up (s->sing), and around a band
+// solve the right-hand sides kept before and the correction after.
+int    tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_status);
+int    sing_keep (const sx_msys* s, int nr, hipStream_t st);
+int    sing_refine (const sx_msys* s, int nr, hipStream_t st);
+// A system's band factor (built on first use where the system solves by
+// dissection) and its use from now on: the batches plan band sweeps, and
+// their systems' own solves stay equal to the batch's (sx_solver.hip).
+int    msys_use_band (sx_msys* s);
 // Banded FP64 Cholesky of every mode's band, the offset-major sweep copies
 // of the factor and of its reversal (with inverted diagonal blocks), and
 // the two-sweep solve of the right-hand sides in d_rhs ([mode][2][nmax])
@@ -155,6 +178,13 @@ struct sx_mesh {
   // the element count, 2 unused, the ETILE element numbers (the last one
   // repeated past the count), their emask, then their btog and bmask rows
   int* d_ttab = nullptr;
+  // dissection plans, one per mode count met (sx_tree.hip)
+  std::mutex tree_mu;
+  std::vector<sx::TreeDev*> trees;
+  // meshes without essential nodes: the assembled matrix by rows (columns
+  // and pair numbers, both triangles), for a singular mode's residual
+  std::vector<int> pmn;        // [npairs][2] host copy of d_pmn
+  int *d_sptr = nullptr, *d_scol = nullptr, *d_spair = nullptr;
 };
 constexpr int ETILE = 16;
 constexpr int TT_EL = 4, TT_EM = TT_EL + ETILE, TT_BT = TT_EM + ETILE;
@@ -189,8 +219,8 @@ struct sx_msys {
   unsigned* d_xep = nullptr;   //   [4] epoch, arrivals, status (bit 0: a wait gave up)
   size_t xch_bytes = 0;
   // the panel sweep kernel of the last band solve (diagnostic): 0 none,
-  // 1 k_panel_sweeps, 2 k_unit_sweeps, 3 k_split_sweeps; right-hand sides
-  // per workgroup
+  // 1 k_panel_sweeps, 2 k_unit_sweeps, 3 k_split_sweeps (right-hand sides
+  // per workgroup), 4 the dissection solve (right-hand sides per mode)
   mutable int last_kernel = 0, last_nr = 0;
   // 1: solves may run concurrently with other kernels (a batch graph's
   // branches), so the split sweeps, which need their whole grid resident,
@@ -205,6 +235,13 @@ struct sx_msys {
   int* d_tw = nullptr;         //   [nmodes][8] split of every mode
   double* d_rhsb = nullptr;    //   [nmodes][nr][nmaxb] bottom-piece right-hand sides
   int nmaxb = 0;
+  sx::TreeDev* tree = nullptr; // dissection solve: the mesh's plan, null: band only
+  int use_tree = 0;            //   solves run it
+  sx::TreeSing* sing = nullptr;  // the singular mode's refinement, or null
+  double* d_tops = nullptr;    //   operators [nmodes][ops]
+  double* d_tb = nullptr;      //   assembled right-hand sides by position [nmodes][nr][nsolve]
+  double* d_tv = nullptr;      //   fronts' eliminated parts [nmodes][nr][nsolve]
+  double* d_tc = nullptr;      //   fronts' boundary contributions [nmodes][nr][slots]
   double* d_rhs = nullptr;     // [nmodes][nr][nmax] solve workspace (nr <= rhs_cap)
   double* d_G = nullptr;       // [fields][2*nmodes][nglobal] essential values
   int rhs_cap = 2;             // right-hand sides per mode d_rhs / d_G can hold
@@ -212,6 +249,18 @@ struct sx_msys {
   double* d_pc = nullptr;      // SX_JACPCG: [nmodes][npts] inverse assembled diagonal
   size_t work_doubles = 0;
 };
+// where the assembly writes a solve's right-hand sides: [mode][nr][ld], node
+// g at perm[g] (perm null: at g).  The dissection solve reads them by
+// position and writes the solution to d_rhs by node.
+namespace sx {
+const int* tree_perm (const sx_msys* s);
+struct RhsTo { double* p; int ld; const int* perm; };
+inline RhsTo rhs_in (const sx_msys* s)
+{
+  return s->use_tree ? RhsTo {s->d_tb, s->m->nsolve, tree_perm (s)}
+                     : RhsTo {s->d_rhs, s->nmax, nullptr};
+}
+}
 
 // ---------------------------------------------------------------------------
 // Fused batches (sx_batch.hip).  A batch of independent solves is planned

@@ -309,7 +309,7 @@ __device__ __forceinline__ void k_assemble_m_body (int nglobal, const int* __res
                               const double* __restrict__ F, int stride,
                               const double* __restrict__ lines, int lstride,
                               const int* __restrict__ nsolve, double* rhs, int nmax,
-                              int nz, int base_mode)
+                              int nz, int base_mode, const int* __restrict__ perm)
 {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const int k = solved_plane (blockIdx.y, nz, base_mode);
@@ -320,7 +320,7 @@ __device__ __forceinline__ void k_assemble_m_body (int nglobal, const int* __res
   for (int c = gptr[g]; c < gptr[g + 1]; c++) s += Fk[gsrc[c]];
   if (lines)
     for (int c = nptr[g]; c < nptr[g + 1]; c++) s += lines[(size_t) k * lstride + nidx[c]] * nw[c];
-  rhs[((size_t) mode * 2 + rr) * nmax + g] = s;
+  rhs[((size_t) mode * 2 + rr) * nmax + (perm ? perm[g] : g)] = s;
 }
 
 __global__ void k_assemble_m (int nglobal, const int* __restrict__ gptr,
@@ -329,9 +329,9 @@ __global__ void k_assemble_m (int nglobal, const int* __restrict__ gptr,
                               const double* __restrict__ F, int stride,
                               const double* __restrict__ lines, int lstride,
                               const int* __restrict__ nsolve, double* rhs, int nmax,
-                              int nz, int base_mode)
+                              int nz, int base_mode, const int* __restrict__ perm)
 {
-  k_assemble_m_body (nglobal, gptr, gsrc, nptr, nidx, nw, F, stride, lines, lstride, nsolve, rhs, nmax, nz, base_mode);
+  k_assemble_m_body (nglobal, gptr, gsrc, nptr, nidx, nw, F, stride, lines, lstride, nsolve, rhs, nmax, nz, base_mode, perm);
 }
 
 int inner_solve (sx_msys* s, int nz, int stride, const double* X, double* Fp,
@@ -346,10 +346,11 @@ int inner_solve (sx_msys* s, int nz, int stride, const double* X, double* Fp,
     hipLaunchKernelGGL (k_condense32, dim3 (m->nel, npl), dim3 (64), 0, st, m->np, m->nclass,
                         m->d_emap, m->d_cls, s->d_Bm32, X, Fp, stride, nz, s->base_mode);
   }
+  const RhsTo to = rhs_in (s);
   hipLaunchKernelGGL (k_assemble_m, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw, Fp,
-                      stride, lines, lstride, s->d_nsolve, s->d_rhs, s->nmax, nz,
-                      s->base_mode);
+                      stride, lines, lstride, s->d_nsolve, to.p, to.ld, nz, s->base_mode,
+                      to.perm);
   SX_HIP (hipGetLastError ());
   int rc = band_solve (s, 2, st);
   if (rc) return rc;
@@ -407,7 +408,7 @@ int plan_inner (BatchPlan& P, sx_msys* s, int nz, int stride, const double* X, d
                                (const int*) m->d_nptr, (const int*) m->d_nidx,
                                (const double*) m->d_nw, (const double*) Fp, stride, lines,
                                lstride, (const int*) s->d_nsolve, s->d_rhs, s->nmax, nz,
-                               s->base_mode);
+                               s->base_mode, (const int*) nullptr);
   P.phase++;
   if (int rc = plan_band_solve (P, s, 2)) return rc;
   if (tiled) return plan_recover32_tiled (P, s, nz, stride, Fp, V);

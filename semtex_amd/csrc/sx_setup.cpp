@@ -220,8 +220,10 @@ extern "C" int sx_mesh_destroy (sx_mesh_t m)
                   m->d_emask, m->d_emap, m->d_gptr, m->d_gsrc, m->d_ess,
                   m->d_nptr, m->d_nidx, m->d_nw, m->d_ppos, m->d_pmn,
                   m->d_pptr, m->d_psrc, m->d_tile, m->d_elist, m->d_ess_elem,
-                  m->d_ttab, m->d_ess_slot, m->d_gpos, m->d_gq4};
+                  m->d_ttab, m->d_ess_slot, m->d_gpos, m->d_gq4,
+                  m->d_sptr, m->d_scol, m->d_spair};
   for (void* p : ptrs) if (p) (void) hipFree (p);
+  for (TreeDev* t : m->trees) tree_free (t);
   delete m;
   return SX_OK;
 }
@@ -397,6 +399,7 @@ extern "C" int sx_mesh_create (int np, int nel, int cyl, const double* x,
     pptr.push_back ((int) psrc.size ());
   }
   m->npairs = (int) ppos.size ();
+  if (nglobal == nsolve) m->pmn = pmn;
 
   // class-sorted element tiles and the elements with essential nodes
   std::vector<int> elist, tile, ess_elem;

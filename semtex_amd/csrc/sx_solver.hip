@@ -1321,7 +1321,8 @@ __device__ __forceinline__ void k_assemble_body (int nglobal, const int* __restr
                             const double* __restrict__ F, int stride,
                             const double* __restrict__ lines, int lstride,
                             const int* __restrict__ nsolve, double* rhs,
-                            int nmax, int nz, int base_mode, int rnr, int roff)
+                            int nmax, int nz, int base_mode, int rnr, int roff,
+                            const int* __restrict__ perm)
 {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const int k = solved_plane (blockIdx.y, nz, base_mode);
@@ -1333,7 +1334,7 @@ __device__ __forceinline__ void k_assemble_body (int nglobal, const int* __restr
   if (lines)
     for (int c = nptr[g]; c < nptr[g + 1]; c++)
       s += lines[(size_t) k * lstride + nidx[c]] * nw[c];
-  rhs[((size_t) mode * rnr + rr) * nmax + g] = s;
+  rhs[((size_t) mode * rnr + rr) * nmax + (perm ? perm[g] : g)] = s;
 }
 
 __global__ void k_assemble (int nglobal, const int* __restrict__ gptr,
@@ -1344,9 +1345,10 @@ __global__ void k_assemble (int nglobal, const int* __restrict__ gptr,
                             const double* __restrict__ F, int stride,
                             const double* __restrict__ lines, int lstride,
                             const int* __restrict__ nsolve, double* rhs,
-                            int nmax, int nz, int base_mode, int rnr, int roff)
+                            int nmax, int nz, int base_mode, int rnr, int roff,
+                            const int* __restrict__ perm)
 {
-  k_assemble_body (nglobal, gptr, gsrc, nptr, nidx, nw, F, stride, lines, lstride, nsolve, rhs, nmax, nz, base_mode, rnr, roff);
+  k_assemble_body (nglobal, gptr, gsrc, nptr, nidx, nw, F, stride, lines, lstride, nsolve, rhs, nmax, nz, base_mode, rnr, roff, perm);
 }
 
 // Assembly for a twisted system that also writes the bottom piece's
@@ -1363,7 +1365,7 @@ __global__ void k_assemble_tw (int nglobal, const int* __restrict__ gptr,
                                double* rhsb, int nmaxb, int S)
 {
   k_assemble_body (nglobal, gptr, gsrc, nptr, nidx, nw, F, stride, lines, lstride, nsolve, rhs,
-                   nmax, nz, base_mode, rnr, 0);
+                   nmax, nz, base_mode, rnr, 0, nullptr);
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   const int k = solved_plane (blockIdx.y, nz, base_mode);
   const int mode = k >> 1;
@@ -1382,11 +1384,11 @@ __global__ void k_assemble3 (int nglobal, const int* __restrict__ gptr,
                              const int* __restrict__ nidx, const double* __restrict__ nw,
                              FieldSet fs, int stride, int lstride,
                              const int* __restrict__ nsolve, double* rhs, int nmax, int nz,
-                             int base_mode, int rnr)
+                             int base_mode, int rnr, const int* __restrict__ perm)
 {
   k_assemble_body (nglobal, gptr, gsrc, nptr, nidx, nw, fs.F[blockIdx.z], stride,
                    fs.lines[blockIdx.z], lstride, nsolve, rhs, nmax, nz, base_mode, rnr,
-                   2 * blockIdx.z);
+                   2 * blockIdx.z, perm);
 }
 
 // One wavefront per (element, solved plane): interior recovery and
@@ -1522,8 +1524,10 @@ extern "C" int sx_msys_destroy (sx_msys_t s)
   void* ptrs[] = {s->d_betak2, s->d_nsolve, s->d_Bm, s->d_Hinv, s->d_Mrec, s->d_Mcon,
                   s->d_Mrec32, s->d_Mcon32, s->d_Bm32,
                   s->d_Hinv32, s->d_bandU, s->d_swF, s->d_swR, s->d_rhs, s->d_G,
-                  s->d_work, s->d_pc, s->d_tw, s->d_rhsb, s->d_xch, s->d_xep};
+                  s->d_work, s->d_pc, s->d_tw, s->d_rhsb, s->d_xch, s->d_xep,
+                  s->d_tops, s->d_tb, s->d_tv, s->d_tc};
   for (void* p : ptrs) if (p) (void) hipFree (p);
+  tree_sing_free (s->sing);
   delete s;
   return SX_OK;
 }
@@ -1565,6 +1569,66 @@ static double mode_constant (int cyl, char name, int mode, double beta)
   if (mode == 0) return 1.0;
   return name == 'v' ? beta * mode + 1.0 : beta * mode - 1.0;
 }
+
+// The band of every mode assembled from the condensed element matrices and
+// factorised (waits for st).
+static int band_build (sx_msys* s, const double* d_S, hipStream_t st, int* d_status)
+{
+  const sx_mesh* m = s->m;
+  const size_t nb = sizeof (double) * s->nmodes * s->band_stride;
+  SX_HIP (hipMalloc (&s->d_bandU, nb));
+  SX_HIP (hipMemsetAsync (s->d_bandU, 0, nb, st));
+  if (m->npairs)
+    hipLaunchKernelGGL (k_band_assemble, dim3 ((m->npairs + 255) / 256, s->nmodes), dim3 (256), 0,
+                        st, m->npairs, m->d_ppos, m->d_pmn, m->d_pptr, m->d_psrc, d_S,
+                        (size_t) m->nclass * m->next * m->next, s->d_bandU, s->band_stride,
+                        s->d_nsolve);
+  SX_HIP (hipGetLastError ());
+  if (int rc = band_factor (s, st, d_status)) return rc;
+  SX_HIP (hipStreamSynchronize (st));
+  (void) hipFree (s->d_bandU);
+  s->d_bandU = nullptr;
+  return SX_OK;
+}
+
+namespace sx {
+
+int msys_use_band (sx_msys* s)
+{
+  // (the recorded sweeps refine no singular mode either)
+  tree_sing_free (s->sing);
+  s->sing = nullptr;
+  if (!s->use_tree) return SX_OK;
+  const sx_mesh* m = s->m;
+  const int next = m->next, nint = m->nint, npnp = m->npnp;
+  const size_t nmc = (size_t) s->nmodes * m->nclass;
+  const size_t nws = nmc * ((size_t) npnp * npnp + (size_t) nint * nint), nS = nmc * next * next,
+               nB = nmc * next * nint, nH = nmc * nint * nint;
+  // the condensed element matrices again (k_elem_sc forms them with the
+  // element operators, which the system holds already)
+  double* buf = nullptr;
+  int* d_status = nullptr;
+  SX_HIP (hipMalloc (&buf, sizeof (double) * (nws + nS + nB + nH + 1)));
+  int rc = SX_OK;
+  if (hipMalloc (&d_status, sizeof (int) * (s->nmodes + 1)) != hipSuccess ||
+      hipMemset (d_status, 0, sizeof (int) * (s->nmodes + 1)) != hipSuccess) {
+    rc = hip_fail (hipErrorOutOfMemory, "msys_use_band");
+  } else {
+    hipLaunchKernelGGL (k_elem_sc, dim3 ((unsigned) nmc), dim3 (256), 0, nullptr, m->np,
+                        m->nclass, m->cyl, s->lambda2, s->d_betak2, m->d_cgeo, m->d_D, m->d_emap,
+                        buf, buf + nws, buf + nws + nS, buf + nws + nS + nB, d_status + s->nmodes);
+    rc = band_build (s, buf + nws, nullptr, d_status);
+  }
+  (void) hipFree (buf);
+  (void) hipFree (d_status);
+  if (rc) return rc;
+  s->use_tree = 0;
+  // (more than 2 reserved right-hand sides: their bottom-piece workspace
+  // came with the factor, band_factor sizes it by rhs_cap)
+  return SX_OK;
+}
+
+}  // namespace sx
 
 extern "C" int sx_msys_create (sx_mesh_t m, double lambda2, double beta,
                                int base_mode, int num_modes, int precision,
@@ -1617,11 +1681,12 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
   }
   TRY (hipMalloc (&s->d_Bm, sizeof (double) * std::max<size_t> (nmc * next * nint, 1)));
   TRY (hipMalloc (&s->d_Hinv, sizeof (double) * std::max<size_t> (nmc * nint * nint, 1)));
-  TRY (hipMalloc (&s->d_bandU, sizeof (double) * num_modes * s->band_stride));
-  TRY (hipMalloc (&s->d_rhs, sizeof (double) * num_modes * 2 * std::max (s->nmax, 1)));
+  if ((rc = tree_prepare (m, num_modes, &s->tree))) return fail (rc);
+  s->use_tree = s->tree != nullptr;
+  const size_t nrhs = sizeof (double) * num_modes * 2 * std::max (s->nmax, 1);
+  TRY (hipMalloc (&s->d_rhs, nrhs));
   TRY (hipMalloc (&s->d_G, sizeof (double) * 2 * num_modes * m->nglobal));
-  TRY (hipMemsetAsync (s->d_rhs, 0, sizeof (double) * num_modes * 2 * std::max (s->nmax, 1), st));
-  TRY (hipMemsetAsync (s->d_bandU, 0, sizeof (double) * num_modes * s->band_stride, st));
+  TRY (hipMemsetAsync (s->d_rhs, 0, nrhs, st));
 
   double *d_ws = nullptr, *d_S = nullptr;
   int* d_status = nullptr;
@@ -1648,20 +1713,14 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
                         s->d_Mrec, s->d_Mcon);
     TRY (hipGetLastError ());
   }
-  if (m->npairs)
-    hipLaunchKernelGGL (k_band_assemble, dim3 ((m->npairs + 255) / 256, num_modes),
-                        dim3 (256), 0, st, m->npairs, m->d_ppos, m->d_pmn, m->d_pptr,
-                        m->d_psrc, d_S, (size_t) m->nclass * next * next, s->d_bandU,
-                        s->band_stride, s->d_nsolve);
-  TRY (hipGetLastError ());
-  if ((rc = band_factor (s, st, d_status))) return fail (rc);
+  rc = s->use_tree ? tree_factor (s, d_S, st, d_status) : band_build (s, d_S, st, d_status);
+  if (rc || (rc = tree_sing_setup (s, d_S, st, d_status)) || (rc = tree_workspace (s, 2)))
+    return fail (rc);
   std::vector<int> status (num_modes + 1);
   TRY (hipMemcpyAsync (status.data (), d_status, sizeof (int) * (num_modes + 1),
                        hipMemcpyDeviceToHost, st));
   TRY (hipStreamSynchronize (st));
   (void) hipFree (d_ws); (void) hipFree (d_S); (void) hipFree (d_status);
-  (void) hipFree (s->d_bandU);
-  s->d_bandU = nullptr;
   if (status[num_modes]) {
     set_error ("sx_msys_create: matrix hii is not positive definite");
     return fail (SX_ERR_FACTOR);
@@ -1927,6 +1986,7 @@ int field_solve_direct (const sx_msys* s, int nz, int stride, double* d_f, doubl
   const int npl = n_solved_planes (nz, s->base_mode);
   const int lstride = m->nbound * m->np;
   const double* lines = (d_lines && m->nbound) ? d_lines : nullptr;
+  const RhsTo to = rhs_in (s);
   // the essential values and the essential elements' weak form in one
   // launch where the tiled condensation follows
   const bool ew = tiled_ok (m) && m->ness;
@@ -1953,7 +2013,7 @@ int field_solve_direct (const sx_msys* s, int nz, int stride, double* d_f, doubl
   }
   // a twisted system's bottom piece addressed by the assembly and the
   // recovery themselves (no gather and scatter launches around the sweeps)
-  const bool fold = s->tw && s->sw_panel && tiled_ok (m) && s->tile_mf;
+  const bool fold = !s->use_tree && !s->sing && s->tw && s->sw_panel && tiled_ok (m) && s->tile_mf;
   {
     PhaseScope ps (2, st, timed);
     if (fold)
@@ -1964,8 +2024,8 @@ int field_solve_direct (const sx_msys* s, int nz, int stride, double* d_f, doubl
     else
       hipLaunchKernelGGL (k_assemble, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0,
                           st, m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw,
-                          d_f, stride, lines, lstride, s->d_nsolve, s->d_rhs, s->nmax, nz,
-                          s->base_mode, 2, 0);
+                          d_f, stride, lines, lstride, s->d_nsolve, to.p, to.ld, nz, s->base_mode, 2, 0,
+                          to.perm);
   }
   SX_HIP (hipGetLastError ());
   {
@@ -2008,7 +2068,7 @@ int msys_reserve_rhs (sx_msys* s, int nr)
     return SX_ERR_ARG;
   }
   if (nr <= s->rhs_cap) return SX_OK;
-  if (!s->sw_panel || s->sw_D > 6) {
+  if (!s->use_tree && (!s->sw_panel || s->sw_D > 6)) {
     set_error ("msys_reserve_rhs: more than 2 right-hand sides per mode need the panel "
                "sweeps with at most 6 off-diagonal blocks (band offsets kd <= 447)");
     return SX_ERR_LIMIT;
@@ -2031,7 +2091,7 @@ int msys_reserve_rhs (sx_msys* s, int nr)
   s->d_rhs = r;
   s->d_G = g;
   s->rhs_cap = nr;
-  return SX_OK;
+  return tree_workspace (s, nr);
 }
 
 int condense32_tiled (const sx_msys* s, int nz, int stride, const double* X, double* Fp,
@@ -2164,7 +2224,7 @@ int plan_field_solve_direct (BatchPlan& P, const sx_msys* s, int nz, int stride,
                               (const int*) m->d_nidx, (const double*) m->d_nw,
                               (const double*) d_f, stride, lines, lstride,
                               (const int*) s->d_nsolve, s->d_rhs, s->nmax, nz, s->base_mode,
-                              rnr, roff);
+                              rnr, roff, (const int*) nullptr);
   P.phase++;
   if (int rc = plan_band_solve (P, s, 2)) return rc;
   auto rec_r = [&] (auto fn) {
@@ -2240,6 +2300,7 @@ int field_solve_group (sx_msys* s, int nf, int nz, int stride, double* const* d_
   const int npl = n_solved_planes (nz, s->base_mode), nr = 2 * nf;
   const int lstride = m->nbound * m->np;
   const size_t gstride = (size_t) 2 * s->nmodes * m->nglobal;
+  const RhsTo to = rhs_in (s);
   // the register-operand element kernels take up to three fields per launch
   const bool grouped = nf <= 3 && tiled_ok (m) && s->tile_mf;
   const int npmr = reg_npm (m->np);
@@ -2264,7 +2325,7 @@ int field_solve_group (sx_msys* s, int nf, int nz, int stride, double* const* d_
     if (rc) return rc;
     hipLaunchKernelGGL (k_assemble3, dim3 ((m->nglobal + 255) / 256, npl, nf), dim3 (256), 0,
                         st, m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw, fs,
-                        stride, lstride, s->d_nsolve, s->d_rhs, s->nmax, nz, s->base_mode, nr);
+                        stride, lstride, s->d_nsolve, to.p, to.ld, nz, s->base_mode, nr, to.perm);
   }
   for (int f = 0; f < nf && !grouped; f++) {
     const double* lines = (d_lines && d_lines[f] && m->nbound) ? d_lines[f] : nullptr;
@@ -2274,8 +2335,8 @@ int field_solve_group (sx_msys* s, int nf, int nz, int stride, double* const* d_
     if (int rc = condense (s, nz, stride, d_f[f], G, st)) return rc;
     hipLaunchKernelGGL (k_assemble, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0,
                         st, m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw,
-                        d_f[f], stride, lines, lstride, s->d_nsolve, s->d_rhs, s->nmax, nz,
-                        s->base_mode, nr, 2 * f);
+                        d_f[f], stride, lines, lstride, s->d_nsolve, to.p, to.ld, nz, s->base_mode, nr,
+                        2 * f, to.perm);
   }
   SX_HIP (hipGetLastError ());
   if (int rc = band_solve (s, nr, st)) return rc;
@@ -2404,9 +2465,10 @@ extern "C" int sx_field_solve_weak (sx_msys_t s, int nz, int stride, double* d_w
   hipLaunchKernelGGL (k_essential, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_ess, nullptr, 0, s->d_G, nz, s->base_mode);
   if ((rc = condense (s, nz, stride, d_w, s->d_G, st, 1))) return rc;
+  const RhsTo to = rhs_in (s);
   hipLaunchKernelGGL (k_assemble, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw, d_w,
-                      stride, nullptr, 0, s->d_nsolve, s->d_rhs, s->nmax, nz, s->base_mode, 2, 0);
+                      stride, nullptr, 0, s->d_nsolve, to.p, to.ld, nz, s->base_mode, 2, 0, to.perm);
   SX_HIP (hipGetLastError ());
   if ((rc = band_solve (s, 2, st))) return rc;
   return recover (s, nz, stride, d_w, d_u, s->d_G, 2, 0, st);

@@ -1,0 +1,811 @@
+// sx_tree.hip -- dissection solve of the condensed FP64 systems (the matrix
+// of src/matrix.cpp:132-267, solved by the reference with a banded
+// Cholesky, src/field.cpp:672-709).
+//
+// The banded factor makes a solve a chain of 64-row block steps; its length
+// (132 steps at 4,208 rows, 72 for the twisted split) bounds the solve, not
+// its bytes.  Here the elements are split recursively (sx_tree_plan.cpp)
+// and the unknowns eliminated front by front, a level of fronts at once:
+// 1 to 5 levels instead of tens of block steps.  A front with eliminated
+// unknowns K and boundary B has its operators formed at set-up,
+//   E = A_KK^-1 A_KB,   A_KK^-1,   S = A_BB - A_KB^T E  (passed up),
+// and a solve is two dense products per front,
+//   up:    v_K = r_K + (parts' contributions),  c_B = (parts') - E^T v_K
+//   down:  x_K = A_KK^-1 v_K - E x_B
+// so every level is one launch of independent products on FP64 MFMA tiles.
+// Fronts of one class share their operators (a uniform 16x16-element mesh
+// has a few classes per level), so up to 16 right-hand-side columns of a
+// class are taken by one tile and the operators come from the L2s.
+//
+// Operators are stored in MFMA fragment order: per 16-row block and pair of
+// k steps, [lane][2] doubles, so a wavefront reads 1 KB by 16-byte loads.
+#include <algorithm>
+#include <cstdlib>
+#include <string>
+#include <vector>
+
+#include "sx_internal.h"
+#include "sx_tree.h"
+
+namespace sx {
+namespace {
+
+typedef double v4d __attribute__ ((ext_vector_type (4)));
+
+constexpr int TB = 64;                 // pivot block and tile of the factorisation
+
+// ---------------------------------------------------------------------------
+// Set-up
+// ---------------------------------------------------------------------------
+// Front matrices of a level: each entry the sum of its parts' entries
+// (elements: their condensed matrix; fronts: their trailing block).  In a
+// singular mode (the last unknown dropped) the pinned unknown is replaced
+// by the identity.
+__global__ __launch_bounds__(256) void k_tree_assemble (
+    const TreeClass* __restrict__ cls, int cls0, const TreeChild* __restrict__ child,
+    const int* __restrict__ map, const double* __restrict__ Sel, int next, int nec,
+    const double* __restrict__ Fc, size_t fcs, double* F, size_t fs,
+    const int* __restrict__ nsolve, int nsfull)
+{
+  const TreeClass C = cls[cls0 + blockIdx.y];
+  const int mode = blockIdx.z, n = C.k + C.b;
+  const bool pinned = C.pin >= 0 && nsolve[mode] < nsfull;
+  for (size_t e = (size_t) blockIdx.x * 256 + threadIdx.x; e < (size_t) n * n;
+       e += (size_t) gridDim.x * 256) {
+    const int i = (int) (e / n), j = (int) (e % n);
+    double s = 0.0;
+    if (pinned && (i == C.pin || j == C.pin)) {
+      s = i == j ? 1.0 : 0.0;
+    } else {
+      for (int c = 0; c < C.nch; c++) {
+        const TreeChild ch = child[C.ch0 + c];
+        const int a = map[ch.map0 + i], b = map[ch.map0 + j];
+        if (a < 0 || b < 0) continue;
+        if (ch.front) {
+          const TreeClass D = cls[ch.cls];
+          const int nd = D.k + D.b;
+          s += Fc[(size_t) mode * fcs + D.foff + (size_t) (D.k + a) * nd + D.k + b];
+        } else {
+          s += Sel[(((size_t) mode * nec + ch.cls) * next + a) * next + b];
+        }
+      }
+    }
+    F[(size_t) mode * fs + C.foff + e] = s;
+  }
+}
+
+// One step of the in-place Gauss-Jordan elimination of a front's first k
+// unknowns, pivots P = [p0, p0 + pb): this kernel inverts the pivot block
+// and forms, for a tile of 64 columns, R = F_P (the rows as they are) and
+// W = F_PP^-1 F_P (F_PP^-1 itself in the columns of P) into RW.  Every
+// tile's workgroup inverts the block for itself, so a step is two launches.
+__global__ __launch_bounds__(256) void k_tree_panel (
+    const TreeClass* __restrict__ cls, int cls0, const double* __restrict__ F, size_t fs,
+    double* RW, int ldw, int step, int* status)
+{
+  const TreeClass C = cls[cls0 + blockIdx.y];
+  const int mode = blockIdx.z, n = C.k + C.b, p0 = TB * step;
+  const int pb = min (TB, C.k - p0), c0 = TB * blockIdx.x;
+  if (pb <= 0 || c0 >= n) return;
+  __shared__ double piv[TB * (TB + 1)], Rs[TB * (TB + 2)], lines[2][2][TB];
+  __shared__ int s_bad;
+  const double* Fm = F + (size_t) mode * fs + C.foff;
+  const int tid = threadIdx.x, ti = tid >> 4, tj = tid & 15;
+  if (tid == 0) s_bad = 0;
+  // rows of P, columns [c0, c0 + 64)
+  for (int i = tid; i < TB * TB; i += 256) {
+    const int r = i >> 6, c = i & 63;
+    Rs[r * (TB + 2) + c] = (r < pb && c0 + c < n) ? Fm[(size_t) (p0 + r) * n + c0 + c] : 0.0;
+  }
+  double a[4][4];
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const int i = 4 * ti + r, j = 4 * tj + c;
+      a[r][c] = (i < pb && j < pb) ? Fm[(size_t) (p0 + i) * n + p0 + j] : (i == j ? 1.0 : 0.0);
+    }
+  // Gauss-Jordan inversion of the (symmetric positive definite) block, a
+  // 4x4 patch per thread; the pivot row and column pass through LDS
+  for (int t4 = 0; t4 < TB / 4 && 4 * t4 < pb; t4++) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int t = 4 * t4 + u, h = u & 1;
+      if (ti == t4)
+#pragma unroll
+        for (int c = 0; c < 4; c++) lines[h][0][4 * tj + c] = a[u][c];
+      if (tj == t4)
+#pragma unroll
+        for (int r = 0; r < 4; r++) lines[h][1][4 * ti + r] = a[r][u];
+      __syncthreads ();
+      if (t >= pb) continue;
+      const double p = lines[h][0][t];
+      if (tid == 0 && !(p > 0.0) && !s_bad) s_bad = p0 + t + 1;
+      const double d = 1.0 / p;
+      double row[4], col[4];
+#pragma unroll
+      for (int c = 0; c < 4; c++) row[c] = lines[h][0][4 * tj + c] * d;
+#pragma unroll
+      for (int r = 0; r < 4; r++) col[r] = lines[h][1][4 * ti + r];
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const bool ir = ti == t4 && r == u, jc = tj == t4 && c == u;
+          a[r][c] = ir ? (jc ? d : row[c]) : jc ? -col[r] * d : a[r][c] - col[r] * row[c];
+        }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) piv[(4 * ti + r) * (TB + 1) + 4 * tj + c] = a[r][c];
+  __syncthreads ();
+  if (tid == 0 && s_bad && blockIdx.x == 0) atomicMax (status + mode, s_bad);
+  double* Rg = RW + ((size_t) mode * gridDim.y + blockIdx.y) * 2 * TB * ldw;
+  double* Wg = Rg + (size_t) TB * ldw;
+  const int wave = tid >> 6, lane = tid & 63;
+  v4d acc[4] = {};
+#pragma unroll
+  for (int s = 0; s < TB / 4; s++) {
+    const double av = piv[(16 * wave + (lane & 15)) * (TB + 1) + 4 * s + (lane >> 4)];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64 (
+          av, Rs[(4 * s + (lane >> 4)) * (TB + 2) + 16 * q + (lane & 15)], acc[q], 0, 0, 0);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int i = 16 * wave + 4 * r + (lane >> 4), j = c0 + 16 * q + (lane & 15);
+      if (j >= n) continue;
+      Rg[(size_t) i * ldw + j] = Rs[i * (TB + 2) + j - c0];
+      const int jp = j - p0;
+      Wg[(size_t) i * ldw + j] = jp >= 0 && jp < pb ? piv[i * (TB + 1) + jp] : acc[q][r];
+    }
+}
+
+// The rest of the step, one 64x64 tile of the front per workgroup:
+//   i, j not in P:  F_ij -= F_iP W_j,  F_iP = s_i R_i^T
+//   i in P:         F_ij  = W_ij
+//   j in P:         F_ij  = -s_i W_ji
+// with s_i = -1 for unknowns already eliminated (i < p0), +1 otherwise: the
+// matrix stays symmetric up to that sign, so only rows of P are ever read.
+__global__ __launch_bounds__(256) void k_tree_update (
+    const TreeClass* __restrict__ cls, int cls0, double* F, size_t fs,
+    const double* __restrict__ RW, int ldw, int step, int nt)
+{
+  const TreeClass C = cls[cls0 + blockIdx.y];
+  const int mode = blockIdx.z, n = C.k + C.b, p0 = TB * step;
+  const int pb = min (TB, C.k - p0);
+  const int i0 = TB * (blockIdx.x / nt), j0 = TB * (blockIdx.x % nt);
+  if (pb <= 0 || i0 >= n || j0 >= n) return;
+  __shared__ double Rs[TB * (TB + 2)], Ws[TB * (TB + 2)];
+  const double* Rg = RW + ((size_t) mode * gridDim.y + blockIdx.y) * 2 * TB * ldw;
+  const double* Wg = Rg + (size_t) TB * ldw;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  for (int i = tid; i < TB * TB; i += 256) {
+    const int r = i >> 6, c = i & 63;
+    const double v = i0 + c < n ? Rg[(size_t) r * ldw + i0 + c] : 0.0;
+    Rs[r * (TB + 2) + c] = i0 + c < p0 ? -v : v;
+    Ws[r * (TB + 2) + c] = j0 + c < n ? Wg[(size_t) r * ldw + j0 + c] : 0.0;
+  }
+  __syncthreads ();
+  const int wi = 32 * (wave & 1), wj = 32 * (wave >> 1);
+  v4d acc[2][2] = {};
+  const int ks = (pb + 3) / 4;
+  for (int s = 0; s < ks; s++) {
+    const double* ra = Rs + (4 * s + (lane >> 4)) * (TB + 2) + wi + (lane & 15);
+    const double* wb = Ws + (4 * s + (lane >> 4)) * (TB + 2) + wj + (lane & 15);
+    const double a0 = ra[0], a1 = ra[16], b0 = wb[0], b1 = wb[16];
+    acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a0, b0, acc[0][0], 0, 0, 0);
+    acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a0, b1, acc[0][1], 0, 0, 0);
+    acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a1, b0, acc[1][0], 0, 0, 0);
+    acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a1, b1, acc[1][1], 0, 0, 0);
+  }
+  double* Fm = F + (size_t) mode * fs + C.foff;
+#pragma unroll
+  for (int x = 0; x < 2; x++)
+#pragma unroll
+    for (int y = 0; y < 2; y++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int il = wi + 16 * x + 4 * r + (lane >> 4), jl = wj + 16 * y + (lane & 15);
+        const int i = i0 + il, j = j0 + jl;
+        if (i >= n || j >= n) continue;
+        const bool ip = i >= p0 && i < p0 + pb, jp = j >= p0 && j < p0 + pb;
+        double* f = Fm + (size_t) i * n + j;
+        if (ip) *f = Wg[(size_t) (i - p0) * ldw + j];
+        else if (jp) *f = (i < p0 ? 1.0 : -1.0) * Wg[(size_t) (j - p0) * ldw + i];
+        else *f -= acc[x][y][r];
+      }
+}
+
+// Operators of a level in fragment order.  Forward: rows B, k steps over K,
+// entry E[kk][row].  Backward: rows K, k steps over [K | B], entries
+// A_KK^-1[row][j] and -E[row][j-k].
+__global__ __launch_bounds__(256) void k_tree_operators (
+    const TreeClass* __restrict__ cls, int cls0, const double* __restrict__ F, size_t fs,
+    double* ops, size_t os)
+{
+  const TreeClass C = cls[cls0 + blockIdx.y];
+  const int mode = blockIdx.z, n = C.k + C.b;
+  const size_t nf = (size_t) ((C.b + 15) / 16) * C.mfp * 128,
+               nb = (size_t) ((C.k + 15) / 16) * C.mbp * 128;
+  const double* Fm = F + (size_t) mode * fs + C.foff;
+  double* O = ops + (size_t) mode * os;
+  for (size_t e = (size_t) blockIdx.x * 256 + threadIdx.x; e < nf + nb;
+       e += (size_t) gridDim.x * 256) {
+    const bool fw = e < nf;
+    const size_t q = fw ? e : e - nf;
+    const int np = fw ? C.mfp : C.mbp;
+    const int h = (int) (q & 1), l = (int) ((q >> 1) & 63), pair = (int) ((q >> 7) % np),
+              rb = (int) ((q >> 7) / np);
+    const int row = 16 * rb + (l & 15), kk = 4 * (2 * pair + h) + (l >> 4);
+    double v = 0.0;
+    if (fw) {
+      if (row < C.b && kk < C.k) v = Fm[(size_t) kk * n + C.k + row];
+      O[C.mf + q] = v;
+    } else {
+      if (row < C.k && kk < n) v = Fm[(size_t) row * n + kk];
+      O[C.mb + q] = kk < C.k ? v : -v;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Solve: one launch per level and direction
+// ---------------------------------------------------------------------------
+struct TreeArgs {
+  const TreeItem* item;
+  int nitem, nmodes, xcd;
+  const int *gk, *gb, *tgt;
+  const double* ops;
+  size_t os;
+  const double* in;                    // [mode][nr][nsp] by position
+  double *rhs, *v, *cb;                // [mode][nr][nmax] by node, [..][nsp], [..][slots]
+  double* sum;                         // solution added to here as well (or null)
+  int nmax, nsp, nr;
+  size_t slots;
+  const int* nsolve;
+};
+
+enum { T_UP = 0, T_DOWN = 1, T_ROOT = 2 };
+
+// UP: forward product of a level, DOWN: backward; ROOT: backward of the
+// root, which gathers its v_K itself (no forward product: no boundary).
+// A level is bound by its chain of dependent loads, not by its bytes: the
+// work item; then the operator's fragments, the right-hand sides and the
+// parts' contributions (W neighbouring values each); DOWN one more, the
+// solution at the boundary nodes.  Every load of a round is issued before
+// any of it is used.
+template <int DIR, int W>
+__global__ __launch_bounds__(256) void k_tree_level (TreeArgs T)
+{
+  extern __shared__ double sm[];
+  // a mode's work stays on one XCD where the modes fill all eight: its
+  // tiles of one class then share the operators in that L2
+  int mode, item;
+  if (T.xcd) {
+    const int q = blockIdx.x >> 3;
+    mode = 8 * (q / T.nitem) + (blockIdx.x & 7);
+    item = q % T.nitem;
+    if (mode >= T.nmodes) return;
+  } else {
+    mode = blockIdx.x / T.nitem;
+    item = blockIdx.x % T.nitem;
+  }
+  const TreeItem it = T.item[item];
+  const int nr = T.nr, ns = T.nsolve[mode];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane (tid >> 6);
+  const int k = it.k, n = it.k + it.b;
+  const int K = DIR == T_DOWN ? n : k, rows = DIR == T_UP ? it.b : k;
+  const int np = (K + 7) / 8;
+  const int ncol = it.nf * nr, ldx = ncol | 1;
+  const int kw = it.kw, kp = wave & (kw - 1), rb = it.rb0 + wave / kw;
+  const bool active = 16 * rb < rows;
+  const double2* A = (const double2*) (T.ops + (size_t) mode * T.os + it.op) +
+                     (size_t) rb * np * 64 + lane;
+  const int q0 = np * kp / kw, q1 = active ? np * (kp + 1) / kw : 0;
+  constexpr int U = 8;
+  double2 a[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) a[u] = q0 + u < q1 ? A[(size_t) (q0 + u) * 64] : make_double2 (0.0, 0.0);
+  // this lane's outputs: rows 16 rb + 4 i + lane/16 of column lane%16
+  const size_t mrow = (size_t) mode * nr;
+  const int col = min (lane & 15, ncol - 1), oj = col / nr;
+  const size_t orow = mrow + col % nr;
+  const bool out = active && kp == 0 && (lane & 15) < ncol;
+  double base[4];
+  int to[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int row = 16 * rb + 4 * i + (lane >> 4);
+    const bool ok = out && row < rows;
+    to[i] = -1;
+    base[i] = 0.0;
+    if (DIR == T_UP) {
+      if (ok) to[i] = T.tgt[it.offb + oj * it.b + row];
+      if (ok && it.src) {
+        const double2* c = (const double2*) (T.cb + orow * T.slots) +
+                           (size_t) (it.offn + oj * n + k + row) * (W / 2);
+        double2 w[W / 2];
+#pragma unroll
+        for (int q = 0; q < W / 2; q++) w[q] = c[q];
+#pragma unroll
+        for (int q = 0; q < W / 2; q++) base[i] += w[q].x + w[q].y;
+      }
+    } else if (ok) {
+      to[i] = T.gk[it.offk + oj * k + row];
+    }
+  }
+  // the column operand [k rows padded to 8][ldx], chunks of 64 rows of a column
+  const int Kp = np * 8, nk = (Kp + 63) / 64, nc = nk * ncol;
+  constexpr int G = DIR == T_DOWN ? 8 : 6;
+  for (int c0 = wave; c0 < nc; c0 += 4 * G) {
+    double x[G];
+    int g[G];
+    if (DIR == T_DOWN) {
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
+        g[u] = c < nc && kk >= k && kk < n ? T.gb[it.offb + (cl / nr) * it.b + kk - k] : ns;
+      }
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
+        const size_t r = mrow + cl % nr;
+        x[u] = 0.0;
+        if (c < nc && kk < k) x[u] = T.v[r * T.nsp + it.offk + (cl / nr) * k + kk];
+        else if (g[u] < ns) x[u] = T.rhs[r * T.nmax + g[u]];
+      }
+    } else {
+      double2 w[G][W / 2];
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
+        const size_t r = mrow + cl % nr;
+        const bool ok = c < nc && kk < k;
+        x[u] = ok ? T.in[r * T.nsp + it.offk + (cl / nr) * k + kk] : 0.0;
+        const double2* cb = (const double2*) (T.cb + r * T.slots) +
+                            (size_t) (it.offn + (cl / nr) * n + kk) * (W / 2);
+#pragma unroll
+        for (int q = 0; q < W / 2; q++) w[u][q] = ok && it.src ? cb[q] : make_double2 (0.0, 0.0);
+      }
+#pragma unroll
+      for (int u = 0; u < G; u++) {
+        const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
+#pragma unroll
+        for (int q = 0; q < W / 2; q++) x[u] += w[u][q].x + w[u][q].y;
+        if (DIR == T_UP && it.rb0 == 0 && c < nc && kk < k)
+          T.v[(mrow + cl % nr) * T.nsp + it.offk + (cl / nr) * k + kk] = x[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
+      if (c < nc && kk < Kp) sm[kk * ldx + cl] = x[u];
+    }
+  }
+  __syncthreads ();
+  // columns past ncol read a valid column (their results are not stored)
+  const double* X = sm + (lane >> 4) * ldx + col;
+  v4d acc0 = {}, acc1 = {};
+  for (int q = q0; q < q1; q += U) {
+    double2 b[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      b[u] = a[u];
+      if (q + U + u < q1) a[u] = A[(size_t) (q + U + u) * 64];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (q + u < q1) {
+        const double* x = X + (size_t) 8 * (q + u) * ldx;
+        acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64 (b[u].x, x[0], acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64 (b[u].y, x[4 * ldx], acc1, 0, 0, 0);
+      }
+  }
+  v4d acc = acc0 + acc1;
+  if (kw > 1) {
+    double* red = sm + (size_t) Kp * ldx;
+    if (kp)
+#pragma unroll
+      for (int i = 0; i < 4; i++) red[(wave * 4 + i) * 64 + lane] = acc[i];
+    __syncthreads ();
+    if (kp == 0)
+      for (int p = 1; p < kw; p++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[i] += red[((wave + p) * 4 + i) * 64 + lane];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    if (to[i] < 0) continue;
+    if (DIR == T_UP) {
+      T.cb[orow * T.slots + to[i]] = base[i] - acc[i];
+    } else if (to[i] < ns) {
+      T.rhs[orow * T.nmax + to[i]] = acc[i];
+      if (T.sum) T.sum[orow * T.nmax + to[i]] += acc[i];
+    }
+  }
+}
+
+// Entries of a mode's assembled matrix, each pair (row <= column) summed
+// over its elements in the band assembly's order
+__global__ __launch_bounds__(256) void k_tree_entries (int npairs, const int* __restrict__ pptr,
+                                                       const int* __restrict__ psrc,
+                                                       const double* __restrict__ S, double* val)
+{
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= npairs) return;
+  double s = 0.0;
+  for (int c = pptr[p]; c < pptr[p + 1]; c++) s += S[psrc[c]];
+  val[p] = s;
+}
+
+// out = b - A x for one mode's nr right-hand sides (b by bperm, out by
+// operm: the positions of their dissections), accumulated in twice
+// the working precision (error-free products and sums); a wavefront per row
+__global__ __launch_bounds__(256) void k_tree_residual (
+    int ns, int nmax, int nr, const int* __restrict__ ptr, const int* __restrict__ col,
+    const int* __restrict__ pair, const double* __restrict__ val, const double* __restrict__ b,
+    int ldb, const int* __restrict__ bperm, const double* __restrict__ x, double* out, int ldo,
+    const int* __restrict__ operm)
+{
+#pragma clang fp contract(off)
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= ns) return;
+  auto two_sum = [] (double& s, double& e, double v) {
+    const double t = s + v, z = t - s;
+    e += (s - (t - z)) + (v - z);
+    s = t;
+  };
+  for (int r = 0; r < nr; r++) {
+    double s = 0.0, e = 0.0;
+    for (int c = ptr[row] + lane; c < ptr[row + 1]; c += 64) {
+      const int j = col[c];
+      if (j >= ns) continue;
+      const double a = -val[pair[c]], xv = x[(size_t) r * nmax + j], q = a * xv;
+      e += __builtin_fma (a, xv, -q);
+      two_sum (s, e, q);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      const double so = __shfl_xor (s, o, 64), eo = __shfl_xor (e, o, 64);
+      two_sum (s, e, so);
+      e += eo;
+    }
+    if (lane == 0) {
+      two_sum (s, e, b[(size_t) r * ldb + (bperm ? bperm[row] : row)]);
+      out[(size_t) r * ldo + operm[row]] = s + e;
+    }
+  }
+}
+
+template <typename V> int upload (V** d, const std::vector<V>& h)
+{
+  *d = nullptr;
+  if (h.empty ()) return SX_OK;
+  SX_HIP (hipMalloc (d, sizeof (V) * h.size ()));
+  SX_HIP (hipMemcpy (*d, h.data (), sizeof (V) * h.size (), hipMemcpyHostToDevice));
+  return SX_OK;
+}
+
+}  // namespace
+
+// A mesh's plan for one mode count with its tables on the device
+struct TreeDev {
+  TreePlan P;
+  int nmodes = 0;
+  bool ok = false;
+  TreeClass* cls = nullptr;
+  TreeChild* child = nullptr;
+  TreeItem* item = nullptr;
+  int *map = nullptr, *gk = nullptr, *gb = nullptr, *tgt = nullptr, *perm = nullptr;
+};
+
+void tree_free (TreeDev* t)
+{
+  if (!t) return;
+  void* p[] = {t->cls, t->child, t->item, t->map, t->gk, t->gb, t->tgt, t->perm};
+  for (void* q : p) if (q) (void) hipFree (q);
+  delete t;
+}
+
+// The environment variables that choose a band layout keep the band solve.
+static bool band_forced ()
+{
+  for (const char* v : {"SX_BAND_TWIST", "SX_BAND_UNIT", "SX_BAND_SPLIT", "SX_BAND_SWEEP",
+                        "SX_BAND_BLOCK", "SX_BAND_LL", "SX_PANEL_NR"})
+    if (std::getenv (v)) return true;
+  return false;
+}
+
+// The band solve stays for systems outside the dissection's bounds: bands
+// past 768 (refused as before by the band solve), a mesh tree_plan does not
+// suit, and operators of more than 24 GB.  always: also under a variable
+// that chooses a band layout.
+constexpr size_t TREE_OPS_MAX = (size_t) 3 << 30;      // doubles
+
+int tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always)
+{
+  *out = nullptr;
+  if ((!always && band_forced ()) || m->nband > 768) return SX_OK;
+  std::lock_guard<std::mutex> lock (m->tree_mu);
+  for (TreeDev* t : m->trees)
+    if (t->nmodes == nmodes) {
+      *out = t->ok ? t : nullptr;
+      return SX_OK;
+    }
+  TreeDev* t = new TreeDev;
+  t->nmodes = nmodes;
+  m->trees.push_back (t);
+  size_t f = 0;
+  t->ok = tree_plan (m, nmodes, t->P);
+  for (const TreeLevel& L : t->P.lev) f = std::max (f, L.fsize);
+  t->ok = t->ok && t->P.ops * nmodes <= TREE_OPS_MAX && f * nmodes <= TREE_OPS_MAX;
+  if (!t->ok) { t->P = TreePlan (); return SX_OK; }
+  int rc;
+  if ((rc = upload (&t->cls, t->P.cls)) || (rc = upload (&t->child, t->P.child)) ||
+      (rc = upload (&t->item, t->P.item)) || (rc = upload (&t->map, t->P.map)) ||
+      (rc = upload (&t->gk, t->P.gk)) || (rc = upload (&t->gb, t->P.gb)) ||
+      (rc = upload (&t->tgt, t->P.tgt)) || (rc = upload (&t->perm, t->P.perm))) {
+    t->ok = false;
+    return rc;
+  }
+  *out = t;
+  return SX_OK;
+}
+
+// Factorisation of nm modes: the levels from the elements to the root (Sel:
+// the condensed element matrices [nm][nclass][next][next]) into *ops.
+// status[mode] > 0: a pivot was not positive.  Waits for st.
+static int factor (const TreeDev* t, const sx_mesh* m, int nm, const int* d_nsolve,
+                   const double* Sel, double** ops, hipStream_t st, int* d_status)
+{
+  const TreePlan& P = t->P;
+  const int nl = (int) P.lev.size ();
+  size_t fmax[2] = {0, 0}, rw = 0;
+  for (int j = 0; j < nl; j++) {
+    const TreeLevel& L = P.lev[j];
+    fmax[j & 1] = std::max (fmax[j & 1], L.fsize);
+    rw = std::max (rw, (size_t) L.ncls * 2 * TB * ((L.nmax + TB - 1) / TB * TB));
+  }
+  double* buf = nullptr;
+  SX_HIP (hipMalloc (ops, sizeof (double) * std::max<size_t> (P.ops * nm, 2)));
+  SX_HIP (hipMalloc (&buf, sizeof (double) * (fmax[0] + fmax[1] + rw) * nm));
+  double* F[2] = {buf, buf + fmax[0] * nm};
+  double* RW = F[1] + fmax[1] * nm;
+  for (int j = nl - 1; j >= 0; j--) {
+    const TreeLevel& L = P.lev[j];
+    const int nt = (L.nmax + TB - 1) / TB, ldw = nt * TB;
+    const size_t n2 = (size_t) L.nmax * L.nmax;
+    double* Fj = F[j & 1];
+    const dim3 gb ((unsigned) std::min<size_t> ((n2 + 255) / 256, 1024), L.ncls, nm);
+    hipLaunchKernelGGL (k_tree_assemble, gb, dim3 (256), 0, st, t->cls, L.cls0, t->child, t->map,
+                        Sel, m->next, m->nclass, F[(j + 1) & 1],
+                        j + 1 < nl ? P.lev[j + 1].fsize : (size_t) 0, Fj, L.fsize, d_nsolve,
+                        m->nsolve);
+    for (int step = 0; TB * step < L.kmax; step++) {
+      hipLaunchKernelGGL (k_tree_panel, dim3 (nt, L.ncls, nm), dim3 (256), 0, st, t->cls, L.cls0,
+                          Fj, L.fsize, RW, ldw, step, d_status);
+      hipLaunchKernelGGL (k_tree_update, dim3 (nt * nt, L.ncls, nm), dim3 (256), 0, st, t->cls,
+                          L.cls0, Fj, L.fsize, RW, ldw, step, nt);
+    }
+    hipLaunchKernelGGL (k_tree_operators, gb, dim3 (256), 0, st, t->cls, L.cls0, Fj, L.fsize,
+                        *ops, P.ops);
+  }
+  const hipError_t e = hipGetLastError ();
+  if (e == hipSuccess) (void) hipStreamSynchronize (st);
+  (void) hipFree (buf);
+  return e == hipSuccess ? (int) SX_OK : hip_fail (e, "tree_factor");
+}
+
+// The launches of a solve: up to the root's children, down from the root
+static int sweep (const TreeDev* t, TreeArgs T, int nm, int nr, hipStream_t st)
+{
+  const TreePlan& P = t->P;
+  const int q = nr / 2 - 1, nl = (int) P.lev.size ();
+  T.gk = t->gk; T.gb = t->gb; T.tgt = t->tgt;
+  T.os = P.ops;
+  T.nsp = P.nsolve; T.slots = P.slots; T.nr = nr;
+  T.nmodes = nm;
+  T.xcd = nm >= 32 || (nm >= 8 && nm % 8 == 0);
+  auto launch = [&] (auto kern, int first, int count, size_t lds) {
+    if (!count) return (int) SX_OK;
+    SX_HIP (hipFuncSetAttribute ((const void*) kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int) lds));
+    T.item = t->item + first;
+    T.nitem = count;
+    const int blocks = count * (T.xcd ? (nm + 7) / 8 * 8 : nm);
+    hipLaunchKernelGGL (kern, dim3 (blocks), dim3 (256), lds, st, T);
+    SX_HIP (hipGetLastError ());
+    return (int) SX_OK;
+  };
+  auto level = [&] (int j, int dir) {
+    const TreeLevel& L = P.lev[j];
+    const int first = dir ? L.it_b[q] : L.it_f[q], count = dir ? L.nit_b[q] : L.nit_f[q];
+    const size_t lds = dir ? L.lds_b[q] : L.lds_f[q];
+    auto with = [&] (auto w) {
+      constexpr int W = decltype (w)::value;
+      return dir == 0 ? launch (k_tree_level<T_UP, W>, first, count, lds)
+             : j      ? launch (k_tree_level<T_DOWN, W>, first, count, lds)
+                      : launch (k_tree_level<T_ROOT, W>, first, count, lds);
+    };
+    return P.W == 2   ? with (std::integral_constant<int, 2> {})
+           : P.W == 4 ? with (std::integral_constant<int, 4> {})
+                      : with (std::integral_constant<int, 8> {});
+  };
+  for (int j = nl - 1; j > 0; j--)
+    if (int rc = level (j, 0)) return rc;
+  for (int j = 0; j < nl; j++)
+    if (int rc = level (j, 1)) return rc;
+  return SX_OK;
+}
+
+// Refinement of a singular mode's solution (pure Neumann, its last unknown
+// dropped: condition ~1e5 against the constant vector, so two eliminations
+// in working precision end ~2e-11 of the pressure apart).  One correction
+// from a residual in twice the working precision, formed with the entries
+// the band assembly rounds to, leaves the exact solution of the assembled
+// system to rounding, after a dissection and after a band solve alike.  The
+// correction runs on a dissection of that mode alone, cut for one mode
+// (fewer levels).
+struct TreeSing {
+  int mode = 0;
+  TreeDev* t = nullptr;
+  double *ops = nullptr, *val = nullptr, *r = nullptr, *dx = nullptr, *v = nullptr, *cb = nullptr,
+         *b = nullptr;                 // band solves: the right-hand sides kept
+};
+
+// row lists of the assembled matrix (both triangles), once per mesh
+static int sing_rows (sx_mesh* m)
+{
+  std::lock_guard<std::mutex> lock (m->tree_mu);
+  if (m->d_sptr) return SX_OK;
+  std::vector<int> ptr (m->nsolve + 1, 0), col, pr;
+  for (int p = 0; p < m->npairs; p++) {
+    const int a = m->pmn[2 * p], b = m->pmn[2 * p + 1];
+    ptr[a + 1]++;
+    if (a != b) ptr[b + 1]++;
+  }
+  for (int i = 0; i < m->nsolve; i++) ptr[i + 1] += ptr[i];
+  col.resize (ptr[m->nsolve]);
+  pr.resize (ptr[m->nsolve]);
+  std::vector<int> at (ptr.begin (), ptr.end () - 1);
+  for (int p = 0; p < m->npairs; p++) {
+    const int a = m->pmn[2 * p], b = m->pmn[2 * p + 1];
+    col[at[a]] = b;
+    pr[at[a]++] = p;
+    if (a != b) { col[at[b]] = a; pr[at[b]++] = p; }
+  }
+  int rc;
+  if ((rc = upload (&m->d_scol, col)) || (rc = upload (&m->d_spair, pr)) ||
+      (rc = upload (&m->d_sptr, ptr)))
+    return rc;
+  return SX_OK;
+}
+
+void tree_sing_free (TreeSing* g)
+{
+  if (!g) return;
+  for (double* p : {g->ops, g->val, g->r, g->dx, g->v, g->cb, g->b}) if (p) (void) hipFree (p);
+  delete g;
+}
+
+// Workspace of a solve with nr right-hand sides per mode
+int tree_workspace (sx_msys* s, int nr)
+{
+  auto grow = [] (double** p, size_t n) {
+    double* q = nullptr;
+    SX_HIP (hipMalloc (&q, sizeof (double) * std::max<size_t> (n, 1)));
+    SX_HIP (hipMemset (q, 0, sizeof (double) * n));
+    (void) hipFree (*p);
+    *p = q;
+    return (int) SX_OK;
+  };
+  const size_t n = (size_t) s->nmodes * nr;
+  int rc;
+  if (s->use_tree) {
+    const TreePlan& P = s->tree->P;
+    if ((rc = grow (&s->d_tb, n * P.nsolve)) || (rc = grow (&s->d_tv, n * P.nsolve)) ||
+        (rc = grow (&s->d_tc, n * P.slots)))
+      return rc;
+  }
+  if (TreeSing* g = s->sing) {
+    const TreePlan& P = g->t->P;
+    if ((rc = grow (&g->b, (size_t) nr * s->nmax)) || (rc = grow (&g->dx, (size_t) nr * s->nmax)) ||
+        (rc = grow (&g->v, (size_t) nr * P.nsolve)) || (rc = grow (&g->cb, nr * P.slots)) ||
+        (rc = grow (&g->r, (size_t) nr * P.nsolve)))
+      return rc;
+  }
+  SX_HIP (hipStreamSynchronize (nullptr));
+  return SX_OK;
+}
+
+const int* tree_perm (const sx_msys* s) { return s->use_tree ? s->tree->perm : nullptr; }
+
+int tree_factor (sx_msys* s, const double* Sel, hipStream_t st, int* d_status)
+{
+  return factor (s->tree, s->m, s->nmodes, s->d_nsolve, Sel, &s->d_tops, st, d_status);
+}
+
+int tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_status)
+{
+  sx_mesh* m = s->m;
+  for (int md = 0; md < s->nmodes; md++) {
+    if (s->nsolve[md] == m->nsolve || s->nsolve[md] < 1) continue;
+    TreeDev* t = nullptr;
+    if (int rc = tree_prepare (m, 1, &t, true)) return rc;
+    if (!t) return SX_OK;
+    TreeSing* g = s->sing = new TreeSing;
+    g->mode = md;
+    g->t = t;
+    const double* S = Sel + (size_t) md * m->nclass * m->next * m->next;
+    if (int rc = factor (t, m, 1, s->d_nsolve + md, S, &g->ops, st, d_status + md)) return rc;
+    if (int rc = sing_rows (m)) return rc;
+    SX_HIP (hipMalloc (&g->val, sizeof (double) * std::max (m->npairs, 1)));
+    hipLaunchKernelGGL (k_tree_entries, dim3 ((m->npairs + 255) / 256), dim3 (256), 0, st,
+                        m->npairs, m->d_pptr, m->d_psrc, S, g->val);
+    SX_HIP (hipGetLastError ());
+    return SX_OK;                      // at most mode 0 has a zero constant
+  }
+  return SX_OK;
+}
+
+static int refine (const sx_msys* s, int nr, const double* b, int ldb, const int* bperm,
+                   hipStream_t st)
+{
+  const TreeSing* g = s->sing;
+  const sx_mesh* m = s->m;
+  const int ns = s->nsolve[g->mode];
+  double* x = s->d_rhs + (size_t) g->mode * nr * s->nmax;
+  hipLaunchKernelGGL (k_tree_residual, dim3 ((ns + 3) / 4), dim3 (256), 0, st, ns, s->nmax, nr,
+                      m->d_sptr, m->d_scol, m->d_spair, g->val, b, ldb, bperm, x, g->r,
+                      g->t->P.nsolve, g->t->perm);
+  SX_HIP (hipGetLastError ());
+  TreeArgs T {};
+  T.ops = g->ops;
+  T.in = g->r; T.rhs = g->dx; T.v = g->v; T.cb = g->cb;
+  T.sum = x;
+  T.nmax = s->nmax;
+  T.nsolve = s->d_nsolve + g->mode;
+  return sweep (g->t, T, 1, nr, st);
+}
+
+int sing_keep (const sx_msys* s, int nr, hipStream_t st)
+{
+  const TreeSing* g = s->sing;
+  SX_HIP (hipMemcpyAsync (g->b, s->d_rhs + (size_t) g->mode * nr * s->nmax,
+                          sizeof (double) * nr * s->nmax, hipMemcpyDeviceToDevice, st));
+  return SX_OK;
+}
+
+int sing_refine (const sx_msys* s, int nr, hipStream_t st)
+{
+  return refine (s, nr, s->sing->b, s->nmax, nullptr, st);
+}
+
+// Solve of the nr (2, 4, 6) right-hand sides per mode from d_tb to d_rhs.
+int tree_solve (const sx_msys* s, int nr, hipStream_t st)
+{
+  if (nr < 2 || nr > 6 || (nr & 1) || nr > s->rhs_cap) {
+    set_error ("tree solve: 2, 4 or 6 reserved right-hand sides per mode");
+    return SX_ERR_ARG;
+  }
+  s->last_kernel = 4;
+  s->last_nr = nr;
+  TreeArgs T {};
+  T.ops = s->d_tops;
+  T.in = s->d_tb; T.rhs = s->d_rhs; T.v = s->d_tv; T.cb = s->d_tc;
+  T.nmax = s->nmax;
+  T.nsolve = s->d_nsolve;
+  const TreeDev* t = s->tree;
+  if (int rc = sweep (t, T, s->nmodes, nr, st)) return rc;
+  if (!s->sing) return SX_OK;
+  const int nsp = t->P.nsolve;
+  return refine (s, nr, s->d_tb + (size_t) s->sing->mode * nr * nsp, nsp, t->perm, st);
+}
+
+}  // namespace sx
