@@ -310,8 +310,7 @@ int launch_sweeps (const sx_msys* s, hipStream_t st)
   const int W = window (s->m->nband, B);
   const size_t lds = sweep_lds<B> (W, 2);
   auto kern = k_band_sweeps<B, QS, 2>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   hipLaunchKernelGGL (kern, dim3 (s->nmodes), dim3 (SW_NW * 64), lds, st, s->d_swF,
                       s->d_swR, s->sw_stride, s->m->nband, W, s->d_nsolve, s->d_rhs,
                       s->nmax);
@@ -856,8 +855,7 @@ int launch_panel_d (const sx_msys* s, int G, int stage, hipStream_t st)
   constexpr int NW = PanelSweep<NR, D>::NW;
   const size_t lds = sizeof (double) * ((size_t) PB * NR * (2 * D + NW));
   auto kern = k_panel_sweeps<NR, D>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   const int pieces = (stage == 1 || stage == 3) ? 2 : 1;
   const int nblocks = (s->nmodes + 7) / 8 * 8 * G * pieces;
   hipLaunchKernelGGL (kern, dim3 (nblocks), dim3 (NW * 64), lds, st, s->d_swF, s->d_swR,
@@ -2118,8 +2116,7 @@ int launch_unit_d (const sx_msys* s, int G, int stage, hipStream_t st)
 {
   const size_t lds = sizeof (double) * ((size_t) (D + 3) * UW * PB * NR);
   auto kern = band_ll () ? k_unit_sweeps<NR, D, true> : k_unit_sweeps<NR, D, false>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   const int pieces = (stage == 1 || stage == 3) ? 2 : 1;
   const int nblocks = (s->nmodes + 7) / 8 * 8 * G * pieces;
   hipLaunchKernelGGL (kern, dim3 (nblocks), dim3 (UW * 64), lds, st, s->d_swF, s->d_swR,
@@ -2198,8 +2195,7 @@ int launch_split_d (const sx_msys* s, int G, int stage, hipStream_t st, bool pro
                ? SX_OK : SX_ERR_LIMIT;
   const size_t lds = split_lds<NR, D, R> ();
   auto kern = ll ? k_split_sweeps<NR, D, R, true, 2> : k_split_sweeps<NR, D, R, false, 2>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   hipLaunchKernelGGL (kern, dim3 (nblocks), dim3 (UW * 64), lds, st, s->d_swF, s->d_swR,
                       s->sw_stride, s->d_nsolve, s->d_rhs, s->nmax, s->nmodes, G,
                       s->d_tw, stage, s->tw_boff, s->d_rhsb, s->nmaxb, s->m->nband - 1,
@@ -2247,8 +2243,7 @@ int split_alloc (sx_msys* s, hipStream_t st)
 int unit_panels (const sx_msys* s, double* P, int nbp, hipStream_t st)
 {
   const size_t lds = sizeof (double) * 2 * PB * (PB + 1);
-  SX_HIP (hipFuncSetAttribute ((const void*) k_panel_unit,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) k_panel_unit, lds)) return rc;
   hipLaunchKernelGGL (k_panel_unit, dim3 ((unsigned) (nbp * s->sw_D), s->nmodes), dim3 (256),
                       lds, st, P, s->sw_stride, s->sw_D, nbp);
   SX_HIP (hipGetLastError ());

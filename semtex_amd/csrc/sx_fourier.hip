@@ -464,8 +464,7 @@ int launch_fft2_t (int S, int nb, const FusedBatch& bt, int sign, const double2*
           al (fu.fsub);
   }
   auto kern = v16 ? k_fft2_z<N, R1, TH, true> : k_fft2_z<N, R1, TH, false>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = sx::lds_limit ((const void*) kern, lds)) return rc;
   hipLaunchKernelGGL (kern, dim3 (ntiles, nb), dim3 (TH), lds, st, bt, S, sign, tw);
   SX_HIP (hipGetLastError ());
   return SX_OK;
@@ -504,8 +503,7 @@ int launch_fft (int S, const double* in, double* out, int sign, const double2* t
 {
   const size_t lds = FftTile<N>::lds ();
   auto kern = k_fft_z<N>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = sx::lds_limit ((const void*) kern, lds)) return rc;
   const int TS = FftTile<N>::TS;
   hipLaunchKernelGGL (kern, dim3 ((S + TS - 1) / TS), dim3 (FT_THREADS), lds, st, in, out, S,
                       sign, tw);

@@ -24,6 +24,15 @@ int  hip_fail (hipError_t e, const char* what);
     if (_e != hipSuccess) return sx::hip_fail (_e, #call);            \
   } while (0)
 
+// Dynamic LDS above the 64 KiB every kernel may have needs the kernel's
+// attribute raised; below it the call (about 1 us of a launch) is left out.
+inline int lds_limit (const void* kern, size_t lds)
+{
+  if (lds > 64 * 1024)
+    SX_HIP (hipFuncSetAttribute (kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  return SX_OK;
+}
+
 // GLL rule (femlib/polylib.c:312 zwglj, :513 Dglj), host.
 void gll (int np, double* z, double* w, double* D);
 // edge-major permutation (femlib/mapping.c:46-132), host.

@@ -1835,8 +1835,7 @@ int launch_condense_r (const sx_msys* s, int nz, int stride, double* F, int weak
   const sx_mesh* m = s->m;
   const size_t lds = reg_lds (m, false);
   auto kern = k_condense_r<NPM>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   hipLaunchKernelGGL (kern, dim3 (m->ntile, n_mode_blocks (nz)), dim3 (CT_THREADS), lds, st,
                       m->np, m->nclass, m->d_ttab, m->d_emap, m->d_geo, s->d_Mcon, F, stride, nz,
                       s->base_mode, weak);
@@ -1851,8 +1850,7 @@ int launch_recover_r (const sx_msys* s, int nz, int stride, const double* F, dou
   const sx_mesh* m = s->m;
   const size_t lds = reg_lds (m, true);
   auto kern = k_recover_r<NPM>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   hipLaunchKernelGGL (kern, dim3 (m->ntile, n_mode_blocks (nz)), dim3 (CT_THREADS), lds, st,
                       m->np, m->nclass, m->d_ttab, m->d_emap, s->d_Mrec, G, m->nglobal, F, U,
                       stride, s->d_nsolve, s->d_rhs, s->nmax, nz, s->base_mode, rnr, roff,
@@ -1871,8 +1869,7 @@ int launch_condense_group (const sx_msys* s, int nf, int nz, int stride, const F
   const sx_mesh* m = s->m;
   const size_t lds = reg_lds (m, false);
   auto kern = k_condense_rb<NPM>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   hipLaunchKernelGGL (kern, dim3 (m->ntile, n_mode_blocks (nz), nf), dim3 (CT_THREADS), lds, st,
                       m->np, m->nclass, m->d_ttab, m->d_emap, m->d_geo, s->d_Mcon, F, stride, nz,
                       s->base_mode, 0);
@@ -1886,8 +1883,7 @@ int launch_recover_group (const sx_msys* s, int nf, int nz, int stride, const Fi
   const sx_mesh* m = s->m;
   const size_t lds = reg_lds (m, true);
   auto kern = k_recover_rb<NPM>;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   hipLaunchKernelGGL (kern, dim3 (m->ntile, n_mode_blocks (nz), nf), dim3 (CT_THREADS), lds, st,
                       m->np, m->nclass, m->d_ttab, m->d_emap, s->d_Mrec, G, m->nglobal, F, U,
                       stride, s->d_nsolve, s->d_rhs, s->nmax, nz, s->base_mode, rnr);
@@ -1927,8 +1923,7 @@ int condense (const sx_msys* s, int nz, int stride, double* F, const double* G, 
   }
   const size_t lds = tiled_lds (m, false, false);
   auto kern = k_condense_t;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   hipLaunchKernelGGL (kern, dim3 (m->ntile, n_mode_blocks (nz)), dim3 (CT_THREADS),
                       lds, st, m->np, m->nclass, m->d_tile, m->d_elist, m->d_emap, m->d_emask,
                       m->d_geo, s->d_Mcon, F, stride, nz, s->base_mode, weak);
@@ -1959,8 +1954,7 @@ int recover (const sx_msys* s, int nz, int stride, const double* F, double* U, c
   }
   const size_t lds = tiled_lds (m, true, false);
   auto kern = k_recover_t;
-  SX_HIP (hipFuncSetAttribute ((const void*) kern,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) kern, lds)) return rc;
   hipLaunchKernelGGL (kern, dim3 (m->ntile, n_mode_blocks (nz)), dim3 (CT_THREADS), lds,
                       st, m->np, m->nclass, m->d_tile, m->d_elist, m->d_emap, m->d_btog,
                       m->d_bmask, m->d_emask, s->d_Mrec, G, m->nglobal, F, U, stride,
@@ -2102,8 +2096,7 @@ int condense32_tiled (const sx_msys* s, int nz, int stride, const double* X, dou
   const size_t lds = sizeof (double) * m->next * CG_EP +
                      sizeof (float) * ((size_t) Cs.KR * Cs.NA + (size_t) Cs.KR * CG_EP) +
                      sizeof (int) * m->npnp;
-  SX_HIP (hipFuncSetAttribute ((const void*) k_condense32_t,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) k_condense32_t, lds)) return rc;
   hipLaunchKernelGGL (k_condense32_t, dim3 (m->ntile, n_mode_blocks (nz)), dim3 (CT_THREADS),
                       lds, st, m->np, m->nclass, m->d_tile, m->d_elist, m->d_emap, s->d_Mcon32,
                       X, Fp, stride, nz, s->base_mode);
@@ -2119,8 +2112,7 @@ int recover32_tiled (const sx_msys* s, int nz, int stride, const double* Fp, dou
   const size_t lds = sizeof (double) * m->next * CG_EP +
                      sizeof (float) * ((size_t) R.KR * R.NA + (size_t) R.KR * CG_EP) +
                      sizeof (int) * m->npnp;
-  SX_HIP (hipFuncSetAttribute ((const void*) k_recover32_t,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+  if (int rc = lds_limit ((const void*) k_recover32_t, lds)) return rc;
   hipLaunchKernelGGL (k_recover32_t, dim3 (m->ntile, n_mode_blocks (nz)), dim3 (CT_THREADS),
                       lds, st, m->np, m->nclass, m->d_tile, m->d_elist, m->d_emap, m->d_btog,
                       s->d_Mrec32, Fp, V, stride, s->d_nsolve, s->d_rhs, s->nmax, nz,

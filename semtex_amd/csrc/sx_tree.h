@@ -41,17 +41,14 @@ struct TreeLevel {
 };
 
 // A workgroup's share of a level: nf consecutive fronts of one class (their
-// right-hand sides are the columns), the 16-row blocks [rb0, rb0 + 4 / kw)
-// of the operator, the k steps split over kw wavefronts.  Everything the
-// kernel addresses by is here, so its loads depend on this one.
+// right-hand sides are the columns), the 16-row blocks [rb0, rb0 + nrb) of
+// the operator, the k steps of a block split over kw wavefronts.  Everything
+// the kernel addresses by is here, so its loads depend on this one.
 struct TreeItem {
-  int k, b, nf, rb0, kw, src;
+  int k, b, nf, rb0, nrb, kw, src;
   int offk, offb, offn;        // of the first front; front j of the tile: + j k, + j b, + j (k + b)
-  int pad;
   long long op;                // the class's operator (doubles per mode)
-  long long pad2;
 };
-static_assert (sizeof (TreeItem) == 56 || sizeof (TreeItem) == 64, "work items are read whole");
 
 struct TreePlan {
   std::vector<TreeLevel> lev;      // lev[0]: the root
@@ -69,7 +66,7 @@ struct TreePlan {
   std::vector<int> perm;
   size_t slots = 0;
   std::vector<TreeItem> item;
-  int W = 2;                       // 2, 4 or 8
+  int W = 4;                       // 4 or 8
   int nsolve = 0;                  // unknowns (= gk.size())
   size_t ops = 0;                  // operator doubles per mode
   double est_us = 0.0;             // the cost the level cuts were chosen by

@@ -304,130 +304,158 @@ __global__ __launch_bounds__(256) void k_tree_level (TreeArgs T)
   const int K = DIR == T_DOWN ? n : k, rows = DIR == T_UP ? it.b : k;
   const int np = (K + 7) / 8;
   const int ncol = it.nf * nr, ldx = ncol | 1;
-  const int kw = it.kw, kp = wave & (kw - 1), rb = it.rb0 + wave / kw;
-  const bool active = 16 * rb < rows;
+  // wavefront: k steps [q0, q1) of the row blocks rw, rw + step, ...
+  const int kw = it.kw, kp = wave & (kw - 1), step = 4 / kw, rw = wave / kw;
+  const int turns = (it.nrb + step - 1) / step;
   const double2* A = (const double2*) (T.ops + (size_t) mode * T.os + it.op) +
-                     (size_t) rb * np * 64 + lane;
-  const int q0 = np * kp / kw, q1 = active ? np * (kp + 1) / kw : 0;
+                     (size_t) (it.rb0 + rw) * np * 64 + lane;
+  const int q0 = np * kp / kw, q1 = np * (kp + 1) / kw;
   constexpr int U = 8;
   double2 a[U];
 #pragma unroll
-  for (int u = 0; u < U; u++) a[u] = q0 + u < q1 ? A[(size_t) (q0 + u) * 64] : make_double2 (0.0, 0.0);
-  // this lane's outputs: rows 16 rb + 4 i + lane/16 of column lane%16
+  for (int u = 0; u < U; u++)
+    a[u] = rw < it.nrb && q0 + u < q1 ? A[(size_t) (q0 + u) * 64] : make_double2 (0.0, 0.0);
+  // the column operand [k rows padded to 8][ldx]; G entries a thread in
+  // flight (entry e: row e % K of column e / K, by a float quotient that is
+  // exact for K * 16 < 2^16 entries)
   const size_t mrow = (size_t) mode * nr;
-  const int col = min (lane & 15, ncol - 1), oj = col / nr;
-  const size_t orow = mrow + col % nr;
-  const bool out = active && kp == 0 && (lane & 15) < ncol;
-  double base[4];
-  int to[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int row = 16 * rb + 4 * i + (lane >> 4);
-    const bool ok = out && row < rows;
-    to[i] = -1;
-    base[i] = 0.0;
-    if (DIR == T_UP) {
-      if (ok) to[i] = T.tgt[it.offb + oj * it.b + row];
-      if (ok && it.src) {
-        const double2* c = (const double2*) (T.cb + orow * T.slots) +
-                           (size_t) (it.offn + oj * n + k + row) * (W / 2);
-        double2 w[W / 2];
-#pragma unroll
-        for (int q = 0; q < W / 2; q++) w[q] = c[q];
-#pragma unroll
-        for (int q = 0; q < W / 2; q++) base[i] += w[q].x + w[q].y;
-      }
-    } else if (ok) {
-      to[i] = T.gk[it.offk + oj * k + row];
-    }
-  }
-  // the column operand [k rows padded to 8][ldx], chunks of 64 rows of a column
-  const int Kp = np * 8, nk = (Kp + 63) / 64, nc = nk * ncol;
+  const int Kp = np * 8, ne = K * ncol;
+  const float rK = 1.0f / (float) K;
   constexpr int G = DIR == T_DOWN ? 8 : 6;
-  for (int c0 = wave; c0 < nc; c0 += 4 * G) {
+  for (int e0 = tid; e0 < ne; e0 += 256 * G) {
     double x[G];
-    int g[G];
+    int g[G], cl[G], kk[G];
+    size_t r[G];
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      const int e = min (e0 + 256 * u, ne - 1);
+      cl[u] = (int) (((float) e + 0.5f) * rK);
+      kk[u] = e - cl[u] * K;
+      const int j = cl[u] / nr;
+      r[u] = mrow + cl[u] - j * nr;
+      g[u] = j;
+    }
     if (DIR == T_DOWN) {
+      int node[G];
+#pragma unroll
+      for (int u = 0; u < G; u++)
+        node[u] = T.gb[it.offb + (kk[u] < k ? 0 : g[u] * it.b + kk[u] - k)];
 #pragma unroll
       for (int u = 0; u < G; u++) {
-        const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
-        g[u] = c < nc && kk >= k && kk < n ? T.gb[it.offb + (cl / nr) * it.b + kk - k] : ns;
+        const double* p = kk[u] < k ? T.v + r[u] * T.nsp + it.offk + g[u] * k + kk[u]
+                                    : T.rhs + r[u] * T.nmax + min (node[u], ns - 1);
+        x[u] = *p;
       }
 #pragma unroll
-      for (int u = 0; u < G; u++) {
-        const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
-        const size_t r = mrow + cl % nr;
-        x[u] = 0.0;
-        if (c < nc && kk < k) x[u] = T.v[r * T.nsp + it.offk + (cl / nr) * k + kk];
-        else if (g[u] < ns) x[u] = T.rhs[r * T.nmax + g[u]];
-      }
+      for (int u = 0; u < G; u++)
+        if (kk[u] >= k && node[u] >= ns) x[u] = 0.0;
     } else {
       double2 w[G][W / 2];
 #pragma unroll
       for (int u = 0; u < G; u++) {
-        const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
-        const size_t r = mrow + cl % nr;
-        const bool ok = c < nc && kk < k;
-        x[u] = ok ? T.in[r * T.nsp + it.offk + (cl / nr) * k + kk] : 0.0;
-        const double2* cb = (const double2*) (T.cb + r * T.slots) +
-                            (size_t) (it.offn + (cl / nr) * n + kk) * (W / 2);
+        x[u] = T.in[r[u] * T.nsp + it.offk + g[u] * k + kk[u]];
+        if (it.src) {
+          const double2* cb = (const double2*) (T.cb + r[u] * T.slots) +
+                              (size_t) (it.offn + g[u] * n + kk[u]) * (W / 2);
 #pragma unroll
-        for (int q = 0; q < W / 2; q++) w[u][q] = ok && it.src ? cb[q] : make_double2 (0.0, 0.0);
+          for (int q = 0; q < W / 2; q++) w[u][q] = cb[q];
+        }
       }
 #pragma unroll
       for (int u = 0; u < G; u++) {
-        const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
+        if (it.src)
 #pragma unroll
-        for (int q = 0; q < W / 2; q++) x[u] += w[u][q].x + w[u][q].y;
-        if (DIR == T_UP && it.rb0 == 0 && c < nc && kk < k)
-          T.v[(mrow + cl % nr) * T.nsp + it.offk + (cl / nr) * k + kk] = x[u];
+          for (int q = 0; q < W / 2; q++) x[u] += w[u][q].x + w[u][q].y;
+        if (DIR == T_UP && it.rb0 == 0 && e0 + 256 * u < ne)
+          T.v[r[u] * T.nsp + it.offk + g[u] * k + kk[u]] = x[u];
       }
     }
 #pragma unroll
-    for (int u = 0; u < G; u++) {
-      const int c = c0 + 4 * u, cl = c / nk, kk = 64 * (c % nk) + lane;
-      if (c < nc && kk < Kp) sm[kk * ldx + cl] = x[u];
-    }
+    for (int u = 0; u < G; u++)
+      if (e0 + 256 * u < ne) sm[kk[u] * ldx + cl[u]] = x[u];
   }
-  __syncthreads ();
-  // columns past ncol read a valid column (their results are not stored)
+  for (int e = tid; e < (Kp - K) * ldx; e += 256) sm[K * ldx + e] = 0.0;
+  // this lane's outputs: rows 16 rb + 4 i + lane/16 of column lane%16
+  // (columns past ncol read a valid one, their results are not stored)
+  const int col = min (lane & 15, ncol - 1), oj = col / nr;
+  const size_t orow = mrow + col - oj * nr;
+  const bool mine = kp == 0 && (lane & 15) < ncol;
   const double* X = sm + (lane >> 4) * ldx + col;
-  v4d acc0 = {}, acc1 = {};
-  for (int q = q0; q < q1; q += U) {
-    double2 b[U];
+  double* red = sm + (size_t) Kp * ldx;
+  __syncthreads ();
+  for (int t = 0; t < turns; t++) {
+    const int rl = rw + t * step, rb = it.rb0 + rl;
+    const bool active = rl < it.nrb, more = rl + step < it.nrb;
+    double base[4];
+    int to[4];
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      b[u] = a[u];
-      if (q + U + u < q1) a[u] = A[(size_t) (q + U + u) * 64];
+    for (int i = 0; i < 4; i++) {
+      const int row = 16 * rb + 4 * i + (lane >> 4);
+      const bool ok = active && mine && row < rows;
+      to[i] = -1;
+      base[i] = 0.0;
+      if (DIR == T_UP) {
+        if (ok) to[i] = T.tgt[it.offb + oj * it.b + row];
+        if (ok && it.src) {
+          const double2* c = (const double2*) (T.cb + orow * T.slots) +
+                             (size_t) (it.offn + oj * n + k + row) * (W / 2);
+          double2 w[W / 2];
+#pragma unroll
+          for (int q = 0; q < W / 2; q++) w[q] = c[q];
+#pragma unroll
+          for (int q = 0; q < W / 2; q++) base[i] += w[q].x + w[q].y;
+        }
+      } else if (ok) {
+        to[i] = T.gk[it.offk + oj * k + row];
+      }
+    }
+    v4d acc0 = {}, acc1 = {};
+    if (active) {
+      const double2* An = A + (size_t) step * np * 64;
+      for (int q = q0; q < q1; q += U) {
+        double2 b[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) b[u] = a[u];
+        if (q + U < q1) {
+#pragma unroll
+          for (int u = 0; u < U; u++)
+            if (q + U + u < q1) a[u] = A[(size_t) (q + U + u) * 64];
+        } else if (more) {             // the next row block's first steps
+#pragma unroll
+          for (int u = 0; u < U; u++)
+            if (q0 + u < q1) a[u] = An[(size_t) (q0 + u) * 64];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          if (q + u < q1) {
+            const double* x = X + (size_t) 8 * (q + u) * ldx;
+            acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64 (b[u].x, x[0], acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64 (b[u].y, x[4 * ldx], acc1, 0, 0, 0);
+          }
+      }
+      A = An;
+    }
+    v4d acc = acc0 + acc1;
+    if (kw > 1) {
+      if (t) __syncthreads ();         // the last turn's partial tiles are read
+      if (kp)
+#pragma unroll
+        for (int i = 0; i < 4; i++) red[(wave * 4 + i) * 64 + lane] = acc[i];
+      __syncthreads ();
+      if (kp == 0)
+        for (int p = 1; p < kw; p++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) acc[i] += red[((wave + p) * 4 + i) * 64 + lane];
     }
 #pragma unroll
-    for (int u = 0; u < U; u++)
-      if (q + u < q1) {
-        const double* x = X + (size_t) 8 * (q + u) * ldx;
-        acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64 (b[u].x, x[0], acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64 (b[u].y, x[4 * ldx], acc1, 0, 0, 0);
+    for (int i = 0; i < 4; i++) {
+      if (to[i] < 0) continue;
+      if (DIR == T_UP) {
+        T.cb[orow * T.slots + to[i]] = base[i] - acc[i];
+      } else if (to[i] < ns) {
+        T.rhs[orow * T.nmax + to[i]] = acc[i];
+        if (T.sum) T.sum[orow * T.nmax + to[i]] += acc[i];
       }
-  }
-  v4d acc = acc0 + acc1;
-  if (kw > 1) {
-    double* red = sm + (size_t) Kp * ldx;
-    if (kp)
-#pragma unroll
-      for (int i = 0; i < 4; i++) red[(wave * 4 + i) * 64 + lane] = acc[i];
-    __syncthreads ();
-    if (kp == 0)
-      for (int p = 1; p < kw; p++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc[i] += red[((wave + p) * 4 + i) * 64 + lane];
-  }
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if (to[i] < 0) continue;
-    if (DIR == T_UP) {
-      T.cb[orow * T.slots + to[i]] = base[i] - acc[i];
-    } else if (to[i] < ns) {
-      T.rhs[orow * T.nmax + to[i]] = acc[i];
-      if (T.sum) T.sum[orow * T.nmax + to[i]] += acc[i];
     }
   }
 }
@@ -614,8 +642,7 @@ static int sweep (const TreeDev* t, TreeArgs T, int nm, int nr, hipStream_t st)
   T.xcd = nm >= 32 || (nm >= 8 && nm % 8 == 0);
   auto launch = [&] (auto kern, int first, int count, size_t lds) {
     if (!count) return (int) SX_OK;
-    SX_HIP (hipFuncSetAttribute ((const void*) kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int) lds));
+    if (int rc = lds_limit ((const void*) kern, lds)) return rc;
     T.item = t->item + first;
     T.nitem = count;
     const int blocks = count * (T.xcd ? (nm + 7) / 8 * 8 : nm);
@@ -633,9 +660,8 @@ static int sweep (const TreeDev* t, TreeArgs T, int nm, int nr, hipStream_t st)
              : j      ? launch (k_tree_level<T_DOWN, W>, first, count, lds)
                       : launch (k_tree_level<T_ROOT, W>, first, count, lds);
     };
-    return P.W == 2   ? with (std::integral_constant<int, 2> {})
-           : P.W == 4 ? with (std::integral_constant<int, 4> {})
-                      : with (std::integral_constant<int, 8> {});
+    return P.W == 4 ? with (std::integral_constant<int, 4> {})
+                    : with (std::integral_constant<int, 8> {});
   };
   for (int j = nl - 1; j > 0; j--)
     if (int rc = level (j, 0)) return rc;

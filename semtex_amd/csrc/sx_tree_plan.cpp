@@ -176,9 +176,24 @@ int tile_fronts (int K, int nr)
   return nf;
 }
 
-// wavefronts that share the k steps of one 16-row block: enough that each
-// keeps its part of the operator in flight at once
-int k_split (int pairs) { return pairs <= 10 ? 1 : pairs <= 24 ? 2 : 4; }
+// How a tile's row blocks go to workgroups.  With workgroups to spare
+// (WG_FILL, three a CU) one takes every block of a tile, four at a time, so
+// the columns are gathered once; with few tiles the blocks are dealt out
+// and the k steps of a block split over wavefronts, as far as each still
+// keeps its part of the operator in flight at once.
+constexpr int WG_FILL = 768;
+void split_rows (int blocks, int pairs, long long tiles, int* nrb, int* kw)
+{
+  const int quads = (blocks + 3) / 4;
+  if (tiles * quads >= WG_FILL) {
+    const int parts = (int) std::min<long long> ((WG_FILL + tiles - 1) / tiles, quads);
+    *kw = 1;
+    *nrb = 4 * ((quads + parts - 1) / parts);
+    return;
+  }
+  *kw = pairs <= 10 ? 1 : pairs <= 24 ? 2 : 4;
+  *nrb = 4 / *kw;
+}
 
 }  // namespace
 
@@ -393,7 +408,7 @@ bool tree_plan (const sx_mesh* m, int nmodes, TreePlan& P)
     }
   }
   if (W > 8) return false;
-  P.W = W <= 2 ? 2 : W <= 4 ? 4 : 8;
+  P.W = W <= 4 ? 4 : 8;
   P.slots = on * P.W;
   if (P.slots >= ((size_t) 1 << 31)) return false;
   for (auto& t : to) P.tgt.push_back (t.first * P.W + t.second);
@@ -418,22 +433,26 @@ bool tree_plan (const sx_mesh* m, int nmodes, TreePlan& P)
         (dir ? L.it_b : L.it_f)[q] = (int) P.item.size ();
         size_t lds = 0;
         const std::vector<int>& fr = level_fronts[j];
-        for (size_t i0 = 0; i0 < fr.size ();) {
-          const int c = fcls[fr[i0]];
-          const TreeClass& C = P.cls[c];
+        std::vector<std::pair<size_t, size_t>> tile;
+        for (size_t i0 = 0, i1; i0 < fr.size (); i0 = i1) {
+          const TreeClass& C = P.cls[fcls[fr[i0]]];
+          const int cap = tile_fronts (C.k + C.b, nr);
+          for (i1 = i0; i1 < fr.size () && fcls[fr[i1]] == fcls[fr[i0]] && (int) (i1 - i0) < cap;) i1++;
+          tile.push_back ({i0, i1});
+        }
+        for (auto& t : tile) {
+          const int f = fr[t.first], n = (int) (t.second - t.first);
+          const TreeClass& C = P.cls[fcls[f]];
           const int K = dir && j ? C.k + C.b : C.k, rows = dir ? C.k : C.b;
-          const int cap = tile_fronts (K, nr), kw = k_split ((K + 7) / 8);
-          size_t i1 = i0;
-          while (i1 < fr.size () && fcls[fr[i1]] == c && (int) (i1 - i0) < cap) i1++;
-          for (int rb = 0; 16 * rb < rows; rb += 4 / kw)
-            P.item.push_back ({C.k, C.b, (int) (i1 - i0), rb, kw, L.src, offk[fr[i0]],
-                               offb[fr[i0]], offn[fr[i0]], 0, (long long) (dir ? C.mb : C.mf), 0});
+          int nrb, kw;
+          split_rows ((rows + 15) / 16, (K + 7) / 8, (long long) tile.size () * nmodes, &nrb, &kw);
+          for (int rb = 0; 16 * rb < rows; rb += nrb)
+            P.item.push_back ({C.k, C.b, n, rb, std::min (nrb, (rows + 15) / 16 - rb), kw, L.src,
+                               offk[f], offb[f], offn[f], (long long) (dir ? C.mb : C.mf)});
           // the column operand, k rows padded to whole pairs of steps, and
           // the partial tiles of split k ranges
-          lds = std::max (lds, sizeof (double) * ((size_t) (K + 7) / 8 * 8 *
-                                                  (((int) (i1 - i0) * nr) | 1) +
+          lds = std::max (lds, sizeof (double) * ((size_t) (K + 7) / 8 * 8 * ((n * nr) | 1) +
                                                   (kw > 1 ? 4 * 256 : 0)));
-          i0 = i1;
         }
         (dir ? L.nit_b : L.nit_f)[q] = (int) P.item.size () - (dir ? L.it_b : L.it_f)[q];
         (dir ? L.lds_b : L.lds_f)[q] = lds;
