@@ -19,10 +19,13 @@
 #include <vector>
 
 #include "sx_internal.h"
+#include "sx_spd.h"
 
 using namespace sx;
 
 namespace {
+
+typedef double v4d __attribute__ ((ext_vector_type (4)));
 
 constexpr double EPSDP = 6.0e-14;   // femlib/cfemdef.h
 constexpr double EPSSP = 6.0e-7;
@@ -187,6 +190,123 @@ __global__ __launch_bounds__(256) void k_elem_sc (
 #undef HII
 }
 
+// The same with the interior block in LDS, inverted there by blocked
+// Gauss-Jordan on FP64 MFMA tiles (spd_invert): up to N_P = 12, whose block
+// (112 x 114 doubles with its padding) is the largest that fits.  k_elem_sc
+// walks its columns through global memory, three barriers each: 184 us at
+// N_P = 8, 645 us at N_P = 10.
+constexpr int ESC_NPMAX = 12;
+size_t esc_lds (int np)
+{
+  const int N = ((np - 2) * (np - 2) + 15) / 16 * 16, LD = N + 2;
+  return sizeof (double) * ((size_t) N * LD + 16 * LD + 16 * 17 + 6 * np * np) +
+         sizeof (int) * np * np;
+}
+
+__global__ __launch_bounds__(256) void k_elem_sc_lds (
+    int np, int nclass, int cyl, double lambda2, const double* __restrict__ betak2,
+    const double* __restrict__ cgeo, const double* __restrict__ Dg,
+    const int* __restrict__ emap_g, double* ws, double* S, double* Bm,
+    double* Hinv, int* status)
+{
+  extern __shared__ double sm[];
+  __shared__ int s_bad, s_hasQ3;
+  const int npnp = np * np, next = 4 * (np - 1), nint = npnp - next;
+  const int N = (nint + 15) / 16 * 16, LD = N + 2;
+  const int blk = blockIdx.x, mode = blk / nclass, cls = blk % nclass;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  double* P = sm;                          // [N][LD]
+  double* W = P + (size_t) N * LD;         // [16][LD]
+  double* Di = W + 16 * LD;                // [16][17]
+  double* D = Di + 16 * 17;                // [npnp]
+  double* G = D + npnp;                    // [5][npnp]
+  int* emap = (int*) (G + 5 * npnp);
+  const double* geo = cgeo + (size_t) cls * NGEO * npnp;
+  if (tid == 0) { s_bad = 0; s_hasQ3 = 0; }
+  __syncthreads ();
+  for (int k = tid; k < npnp; k += 256) {
+    D[k] = Dg[k];
+    emap[k] = emap_g[k];
+    G[0 * npnp + k] = geo[G_Q1 * npnp + k];
+    G[1 * npnp + k] = geo[G_Q2 * npnp + k];
+    const double q3 = geo[G_Q3 * npnp + k];
+    G[2 * npnp + k] = q3;
+    if (q3 != 0.0) s_hasQ3 = 1;
+    G[3 * npnp + k] = geo[G_Q4 * npnp + k];
+    G[4 * npnp + k] = geo[G_Y * npnp + k];
+  }
+  __syncthreads ();
+  const bool hasQ3 = s_hasQ3 != 0;
+  const double bk2 = betak2[mode];
+  auto entry = [&] (int a, int b) {
+    return helm_entry (np, emap[a], emap[b], G, G + npnp, G + 2 * npnp, G + 3 * npnp,
+                       G + 4 * npnp, D, lambda2, bk2, cyl, hasQ3);
+  };
+  for (int i = tid; i < N * N; i += 256) {
+    const int a = i / N, b = i % N;
+    P[a * LD + b] = a < nint && b < nint ? entry (next + a, next + b) : a == b ? 1.0 : 0.0;
+  }
+  // hbi, kept in this block's workspace
+  double* Hb = ws + (size_t) blk * (npnp * npnp + nint * nint);
+  for (int i = tid; i < next * nint; i += 256) Hb[i] = entry (i / nint, next + i % nint);
+  __syncthreads ();
+  spd_invert (P, LD, N / 16, W, Di, &s_bad);
+  if (s_bad) { if (tid == 0) atomicExch (status, 1); return; }
+  double* Hi = Hinv + ((size_t) mode * nclass + cls) * nint * nint;
+  for (int i = tid; i < nint * nint; i += 256) Hi[i] = P[(i / nint) * LD + i % nint];
+  // Bm = hbi inv(hii), then S = hbb - Bm hbi^T, 16x16 tiles
+  double* B = Bm + ((size_t) mode * nclass + cls) * next * nint;
+  const int ne = (next + 15) / 16, nk = N / 4, lr = lane & 15, lq = lane >> 4;
+  for (int t = wave; t < ne * (N / 16); t += 4) {
+    const int i0 = 16 * (t % ne), j0 = 16 * (t / ne), row = min (i0 + lr, next - 1);
+    v4d acc = {};
+    for (int s = 0; s < nk; s++) {
+      const int kk = 4 * s + lq;
+      const double h = kk < nint ? Hb[(size_t) row * nint + kk] : 0.0;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64 (h, P[kk * LD + j0 + lr], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int a = i0 + 4 * r + lq, b = j0 + lr;
+      if (a < next && b < nint) B[(size_t) a * nint + b] = acc[r];
+    }
+  }
+  __syncthreads ();
+  double* So = S + ((size_t) mode * nclass + cls) * next * next;
+  for (int t = wave; t < ne * ne; t += 4) {
+    const int i0 = 16 * (t % ne), j0 = 16 * (t / ne);
+    const int ra = min (i0 + lr, next - 1), rb = min (j0 + lr, next - 1);
+    v4d acc = {};
+    for (int s = 0; s < nk; s++) {
+      const int kk = min (4 * s + lq, nint - 1);
+      const double b = B[(size_t) ra * nint + kk], h = Hb[(size_t) rb * nint + kk];
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64 (4 * s + lq < nint ? b : 0.0, h, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int a = i0 + 4 * r + lq, b = j0 + lr;
+      if (a < next && b < next) So[(size_t) a * next + b] = entry (a, b) - acc[r];
+    }
+  }
+}
+
+int elem_sc (const sx_mesh* m, int nmodes, double lambda2, const double* d_betak2, double* ws,
+             double* S, double* Bm, double* Hinv, int* d_status, hipStream_t st)
+{
+  const dim3 grid ((unsigned) ((size_t) nmodes * m->nclass));
+  if (m->np <= ESC_NPMAX) {
+    const size_t lds = esc_lds (m->np);
+    if (int rc = lds_limit ((const void*) k_elem_sc_lds, lds)) return rc;
+    hipLaunchKernelGGL (k_elem_sc_lds, grid, dim3 (256), lds, st, m->np, m->nclass, m->cyl,
+                        lambda2, d_betak2, m->d_cgeo, m->d_D, m->d_emap, ws, S, Bm, Hinv, d_status);
+  } else {
+    hipLaunchKernelGGL (k_elem_sc, grid, dim3 (256), 0, st, m->np, m->nclass, m->cyl, lambda2,
+                        d_betak2, m->d_cgeo, m->d_D, m->d_emap, ws, S, Bm, Hinv, d_status);
+  }
+  SX_HIP (hipGetLastError ());
+  return SX_OK;
+}
+
 __global__ void k_band_assemble (int npairs, const long long* __restrict__ ppos,
                                  const int* __restrict__ pmn,
                                  const int* __restrict__ pptr,
@@ -338,7 +458,6 @@ __host__ __device__ inline TileShape con_shape (int np, bool mf)
   const int next = 4 * (np - 1), nint = np * np - next;
   return mf ? TileShape {pad16 (next), pad4 (nint)} : TileShape {pad4 (next), nint};
 }
-typedef double v4d __attribute__ ((ext_vector_type (4)));
 
 // v_mfma_f64_16x16x4f64, D += A B for one 16x16 output tile: lane l
 // supplies A[l%16][k + l/16] and B[k + l/16][l%16]; D[4r + l/16][l%16] is
@@ -1614,10 +1733,9 @@ int msys_use_band (sx_msys* s)
       hipMemset (d_status, 0, sizeof (int) * (s->nmodes + 1)) != hipSuccess) {
     rc = hip_fail (hipErrorOutOfMemory, "msys_use_band");
   } else {
-    hipLaunchKernelGGL (k_elem_sc, dim3 ((unsigned) nmc), dim3 (256), 0, nullptr, m->np,
-                        m->nclass, m->cyl, s->lambda2, s->d_betak2, m->d_cgeo, m->d_D, m->d_emap,
-                        buf, buf + nws, buf + nws + nS, buf + nws + nS + nB, d_status + s->nmodes);
-    rc = band_build (s, buf + nws, nullptr, d_status);
+    rc = elem_sc (m, s->nmodes, s->lambda2, s->d_betak2, buf, buf + nws, buf + nws + nS,
+                  buf + nws + nS + nB, d_status + s->nmodes, nullptr);
+    if (!rc) rc = band_build (s, buf + nws, nullptr, d_status);
   }
   (void) hipFree (buf);
   (void) hipFree (d_status);
@@ -1696,10 +1814,9 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
   TRY (hipMalloc (&d_status, sizeof (int) * (num_modes + 1)));
   TRY (hipMemsetAsync (d_status, 0, sizeof (int) * (num_modes + 1), st));
 
-  hipLaunchKernelGGL (k_elem_sc, dim3 ((unsigned) nmc), dim3 (256), 0, st, m->np,
-                      m->nclass, m->cyl, lambda2, s->d_betak2, m->d_cgeo, m->d_D,
-                      m->d_emap, d_ws, d_S, s->d_Bm, s->d_Hinv, d_status + num_modes);
-  TRY (hipGetLastError ());
+  if ((rc = elem_sc (m, num_modes, lambda2, s->d_betak2, d_ws, d_S, s->d_Bm, s->d_Hinv,
+                     d_status + num_modes, st)))
+    return fail (rc);
   if (tiled_ok (m)) {
     s->tile_mf = tiled_mfma (m) ? 1 : 0;
     if (const char* e = std::getenv ("SX_TILE_MFMA")) s->tile_mf = s->tile_mf && std::atoi (e);

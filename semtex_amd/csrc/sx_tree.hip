@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "sx_internal.h"
+#include "sx_spd.h"
 #include "sx_tree.h"
 
 namespace sx {
@@ -77,8 +78,11 @@ __global__ __launch_bounds__(256) void k_tree_assemble (
 // One step of the in-place Gauss-Jordan elimination of a front's first k
 // unknowns, pivots P = [p0, p0 + pb): this kernel inverts the pivot block
 // and forms, for a tile of 64 columns, R = F_P (the rows as they are) and
-// W = F_PP^-1 F_P (F_PP^-1 itself in the columns of P) into RW.  Every
-// tile's workgroup inverts the block for itself, so a step is two launches.
+// W = F_PP^-1 F_P (F_PP^-1 itself in the columns of P) into RW (rows of ldw,
+// zero past n).  Every tile's workgroup inverts the block for itself, so a
+// step is two launches.  It is bound by that inversion's chain of pivots
+// (one wavefront, 16 at a time): 38 us a step with the 64 pivots one after
+// another, a barrier each.
 __global__ __launch_bounds__(256) void k_tree_panel (
     const TreeClass* __restrict__ cls, int cls0, const double* __restrict__ F, size_t fs,
     double* RW, int ldw, int step, int* status)
@@ -87,82 +91,49 @@ __global__ __launch_bounds__(256) void k_tree_panel (
   const int mode = blockIdx.z, n = C.k + C.b, p0 = TB * step;
   const int pb = min (TB, C.k - p0), c0 = TB * blockIdx.x;
   if (pb <= 0 || c0 >= n) return;
-  __shared__ double piv[TB * (TB + 1)], Rs[TB * (TB + 2)], lines[2][2][TB];
-  __shared__ int s_bad;
+  constexpr int LD = TB + 2;
+  __shared__ double piv[TB * LD], Rs[TB * LD], Wb[16 * LD], D[16 * 17];
+  __shared__ int bad;
   const double* Fm = F + (size_t) mode * fs + C.foff;
-  const int tid = threadIdx.x, ti = tid >> 4, tj = tid & 15;
-  if (tid == 0) s_bad = 0;
-  // rows of P, columns [c0, c0 + 64)
-  for (int i = tid; i < TB * TB; i += 256) {
-    const int r = i >> 6, c = i & 63;
-    Rs[r * (TB + 2) + c] = (r < pb && c0 + c < n) ? Fm[(size_t) (p0 + r) * n + c0 + c] : 0.0;
-  }
-  double a[4][4];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  if (tid == 0) bad = 0;
+  // the pivot block (identity past pb) and the rows of P in this tile's
+  // columns, every load unconditional
+  double x[16], y[16];
 #pragma unroll
-  for (int r = 0; r < 4; r++)
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      const int i = 4 * ti + r, j = 4 * tj + c;
-      a[r][c] = (i < pb && j < pb) ? Fm[(size_t) (p0 + i) * n + p0 + j] : (i == j ? 1.0 : 0.0);
-    }
-  // Gauss-Jordan inversion of the (symmetric positive definite) block, a
-  // 4x4 patch per thread; the pivot row and column pass through LDS
-  for (int t4 = 0; t4 < TB / 4 && 4 * t4 < pb; t4++) {
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int t = 4 * t4 + u, h = u & 1;
-      if (ti == t4)
-#pragma unroll
-        for (int c = 0; c < 4; c++) lines[h][0][4 * tj + c] = a[u][c];
-      if (tj == t4)
-#pragma unroll
-        for (int r = 0; r < 4; r++) lines[h][1][4 * ti + r] = a[r][u];
-      __syncthreads ();
-      if (t >= pb) continue;
-      const double p = lines[h][0][t];
-      if (tid == 0 && !(p > 0.0) && !s_bad) s_bad = p0 + t + 1;
-      const double d = 1.0 / p;
-      double row[4], col[4];
-#pragma unroll
-      for (int c = 0; c < 4; c++) row[c] = lines[h][0][4 * tj + c] * d;
-#pragma unroll
-      for (int r = 0; r < 4; r++) col[r] = lines[h][1][4 * ti + r];
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const bool ir = ti == t4 && r == u, jc = tj == t4 && c == u;
-          a[r][c] = ir ? (jc ? d : row[c]) : jc ? -col[r] * d : a[r][c] - col[r] * row[c];
-        }
-    }
+  for (int q = 0; q < 16; q++) {
+    const int r = 4 * q + wave, rr = p0 + min (r, pb - 1);
+    x[q] = Fm[(size_t) rr * n + p0 + min (lane, pb - 1)];
+    y[q] = Fm[(size_t) rr * n + min (c0 + lane, n - 1)];
   }
 #pragma unroll
-  for (int r = 0; r < 4; r++)
-#pragma unroll
-    for (int c = 0; c < 4; c++) piv[(4 * ti + r) * (TB + 1) + 4 * tj + c] = a[r][c];
+  for (int q = 0; q < 16; q++) {
+    const int r = 4 * q + wave;
+    piv[r * LD + lane] = r < pb && lane < pb ? x[q] : r == lane ? 1.0 : 0.0;
+    Rs[r * LD + lane] = r < pb && c0 + lane < n ? y[q] : 0.0;
+  }
   __syncthreads ();
-  if (tid == 0 && s_bad && blockIdx.x == 0) atomicMax (status + mode, s_bad);
+  spd_invert (piv, LD, (pb + 15) / 16, Wb, D, &bad);
+  if (tid == 0 && bad && blockIdx.x == 0) atomicMax (status + mode, p0 + bad);
   double* Rg = RW + ((size_t) mode * gridDim.y + blockIdx.y) * 2 * TB * ldw;
   double* Wg = Rg + (size_t) TB * ldw;
-  const int wave = tid >> 6, lane = tid & 63;
   v4d acc[4] = {};
 #pragma unroll
   for (int s = 0; s < TB / 4; s++) {
-    const double av = piv[(16 * wave + (lane & 15)) * (TB + 1) + 4 * s + (lane >> 4)];
+    const double av = piv[(16 * wave + (lane & 15)) * LD + 4 * s + (lane >> 4)];
 #pragma unroll
     for (int q = 0; q < 4; q++)
       acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64 (
-          av, Rs[(4 * s + (lane >> 4)) * (TB + 2) + 16 * q + (lane & 15)], acc[q], 0, 0, 0);
+          av, Rs[(4 * s + (lane >> 4)) * LD + 16 * q + (lane & 15)], acc[q], 0, 0, 0);
   }
 #pragma unroll
   for (int q = 0; q < 4; q++)
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int i = 16 * wave + 4 * r + (lane >> 4), j = c0 + 16 * q + (lane & 15);
-      if (j >= n) continue;
-      Rg[(size_t) i * ldw + j] = Rs[i * (TB + 2) + j - c0];
       const int jp = j - p0;
-      Wg[(size_t) i * ldw + j] = jp >= 0 && jp < pb ? piv[i * (TB + 1) + jp] : acc[q][r];
+      Rg[(size_t) i * ldw + j] = Rs[i * LD + j - c0];
+      Wg[(size_t) i * ldw + j] = jp >= 0 && jp < pb ? piv[i * LD + jp] : acc[q][r];
     }
 }
 
@@ -172,6 +143,8 @@ __global__ __launch_bounds__(256) void k_tree_panel (
 //   j in P:         F_ij  = -s_i W_ji
 // with s_i = -1 for unknowns already eliminated (i < p0), +1 otherwise: the
 // matrix stays symmetric up to that sign, so only rows of P are ever read.
+// R and W are padded to whole tiles, so every load is unconditional and
+// issued before the products (46 -> 12 us a step at 96 fronts of 370).
 __global__ __launch_bounds__(256) void k_tree_update (
     const TreeClass* __restrict__ cls, int cls0, double* F, size_t fs,
     const double* __restrict__ RW, int ldw, int step, int nt)
@@ -181,45 +154,58 @@ __global__ __launch_bounds__(256) void k_tree_update (
   const int pb = min (TB, C.k - p0);
   const int i0 = TB * (blockIdx.x / nt), j0 = TB * (blockIdx.x % nt);
   if (pb <= 0 || i0 >= n || j0 >= n) return;
-  __shared__ double Rs[TB * (TB + 2)], Ws[TB * (TB + 2)];
+  constexpr int LD = TB + 2;
+  __shared__ double Rs[TB * LD], Ws[TB * LD];
   const double* Rg = RW + ((size_t) mode * gridDim.y + blockIdx.y) * 2 * TB * ldw;
   const double* Wg = Rg + (size_t) TB * ldw;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  for (int i = tid; i < TB * TB; i += 256) {
-    const int r = i >> 6, c = i & 63;
-    const double v = i0 + c < n ? Rg[(size_t) r * ldw + i0 + c] : 0.0;
-    Rs[r * (TB + 2) + c] = i0 + c < p0 ? -v : v;
-    Ws[r * (TB + 2) + c] = j0 + c < n ? Wg[(size_t) r * ldw + j0 + c] : 0.0;
+  const int wi = 32 * (wave & 1), wj = 32 * (wave >> 1);
+  double* Fm = F + (size_t) mode * fs + C.foff;
+  double x[16], y[16], f[16], wt[16];
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    const size_t r = (size_t) (4 * q + wave) * ldw;
+    x[q] = Rg[r + i0 + lane];
+    y[q] = Wg[r + j0 + lane];
+  }
+  const bool tp = j0 < p0 + pb && j0 + TB > p0;        // the tile holds columns of P
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    const int i = i0 + wi + 16 * (q >> 3) + 4 * (q & 3) + (lane >> 4),
+              j = j0 + wj + 16 * ((q >> 2) & 1) + (lane & 15);
+    f[q] = Fm[(size_t) min (i, n - 1) * n + min (j, n - 1)];
+    wt[q] = tp ? Wg[(size_t) min (max (j - p0, 0), TB - 1) * ldw + i] : 0.0;
+  }
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    const int r = 4 * q + wave;
+    Rs[r * LD + lane] = i0 + lane < p0 ? -x[q] : x[q];
+    Ws[r * LD + lane] = y[q];
   }
   __syncthreads ();
-  const int wi = 32 * (wave & 1), wj = 32 * (wave >> 1);
   v4d acc[2][2] = {};
   const int ks = (pb + 3) / 4;
   for (int s = 0; s < ks; s++) {
-    const double* ra = Rs + (4 * s + (lane >> 4)) * (TB + 2) + wi + (lane & 15);
-    const double* wb = Ws + (4 * s + (lane >> 4)) * (TB + 2) + wj + (lane & 15);
+    const double* ra = Rs + (4 * s + (lane >> 4)) * LD + wi + (lane & 15);
+    const double* wb = Ws + (4 * s + (lane >> 4)) * LD + wj + (lane & 15);
     const double a0 = ra[0], a1 = ra[16], b0 = wb[0], b1 = wb[16];
     acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a0, b0, acc[0][0], 0, 0, 0);
     acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a0, b1, acc[0][1], 0, 0, 0);
     acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a1, b0, acc[1][0], 0, 0, 0);
     acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a1, b1, acc[1][1], 0, 0, 0);
   }
-  double* Fm = F + (size_t) mode * fs + C.foff;
 #pragma unroll
-  for (int x = 0; x < 2; x++)
-#pragma unroll
-    for (int y = 0; y < 2; y++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int il = wi + 16 * x + 4 * r + (lane >> 4), jl = wj + 16 * y + (lane & 15);
-        const int i = i0 + il, j = j0 + jl;
-        if (i >= n || j >= n) continue;
-        const bool ip = i >= p0 && i < p0 + pb, jp = j >= p0 && j < p0 + pb;
-        double* f = Fm + (size_t) i * n + j;
-        if (ip) *f = Wg[(size_t) (i - p0) * ldw + j];
-        else if (jp) *f = (i < p0 ? 1.0 : -1.0) * Wg[(size_t) (j - p0) * ldw + i];
-        else *f -= acc[x][y][r];
-      }
+  for (int q = 0; q < 16; q++) {
+    const int il = wi + 16 * (q >> 3) + 4 * (q & 3) + (lane >> 4),
+              jl = wj + 16 * ((q >> 2) & 1) + (lane & 15);
+    const int i = i0 + il, j = j0 + jl;
+    if (i >= n || j >= n) continue;
+    const bool ip = i >= p0 && i < p0 + pb, jp = j >= p0 && j < p0 + pb;
+    const double v = ip   ? Ws[(i - p0) * LD + jl]
+                     : jp ? (i < p0 ? wt[q] : -wt[q])
+                          : f[q] - acc[q >> 3][(q >> 2) & 1][q & 3];
+    Fm[(size_t) i * n + j] = v;
+  }
 }
 
 // Operators of a level in fragment order.  Forward: rows B, k steps over K,
