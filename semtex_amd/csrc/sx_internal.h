@@ -33,6 +33,19 @@ inline int lds_limit (const void* kern, size_t lds)
   return SX_OK;
 }
 
+// Device blocks of systems and their set-up kept for the next ones: unmapping
+// and mapping one costs 2-6 us a MB, which bounded the making of a system
+// (a changed time step or lambda2).  At most POOL_BYTES in POOL_BLOCKS blocks
+// a device; given back when a device runs out of memory and when the last
+// mesh goes.  block_free: nothing on the GPU uses the block any more (the
+// caller has waited, as hipFree itself would); dev: the device it was
+// allocated on.
+constexpr size_t POOL_BYTES = (size_t) 512 << 20;
+constexpr int POOL_BLOCKS = 8;
+int  block_alloc (void** p, size_t bytes, size_t* size, int* dev);
+void block_free (void* p, size_t size, int dev);
+void block_meshes (int delta);
+
 // GLL rule (femlib/polylib.c:312 zwglj, :513 Dglj), host.
 void gll (int np, double* z, double* w, double* D);
 // edge-major permutation (femlib/mapping.c:46-132), host.
@@ -61,7 +74,10 @@ int    tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always = false)
 void   tree_free (TreeDev* t);
 void   tree_sing_free (TreeSing* g);
 int    tree_workspace (sx_msys* s, int nr);
-int    tree_factor (sx_msys* s, const double* Sel, hipStream_t st, int* d_status);
+size_t tree_ops (const TreeDev* t);                 // doubles per mode of d_tops
+size_t tree_slots (const TreeDev* t);               // and per right-hand side of d_tc
+size_t tree_scratch (const TreeDev* t, int nm);     // doubles
+int    tree_factor (sx_msys* s, const double* Sel, double* buf, hipStream_t st, int* d_status);
 int    tree_solve (const sx_msys* s, int nr, hipStream_t st);
 // A singular mode's refinement: its set-up (s->sing), and around a band
 // solve the right-hand sides kept before and the correction after.
@@ -72,6 +88,8 @@ int    sing_refine (const sx_msys* s, int nr, hipStream_t st);
 // dissection) and its use from now on: the batches plan band sweeps, and
 // their systems' own solves stay equal to the batch's (sx_solver.hip).
 int    msys_use_band (sx_msys* s);
+// Frees a device array of the system unless it lies in its block.
+void   msys_free (sx_msys* s, void* p);
 // Banded FP64 Cholesky of every mode's band, the offset-major sweep copies
 // of the factor and of its reversal (with inverted diagonal blocks), and
 // the two-sweep solve of the right-hand sides in d_rhs ([mode][2][nmax])
@@ -244,6 +262,10 @@ struct sx_msys {
   int* d_tw = nullptr;         //   [nmodes][8] split of every mode
   double* d_rhsb = nullptr;    //   [nmodes][nr][nmaxb] bottom-piece right-hand sides
   int nmaxb = 0;
+  // the arrays a DIRECT system is created with lie in one allocation
+  char* block = nullptr;
+  size_t block_bytes = 0;
+  int block_dev = 0;
   sx::TreeDev* tree = nullptr; // dissection solve: the mesh's plan, null: band only
   int use_tree = 0;            //   solves run it
   sx::TreeSing* sing = nullptr;  // the singular mode's refinement, or null

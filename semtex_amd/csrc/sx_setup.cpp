@@ -213,6 +213,93 @@ static int upload (T** dst, const std::vector<T>& src)
   return SX_OK;
 }
 
+// ---------------------------------------------------------------------------
+// Device block pool (sx_internal.h)
+// ---------------------------------------------------------------------------
+namespace {
+struct Block { int dev; void* p; size_t size; };
+std::mutex pool_mu;
+std::vector<Block> pool;
+int pool_meshes = 0;
+
+void pool_flush (std::vector<Block>& gone, int dev)     // dev < 0: every device
+{
+  for (size_t i = 0; i < pool.size ();)
+    if (dev < 0 || pool[i].dev == dev) {
+      gone.push_back (pool[i]);
+      pool.erase (pool.begin () + i);
+    } else i++;
+}
+}  // namespace
+
+namespace sx {
+
+int block_alloc (void** p, size_t bytes, size_t* size, int* device)
+{
+  int dev = 0;
+  SX_HIP (hipGetDevice (&dev));
+  *device = dev;
+  {
+    std::lock_guard<std::mutex> lock (pool_mu);
+    int best = -1;
+    for (int i = 0; i < (int) pool.size (); i++)
+      if (pool[i].dev == dev && pool[i].size >= bytes && pool[i].size <= 2 * bytes + (1 << 20) &&
+          (best < 0 || pool[i].size < pool[best].size))
+        best = i;
+    if (best >= 0) {
+      *p = pool[best].p;
+      *size = pool[best].size;
+      pool.erase (pool.begin () + best);
+      return SX_OK;
+    }
+  }
+  *size = bytes;
+  hipError_t e = hipMalloc (p, bytes);
+  if (e != hipSuccess) {
+    std::vector<Block> gone;
+    {
+      std::lock_guard<std::mutex> lock (pool_mu);
+      pool_flush (gone, dev);
+    }
+    for (const Block& b : gone) (void) hipFree (b.p);
+    if (!gone.empty ()) {
+      (void) hipGetLastError ();
+      e = hipMalloc (p, bytes);
+    }
+  }
+  return e == hipSuccess ? (int) SX_OK : hip_fail (e, "hipMalloc");
+}
+
+void block_free (void* p, size_t size, int dev)
+{
+  if (!p) return;
+  {
+    std::lock_guard<std::mutex> lock (pool_mu);
+    size_t held = size;
+    int count = 1;
+    for (const Block& b : pool)
+      if (b.dev == dev) { held += b.size; count++; }
+    if (pool_meshes > 0 && held <= POOL_BYTES && count <= POOL_BLOCKS) {
+      pool.push_back ({dev, p, size});
+      return;
+    }
+  }
+  (void) hipFree (p);
+}
+
+void block_meshes (int delta)
+{
+  std::vector<Block> gone;
+  {
+    std::lock_guard<std::mutex> lock (pool_mu);
+    pool_meshes += delta;
+    if (pool_meshes <= 0) pool_flush (gone, -1);
+  }
+  for (const Block& b : gone) (void) hipFree (b.p);
+}
+
+}  // namespace sx
+
 extern "C" int sx_mesh_destroy (sx_mesh_t m)
 {
   if (!m) return SX_OK;
@@ -225,6 +312,7 @@ extern "C" int sx_mesh_destroy (sx_mesh_t m)
   for (void* p : ptrs) if (p) (void) hipFree (p);
   for (TreeDev* t : m->trees) tree_free (t);
   delete m;
+  block_meshes (-1);
   return SX_OK;
 }
 
@@ -249,6 +337,7 @@ extern "C" int sx_mesh_create (int np, int nel, int cyl, const double* x,
       return SX_ERR_ARG;
     }
   sx_mesh* m = new sx_mesh;
+  block_meshes (+1);
   *out = nullptr;
   m->np = np; m->nel = nel; m->cyl = cyl ? 1 : 0;
   m->npnp = np * np; m->next = 4 * (np - 1); m->nint = m->npnp - m->next;

@@ -1637,6 +1637,13 @@ extern "C" int sx_timing_read (double* ms, int* count, int nphase)
 // ===========================================================================
 // C ABI
 // ===========================================================================
+namespace sx {
+void msys_free (sx_msys* s, void* p)
+{
+  if (p && !((char*) p >= s->block && (char*) p < s->block + s->block_bytes)) (void) hipFree (p);
+}
+}  // namespace sx
+
 extern "C" int sx_msys_destroy (sx_msys_t s)
 {
   if (!s) return SX_OK;
@@ -1645,7 +1652,17 @@ extern "C" int sx_msys_destroy (sx_msys_t s)
                   s->d_Hinv32, s->d_bandU, s->d_swF, s->d_swR, s->d_rhs, s->d_G,
                   s->d_work, s->d_pc, s->d_tw, s->d_rhsb, s->d_xch, s->d_xep,
                   s->d_tops, s->d_tb, s->d_tv, s->d_tc};
-  for (void* p : ptrs) if (p) (void) hipFree (p);
+  for (void* p : ptrs) msys_free (s, p);
+  if (s->block) {
+    // the block may serve another system at once: wait for the device, as
+    // freeing it would
+    int dev = 0;
+    (void) hipGetDevice (&dev);
+    if (dev != s->block_dev) (void) hipSetDevice (s->block_dev);
+    (void) hipDeviceSynchronize ();
+    if (dev != s->block_dev) (void) hipSetDevice (dev);
+    block_free (s->block, s->block_bytes, s->block_dev);
+  }
   tree_sing_free (s->sing);
   delete s;
   return SX_OK;
@@ -1784,60 +1801,107 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
   s->band_stride = (size_t) std::max (s->nmax, 1) * ld;
 
   int rc = SX_OK;
-  auto fail = [&] (int r) { sx_msys_destroy (s); return r; };
+  double* d_ws = nullptr;              // set-up scratch, one block
+  size_t ws_bytes = 0;
+  int ws_dev = 0;
+  auto fail = [&] (int r) {
+    if (d_ws) (void) hipFree (d_ws);
+    sx_msys_destroy (s);
+    return r;
+  };
 #define TRY(call) do { hipError_t _e = (call); if (_e != hipSuccess) return fail (hip_fail (_e, #call)); } while (0)
   const size_t nmc = (size_t) num_modes * m->nclass;
-  TRY (hipMalloc (&s->d_betak2, sizeof (double) * num_modes));
-  TRY (hipMalloc (&s->d_nsolve, sizeof (int) * num_modes));
-  TRY (hipMemcpy (s->d_betak2, s->betak2.data (), sizeof (double) * num_modes, hipMemcpyHostToDevice));
-  TRY (hipMemcpy (s->d_nsolve, s->nsolve.data (), sizeof (int) * num_modes, hipMemcpyHostToDevice));
   if (precision == SX_JACPCG) {      // MatrixSys JACPCG: the preconditioner only
+    TRY (hipMalloc (&s->d_betak2, sizeof (double) * num_modes));
+    TRY (hipMalloc (&s->d_nsolve, sizeof (int) * num_modes));
+    TRY (hipMemcpy (s->d_betak2, s->betak2.data (), sizeof (double) * num_modes, hipMemcpyHostToDevice));
+    TRY (hipMemcpy (s->d_nsolve, s->nsolve.data (), sizeof (int) * num_modes, hipMemcpyHostToDevice));
     TRY (hipMalloc (&s->d_G, sizeof (double) * 2 * num_modes * m->nglobal));
     if ((rc = pcg_setup (s, st))) return fail (rc);
     *out = s;
     return SX_OK;
   }
-  TRY (hipMalloc (&s->d_Bm, sizeof (double) * std::max<size_t> (nmc * next * nint, 1)));
-  TRY (hipMalloc (&s->d_Hinv, sizeof (double) * std::max<size_t> (nmc * nint * nint, 1)));
   if ((rc = tree_prepare (m, num_modes, &s->tree))) return fail (rc);
   s->use_tree = s->tree != nullptr;
-  const size_t nrhs = sizeof (double) * num_modes * 2 * std::max (s->nmax, 1);
-  TRY (hipMalloc (&s->d_rhs, nrhs));
-  TRY (hipMalloc (&s->d_G, sizeof (double) * 2 * num_modes * m->nglobal));
-  TRY (hipMemsetAsync (s->d_rhs, 0, nrhs, st));
+  // The system's arrays in one block and the set-up's scratch in another
+  // (block_alloc): two dozen allocations and frees of 10-20 us, and the
+  // unmapping of the large ones, took longer than the GPU did.  The arrays
+  // that start at zero come first, cleared in one go.
+  const bool tiled = tiled_ok (m);
+  s->tile_mf = tiled && tiled_mfma (m) ? 1 : 0;
+  if (const char* e = std::getenv ("SX_TILE_MFMA")) s->tile_mf = s->tile_mf && std::atoi (e);
+  const TileShape R = rec_shape (m->np, s->tile_mf), Cs = con_shape (m->np, s->tile_mf);
+  const size_t nrec = tiled ? (size_t) R.KR * R.NA : 0, ncon = tiled ? (size_t) Cs.KR * Cs.NA : 0;
+  const size_t nrhs = (size_t) num_modes * 2;
+  size_t n = 0;
+  auto take = [] (size_t& at, size_t doubles) {
+    const size_t o = at;
+    at += (std::max<size_t> (doubles, 1) + 31) / 32 * 32;
+    return o;
+  };
+  const size_t o_rhs = take (n, nrhs * std::max (s->nmax, 1));
+  const size_t o_tb = take (n, s->use_tree ? nrhs * m->nsolve : 0),
+               o_tc = take (n, s->use_tree ? nrhs * tree_slots (s->tree) : 0), nzero = n;
+  const size_t o_par = take (n, 2 * (size_t) num_modes), o_G = take (n, nrhs * m->nglobal),
+               o_Bm = take (n, nmc * next * nint), o_Hi = take (n, nmc * nint * nint),
+               o_rec = take (n, nmc * nrec), o_con = take (n, nmc * ncon),
+               o_tv = take (n, s->use_tree ? nrhs * m->nsolve : 0),
+               o_ops = take (n, s->use_tree ? tree_ops (s->tree) * num_modes : 0);
+  if ((rc = block_alloc ((void**) &s->block, sizeof (double) * n, &s->block_bytes, &s->block_dev)))
+    return fail (rc);
+  double* base = (double*) s->block;
+  s->d_rhs = base + o_rhs;
+  s->d_betak2 = base + o_par;
+  s->d_nsolve = (int*) (s->d_betak2 + num_modes);
+  s->d_G = base + o_G;
+  s->d_Bm = base + o_Bm;
+  s->d_Hinv = base + o_Hi;
+  if (tiled) {
+    s->d_Mrec = base + o_rec;
+    s->d_Mcon = base + o_con;
+  }
+  if (s->use_tree) {
+    s->d_tb = base + o_tb;
+    s->d_tc = base + o_tc;
+    s->d_tv = base + o_tv;
+    s->d_tops = base + o_ops;
+  }
+  TRY (hipMemsetAsync (base, 0, sizeof (double) * nzero, st));
+  std::vector<double> par (s->betak2);
+  par.resize (2 * (size_t) num_modes);
+  std::memcpy (par.data () + num_modes, s->nsolve.data (), sizeof (int) * num_modes);
+  TRY (hipMemcpyAsync (s->d_betak2, par.data (), sizeof (double) * par.size (),
+                       hipMemcpyHostToDevice, st));
 
-  double *d_ws = nullptr, *d_S = nullptr;
-  int* d_status = nullptr;
   const size_t ws_per = (size_t) npnp * npnp + (size_t) nint * nint;
-  TRY (hipMalloc (&d_ws, sizeof (double) * nmc * ws_per));
-  TRY (hipMalloc (&d_S, sizeof (double) * nmc * next * next));
-  TRY (hipMalloc (&d_status, sizeof (int) * (num_modes + 1)));
+  size_t nt = 0;
+  const size_t o_st = take (nt, num_modes + 1), o_ws = take (nt, nmc * ws_per),
+               o_S = take (nt, nmc * next * next),
+               o_f = take (nt, s->use_tree ? tree_scratch (s->tree, num_modes) : 0);
+  if ((rc = block_alloc ((void**) &d_ws, sizeof (double) * nt, &ws_bytes, &ws_dev))) return fail (rc);
+  double* d_S = d_ws + o_S;
+  int* d_status = (int*) (d_ws + o_st);
   TRY (hipMemsetAsync (d_status, 0, sizeof (int) * (num_modes + 1), st));
 
-  if ((rc = elem_sc (m, num_modes, lambda2, s->d_betak2, d_ws, d_S, s->d_Bm, s->d_Hinv,
+  if ((rc = elem_sc (m, num_modes, lambda2, s->d_betak2, d_ws + o_ws, d_S, s->d_Bm, s->d_Hinv,
                      d_status + num_modes, st)))
     return fail (rc);
-  if (tiled_ok (m)) {
-    s->tile_mf = tiled_mfma (m) ? 1 : 0;
-    if (const char* e = std::getenv ("SX_TILE_MFMA")) s->tile_mf = s->tile_mf && std::atoi (e);
-    const TileShape R = rec_shape (m->np, s->tile_mf), Cs = con_shape (m->np, s->tile_mf);
-    const size_t nr = (size_t) R.KR * R.NA, nc = (size_t) Cs.KR * Cs.NA;
-    TRY (hipMalloc (&s->d_Mrec, sizeof (double) * nmc * nr));
-    TRY (hipMalloc (&s->d_Mcon, sizeof (double) * nmc * nc));
-    hipLaunchKernelGGL (k_tiled_ops, dim3 ((unsigned) ((nr + nc + 255) / 256),
+  if (tiled) {
+    hipLaunchKernelGGL (k_tiled_ops, dim3 ((unsigned) ((nrec + ncon + 255) / 256),
                                           (unsigned) std::min<size_t> (nmc, 65535)),
                         dim3 (256), 0, st, m->np, (int) nmc, s->tile_mf, s->d_Bm, s->d_Hinv,
                         s->d_Mrec, s->d_Mcon);
     TRY (hipGetLastError ());
   }
-  rc = s->use_tree ? tree_factor (s, d_S, st, d_status) : band_build (s, d_S, st, d_status);
-  if (rc || (rc = tree_sing_setup (s, d_S, st, d_status)) || (rc = tree_workspace (s, 2)))
-    return fail (rc);
+  rc = s->use_tree ? tree_factor (s, d_S, d_ws + o_f, st, d_status)
+                   : band_build (s, d_S, st, d_status);
+  if (rc || (rc = tree_sing_setup (s, d_S, st, d_status))) return fail (rc);
   std::vector<int> status (num_modes + 1);
   TRY (hipMemcpyAsync (status.data (), d_status, sizeof (int) * (num_modes + 1),
                        hipMemcpyDeviceToHost, st));
   TRY (hipStreamSynchronize (st));
-  (void) hipFree (d_ws); (void) hipFree (d_S); (void) hipFree (d_status);
+  block_free (d_ws, ws_bytes, ws_dev);
+  d_ws = nullptr;
   if (status[num_modes]) {
     set_error ("sx_msys_create: matrix hii is not positive definite");
     return fail (SX_ERR_FACTOR);
@@ -2197,12 +2261,13 @@ int msys_reserve_rhs (sx_msys* s, int nr)
   SX_HIP (hipMalloc (&g, sizeof (double) * (nr / 2) * 2 * s->nmodes * s->m->nglobal));
   SX_HIP (hipMemset (r, 0, sizeof (double) * s->nmodes * nr * std::max (s->nmax, 1)));
   SX_HIP (hipMemset (g, 0, sizeof (double) * (nr / 2) * 2 * s->nmodes * s->m->nglobal));
-  (void) hipFree (s->d_rhs);
-  (void) hipFree (s->d_G);
+  msys_free (s, s->d_rhs);
+  msys_free (s, s->d_G);
   s->d_rhs = r;
   s->d_G = g;
+  const int rc = tree_workspace (s, nr);
   s->rhs_cap = nr;
-  return tree_workspace (s, nr);
+  return rc;
 }
 
 int condense32_tiled (const sx_msys* s, int nz, int stride, const double* X, double* Fp,

@@ -41,7 +41,11 @@ constexpr int TB = 64;                 // pivot block and tile of the factorisat
 // Front matrices of a level: each entry the sum of its parts' entries
 // (elements: their condensed matrix; fronts: their trailing block).  In a
 // singular mode (the last unknown dropped) the pinned unknown is replaced
-// by the identity.
+// by the identity.  Front matrices are kept by their upper 64x64 tiles only
+// (diagonal tiles whole): they stay symmetric up to the sign the elimination
+// gives (k_tree_update).
+__device__ __forceinline__ bool upper_tile (int i, int j) { return (i >> 6) <= (j >> 6); }
+
 __global__ __launch_bounds__(256) void k_tree_assemble (
     const TreeClass* __restrict__ cls, int cls0, const TreeChild* __restrict__ child,
     const int* __restrict__ map, const double* __restrict__ Sel, int next, int nec,
@@ -54,6 +58,7 @@ __global__ __launch_bounds__(256) void k_tree_assemble (
   for (size_t e = (size_t) blockIdx.x * 256 + threadIdx.x; e < (size_t) n * n;
        e += (size_t) gridDim.x * 256) {
     const int i = (int) (e / n), j = (int) (e % n);
+    if (!upper_tile (i, j)) continue;
     double s = 0.0;
     if (pinned && (i == C.pin || j == C.pin)) {
       s = i == j ? 1.0 : 0.0;
@@ -64,8 +69,9 @@ __global__ __launch_bounds__(256) void k_tree_assemble (
         if (a < 0 || b < 0) continue;
         if (ch.front) {
           const TreeClass D = cls[ch.cls];
-          const int nd = D.k + D.b;
-          s += Fc[(size_t) mode * fcs + D.foff + (size_t) (D.k + a) * nd + D.k + b];
+          const int nd = D.k + D.b, r = D.k + a, t = D.k + b;
+          const bool up = upper_tile (r, t);
+          s += Fc[(size_t) mode * fcs + D.foff + (size_t) (up ? r : t) * nd + (up ? t : r)];
         } else {
           s += Sel[(((size_t) mode * nec + ch.cls) * next + a) * next + b];
         }
@@ -99,18 +105,23 @@ __global__ __launch_bounds__(256) void k_tree_panel (
   if (tid == 0) bad = 0;
   // the pivot block (identity past pb) and the rows of P in this tile's
   // columns, every load unconditional
+  // (columns already eliminated: F_Pj = -F_jP^T, read from the upper tiles)
+  const bool done = c0 < p0;
   double x[16], y[16];
 #pragma unroll
   for (int q = 0; q < 16; q++) {
     const int r = 4 * q + wave, rr = p0 + min (r, pb - 1);
     x[q] = Fm[(size_t) rr * n + p0 + min (lane, pb - 1)];
-    y[q] = Fm[(size_t) rr * n + min (c0 + lane, n - 1)];
+    const size_t at = done ? (size_t) (c0 + r) * n + p0 + min (lane, pb - 1)
+                           : (size_t) rr * n + min (c0 + lane, n - 1);
+    y[q] = Fm[at];
   }
 #pragma unroll
   for (int q = 0; q < 16; q++) {
     const int r = 4 * q + wave;
     piv[r * LD + lane] = r < pb && lane < pb ? x[q] : r == lane ? 1.0 : 0.0;
-    Rs[r * LD + lane] = r < pb && c0 + lane < n ? y[q] : 0.0;
+    if (done) Rs[lane * LD + r] = lane < pb ? -y[q] : 0.0;
+    else Rs[r * LD + lane] = r < pb && c0 + lane < n ? y[q] : 0.0;
   }
   __syncthreads ();
   spd_invert (piv, LD, (pb + 15) / 16, Wb, D, &bad);
@@ -142,7 +153,7 @@ __global__ __launch_bounds__(256) void k_tree_panel (
 //   i in P:         F_ij  = W_ij
 //   j in P:         F_ij  = -s_i W_ji
 // with s_i = -1 for unknowns already eliminated (i < p0), +1 otherwise: the
-// matrix stays symmetric up to that sign, so only rows of P are ever read.
+// matrix stays symmetric up to that sign, so only upper tiles are formed.
 // R and W are padded to whole tiles, so every load is unconditional and
 // issued before the products (46 -> 12 us a step at 96 fronts of 370).
 __global__ __launch_bounds__(256) void k_tree_update (
@@ -152,7 +163,10 @@ __global__ __launch_bounds__(256) void k_tree_update (
   const TreeClass C = cls[cls0 + blockIdx.y];
   const int mode = blockIdx.z, n = C.k + C.b, p0 = TB * step;
   const int pb = min (TB, C.k - p0);
-  const int i0 = TB * (blockIdx.x / nt), j0 = TB * (blockIdx.x % nt);
+  // upper tile blockIdx.x of nt (nt + 1) / 2, by rows
+  int ti = 0, tj = blockIdx.x;
+  while (tj >= nt - ti) { tj -= nt - ti; ti++; }
+  const int i0 = TB * ti, j0 = TB * (ti + tj);
   if (pb <= 0 || i0 >= n || j0 >= n) return;
   constexpr int LD = TB + 2;
   __shared__ double Rs[TB * LD], Ws[TB * LD];
@@ -234,7 +248,8 @@ __global__ __launch_bounds__(256) void k_tree_operators (
       if (row < C.b && kk < C.k) v = Fm[(size_t) kk * n + C.k + row];
       O[C.mf + q] = v;
     } else {
-      if (row < C.k && kk < n) v = Fm[(size_t) row * n + kk];
+      if (row < C.k && kk < n)
+        v = upper_tile (row, kk) ? Fm[(size_t) row * n + kk] : Fm[(size_t) kk * n + row];
       O[C.mb + q] = kk < C.k ? v : -v;
     }
   }
@@ -572,23 +587,41 @@ int tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always)
   return SX_OK;
 }
 
+// Scratch of a factorisation of nm modes: the front matrices of two levels
+// and a step's rows
+struct Scratch { size_t f0, f1, rw; };
+static Scratch scratch (const TreePlan& P)
+{
+  Scratch z {0, 0, 0};
+  for (size_t j = 0; j < P.lev.size (); j++) {
+    const TreeLevel& L = P.lev[j];
+    size_t& f = j & 1 ? z.f1 : z.f0;
+    f = std::max (f, L.fsize);
+    z.rw = std::max (z.rw, (size_t) L.ncls * 2 * TB * ((L.nmax + TB - 1) / TB * TB));
+  }
+  return z;
+}
+
+size_t tree_scratch (const TreeDev* t, int nm)
+{
+  const Scratch z = scratch (t->P);
+  return (z.f0 + z.f1 + z.rw) * nm;
+}
+
+size_t tree_ops (const TreeDev* t) { return t->P.ops; }
+size_t tree_slots (const TreeDev* t) { return t->P.slots; }
+
 // Factorisation of nm modes: the levels from the elements to the root (Sel:
-// the condensed element matrices [nm][nclass][next][next]) into *ops.
-// status[mode] > 0: a pivot was not positive.  Waits for st.
+// the condensed element matrices [nm][nclass][next][next]) into ops
+// [nm][tree_ops]; buf: tree_scratch doubles.  status[mode] > 0: a pivot was
+// not positive.
 static int factor (const TreeDev* t, const sx_mesh* m, int nm, const int* d_nsolve,
-                   const double* Sel, double** ops, hipStream_t st, int* d_status)
+                   const double* Sel, double* ops, double* buf, hipStream_t st, int* d_status)
 {
   const TreePlan& P = t->P;
   const int nl = (int) P.lev.size ();
-  size_t fmax[2] = {0, 0}, rw = 0;
-  for (int j = 0; j < nl; j++) {
-    const TreeLevel& L = P.lev[j];
-    fmax[j & 1] = std::max (fmax[j & 1], L.fsize);
-    rw = std::max (rw, (size_t) L.ncls * 2 * TB * ((L.nmax + TB - 1) / TB * TB));
-  }
-  double* buf = nullptr;
-  SX_HIP (hipMalloc (ops, sizeof (double) * std::max<size_t> (P.ops * nm, 2)));
-  SX_HIP (hipMalloc (&buf, sizeof (double) * (fmax[0] + fmax[1] + rw) * nm));
+  const Scratch z = scratch (P);
+  const size_t fmax[2] = {z.f0, z.f1};
   double* F[2] = {buf, buf + fmax[0] * nm};
   double* RW = F[1] + fmax[1] * nm;
   for (int j = nl - 1; j >= 0; j--) {
@@ -604,16 +637,14 @@ static int factor (const TreeDev* t, const sx_mesh* m, int nm, const int* d_nsol
     for (int step = 0; TB * step < L.kmax; step++) {
       hipLaunchKernelGGL (k_tree_panel, dim3 (nt, L.ncls, nm), dim3 (256), 0, st, t->cls, L.cls0,
                           Fj, L.fsize, RW, ldw, step, d_status);
-      hipLaunchKernelGGL (k_tree_update, dim3 (nt * nt, L.ncls, nm), dim3 (256), 0, st, t->cls,
+      hipLaunchKernelGGL (k_tree_update, dim3 (nt * (nt + 1) / 2, L.ncls, nm), dim3 (256), 0, st, t->cls,
                           L.cls0, Fj, L.fsize, RW, ldw, step, nt);
     }
     hipLaunchKernelGGL (k_tree_operators, gb, dim3 (256), 0, st, t->cls, L.cls0, Fj, L.fsize,
-                        *ops, P.ops);
+                        ops, P.ops);
   }
-  const hipError_t e = hipGetLastError ();
-  if (e == hipSuccess) (void) hipStreamSynchronize (st);
-  (void) hipFree (buf);
-  return e == hipSuccess ? (int) SX_OK : hip_fail (e, "tree_factor");
+  SX_HIP (hipGetLastError ());
+  return SX_OK;
 }
 
 // The launches of a solve: up to the root's children, down from the root
@@ -706,20 +737,21 @@ void tree_sing_free (TreeSing* g)
   delete g;
 }
 
-// Workspace of a solve with nr right-hand sides per mode
+// Workspace of a solve with nr right-hand sides per mode, grown from the one
+// the system was created with (2)
 int tree_workspace (sx_msys* s, int nr)
 {
-  auto grow = [] (double** p, size_t n) {
+  auto grow = [&] (double** p, size_t n) {
     double* q = nullptr;
     SX_HIP (hipMalloc (&q, sizeof (double) * std::max<size_t> (n, 1)));
     SX_HIP (hipMemset (q, 0, sizeof (double) * n));
-    (void) hipFree (*p);
+    msys_free (s, *p);
     *p = q;
     return (int) SX_OK;
   };
   const size_t n = (size_t) s->nmodes * nr;
   int rc;
-  if (s->use_tree) {
+  if (s->use_tree && nr > s->rhs_cap) {
     const TreePlan& P = s->tree->P;
     if ((rc = grow (&s->d_tb, n * P.nsolve)) || (rc = grow (&s->d_tv, n * P.nsolve)) ||
         (rc = grow (&s->d_tc, n * P.slots)))
@@ -738,9 +770,9 @@ int tree_workspace (sx_msys* s, int nr)
 
 const int* tree_perm (const sx_msys* s) { return s->use_tree ? s->tree->perm : nullptr; }
 
-int tree_factor (sx_msys* s, const double* Sel, hipStream_t st, int* d_status)
+int tree_factor (sx_msys* s, const double* Sel, double* buf, hipStream_t st, int* d_status)
 {
-  return factor (s->tree, s->m, s->nmodes, s->d_nsolve, Sel, &s->d_tops, st, d_status);
+  return factor (s->tree, s->m, s->nmodes, s->d_nsolve, Sel, s->d_tops, buf, st, d_status);
 }
 
 int tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_status)
@@ -755,13 +787,17 @@ int tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_statu
     g->mode = md;
     g->t = t;
     const double* S = Sel + (size_t) md * m->nclass * m->next * m->next;
-    if (int rc = factor (t, m, 1, s->d_nsolve + md, S, &g->ops, st, d_status + md)) return rc;
+    // (the scratch is the later workspace's allocation g->val: entries past
+    // the matrix's are free once the factor is done)
+    const size_t nb = std::max<size_t> (tree_scratch (t, 1), m->npairs);
+    SX_HIP (hipMalloc (&g->ops, sizeof (double) * std::max<size_t> (t->P.ops, 2)));
+    SX_HIP (hipMalloc (&g->val, sizeof (double) * nb));
+    if (int rc = factor (t, m, 1, s->d_nsolve + md, S, g->ops, g->val, st, d_status + md)) return rc;
     if (int rc = sing_rows (m)) return rc;
-    SX_HIP (hipMalloc (&g->val, sizeof (double) * std::max (m->npairs, 1)));
     hipLaunchKernelGGL (k_tree_entries, dim3 ((m->npairs + 255) / 256), dim3 (256), 0, st,
                         m->npairs, m->d_pptr, m->d_psrc, S, g->val);
     SX_HIP (hipGetLastError ());
-    return SX_OK;                      // at most mode 0 has a zero constant
+    return tree_workspace (s, 2);      // at most mode 0 has a zero constant
   }
   return SX_OK;
 }
