@@ -9,9 +9,10 @@
 // phase runs once for all the problems that use it (k_batch: blockIdx.z
 // picks the problem), so the graph holds a few dozen launches instead of
 // ~10 per problem.  Problems that share a system (and so its workspace)
-// are planned one after the other.  The right-hand sides per band-sweep
-// workgroup are chosen per class of band system (D, unit-diagonal,
-// twisted) by sx_batch_tune, which times the alternatives.
+// are planned one after the other.  Systems solve by dissection (a level of
+// every problem's fronts is one launch); those that only have a band factor
+// run band sweeps, whose right-hand sides per workgroup sx_batch_tune chooses
+// per class of band system (D, unit-diagonal, twisted) by timing.
 //
 // Graph-of-launches form (SX_BATCH_FUSED=0, or a system the plans do not
 // cover: offset-major band sweeps, untiled element kernels): the
@@ -112,10 +113,11 @@ struct FnCopy {
 };
 
 // the band-system class of a system: (off-diagonal blocks, unit-diagonal
-// panels, twisted), which decides the sweep kernel instance
+// panels, twisted), which decides the sweep kernel instance; D = -1: dissection
 int class_of (sx_batch* b, const sx_msys* s)
 {
-  const std::array<int, 3> k = {s->sw_D, s->sw_unit, s->tw};
+  const std::array<int, 3> k = s->tree ? std::array<int, 3> {-1, 0, 0}
+                                       : std::array<int, 3> {s->sw_D, s->sw_unit, s->tw};
   for (size_t c = 0; c < b->keys.size (); c++)
     if (b->keys[c] == k) return (int) c;
   b->keys.push_back (k);
@@ -263,9 +265,8 @@ extern "C" int sx_batch_create (int n, const sx_msys_t* systems, const int* nz,
       return SX_ERR_ARG;
     }
   *out = nullptr;
-  // the recorded solves are band sweeps: so are the systems' own from here
   for (int i = 0; i < n; i++)
-    if (int rc = msys_use_band (systems[i])) return rc;
+    if (int rc = msys_hold (systems[i])) return rc;
   sx_batch* b = new sx_batch;
   b->n = n;
   auto fail = [&] (int r) { sx_batch_destroy (b); return r; };
@@ -368,6 +369,7 @@ extern "C" int sx_batch_tune (sx_batch_t b, int reps, void* stream)
   int rc = time_ms (best);
   // coordinate search: each class's right-hand sides per sweep workgroup
   for (size_t c = 0; !rc && c < b->keys.size (); c++) {
+    if (b->keys[c][0] < 0) continue;                 // dissection: nothing to choose
     const int keep = b->per[c];
     for (int cand : {1, 2}) {
       b->per[c] = cand;
@@ -393,6 +395,10 @@ extern "C" int sx_batch_info (sx_batch_t b, char* buf, int len)
   for (size_t c = 0; c < b->keys.size (); c++) {
     int cnt = 0;
     for (int x : b->cls) cnt += x == (int) c;
+    if (b->keys[c][0] < 0) {
+      t += "; dissection problems=" + std::to_string (cnt);
+      continue;
+    }
     t += "; D=" + std::to_string (b->keys[c][0]) + " unit=" + std::to_string (b->keys[c][1]) +
          " twisted=" + std::to_string (b->keys[c][2]) + " problems=" + std::to_string (cnt) +
          " nr=" + std::to_string (b->per[c]);

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstdlib>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -84,10 +85,12 @@ int    tree_solve (const sx_msys* s, int nr, hipStream_t st);
 int    tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_status);
 int    sing_keep (const sx_msys* s, int nr, hipStream_t st);
 int    sing_refine (const sx_msys* s, int nr, hipStream_t st);
-// A system's band factor (built on first use where the system solves by
-// dissection) and its use from now on: the batches plan band sweeps, and
-// their systems' own solves stay equal to the batch's (sx_solver.hip).
-int    msys_use_band (sx_msys* s);
+// A system taken into a batch (sx_solver.hip): the batch records the
+// dissection; the system's own solves run band sweeps from then on (their
+// factor is built here), as systems of a batch always did, unless
+// SX_BAND_SPLIT=0 asks for no split sweeps, when they run what the batch
+// records.
+int    msys_hold (sx_msys* s);
 // Frees a device array of the system unless it lies in its block.
 void   msys_free (sx_msys* s, void* p);
 // Banded FP64 Cholesky of every mode's band, the offset-major sweep copies
@@ -268,6 +271,7 @@ struct sx_msys {
   int block_dev = 0;
   sx::TreeDev* tree = nullptr; // dissection solve: the mesh's plan, null: band only
   int use_tree = 0;            //   solves run it
+  int held = 0;                //   a batch holds the system (msys_hold)
   sx::TreeSing* sing = nullptr;  // the singular mode's refinement, or null
   double* d_tops = nullptr;    //   operators [nmodes][ops]
   double* d_tb = nullptr;      //   assembled right-hand sides by position [nmodes][nr][nsolve]
@@ -285,11 +289,16 @@ struct sx_msys {
 // position and writes the solution to d_rhs by node.
 namespace sx {
 const int* tree_perm (const sx_msys* s);
-struct RhsTo { double* p; int ld; const int* perm; };
-inline RhsTo rhs_in (const sx_msys* s)
+inline bool by_tree (const sx_msys* s)
 {
-  return s->use_tree ? RhsTo {s->d_tb, s->m->nsolve, tree_perm (s)}
-                     : RhsTo {s->d_rhs, s->nmax, nullptr};
+  if (s->use_tree || !s->held || !s->tree) return s->use_tree;
+  const char* e = std::getenv ("SX_BAND_SPLIT");
+  return s->no_split || (e && std::atoi (e) == 0);
+}
+struct RhsTo { double* p; int ld; const int* perm; };
+inline RhsTo rhs_in (const sx_msys* s, bool tree)
+{
+  return tree ? RhsTo {s->d_tb, s->m->nsolve, tree_perm (s)} : RhsTo {s->d_rhs, s->nmax, nullptr};
 }
 }
 
@@ -416,6 +425,7 @@ void batch_rec (BatchPlan& P, dim3 grid, int block, size_t lds, A... a)
 int plan_field_solve_direct (BatchPlan& P, const sx_msys* s, int nz, int stride, double* d_f,
                              double* d_u, const double* d_lines);
 int plan_band_solve (BatchPlan& P, const sx_msys* s, int nr);
+int plan_tree_solve (BatchPlan& P, const sx_msys* s);
 int plan_mixed_passes (BatchPlan& P, sx_msys* s, int nz, int stride, double* d_f,
                        double* d_u, const double* d_lines, int passes);
 int plan_copy (BatchPlan& P, double* dst, const double* src, size_t n);

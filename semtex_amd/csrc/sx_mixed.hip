@@ -346,7 +346,7 @@ int inner_solve (sx_msys* s, int nz, int stride, const double* X, double* Fp,
     hipLaunchKernelGGL (k_condense32, dim3 (m->nel, npl), dim3 (64), 0, st, m->np, m->nclass,
                         m->d_emap, m->d_cls, s->d_Bm32, X, Fp, stride, nz, s->base_mode);
   }
-  const RhsTo to = rhs_in (s);
+  const RhsTo to = rhs_in (s, by_tree (s));
   hipLaunchKernelGGL (k_assemble_m, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw, Fp,
                       stride, lines, lstride, s->d_nsolve, to.p, to.ld, nz, s->base_mode,
@@ -403,14 +403,15 @@ int plan_inner (BatchPlan& P, sx_msys* s, int nz, int stride, const double* X, d
                                  (const float*) s->d_Bm32, X, Fp, stride, nz, s->base_mode);
     P.phase++;
   }
+  const RhsTo to = rhs_in (s, s->tree != nullptr);
   batch_rec<256, FnAssembleM> (P, dim3 ((m->nglobal + 255) / 256, npl), 256, 0, m->nglobal,
                                (const int*) m->d_gptr, (const int*) m->d_gsrc,
                                (const int*) m->d_nptr, (const int*) m->d_nidx,
                                (const double*) m->d_nw, (const double*) Fp, stride, lines,
-                               lstride, (const int*) s->d_nsolve, s->d_rhs, s->nmax, nz,
-                               s->base_mode, (const int*) nullptr);
+                               lstride, (const int*) s->d_nsolve, to.p, to.ld, nz,
+                               s->base_mode, to.perm);
   P.phase++;
-  if (int rc = plan_band_solve (P, s, 2)) return rc;
+  if (int rc = s->tree ? plan_tree_solve (P, s) : plan_band_solve (P, s, 2)) return rc;
   if (tiled) return plan_recover32_tiled (P, s, nz, stride, Fp, V);
   batch_rec<64, FnRecover32> (P, dim3 (m->nel, npl), 64, 0, m->np, m->nclass,
                               (const int*) m->d_emap, (const int*) m->d_cls,

@@ -1729,12 +1729,13 @@ static int band_build (sx_msys* s, const double* d_S, hipStream_t st, int* d_sta
 
 namespace sx {
 
-int msys_use_band (sx_msys* s)
+int msys_hold (sx_msys* s)
 {
-  // (the recorded sweeps refine no singular mode either)
+  if (s->held) return SX_OK;
+  // (neither refines a singular mode in a batch)
   tree_sing_free (s->sing);
   s->sing = nullptr;
-  if (!s->use_tree) return SX_OK;
+  if (!s->use_tree) { s->held = 1; return SX_OK; }
   const sx_mesh* m = s->m;
   const int next = m->next, nint = m->nint, npnp = m->npnp;
   const size_t nmc = (size_t) s->nmodes * m->nclass;
@@ -1758,8 +1759,7 @@ int msys_use_band (sx_msys* s)
   (void) hipFree (d_status);
   if (rc) return rc;
   s->use_tree = 0;
-  // (more than 2 reserved right-hand sides: their bottom-piece workspace
-  // came with the factor, band_factor sizes it by rhs_cap)
+  s->held = 1;
   return SX_OK;
 }
 
@@ -2161,7 +2161,7 @@ int field_solve_direct (const sx_msys* s, int nz, int stride, double* d_f, doubl
   const int npl = n_solved_planes (nz, s->base_mode);
   const int lstride = m->nbound * m->np;
   const double* lines = (d_lines && m->nbound) ? d_lines : nullptr;
-  const RhsTo to = rhs_in (s);
+  const RhsTo to = rhs_in (s, by_tree (s));
   // the essential values and the essential elements' weak form in one
   // launch where the tiled condensation follows
   const bool ew = tiled_ok (m) && m->ness;
@@ -2188,7 +2188,7 @@ int field_solve_direct (const sx_msys* s, int nz, int stride, double* d_f, doubl
   }
   // a twisted system's bottom piece addressed by the assembly and the
   // recovery themselves (no gather and scatter launches around the sweeps)
-  const bool fold = !s->use_tree && !s->sing && s->tw && s->sw_panel && tiled_ok (m) && s->tile_mf;
+  const bool fold = !by_tree (s) && !s->sing && s->tw && s->sw_panel && tiled_ok (m) && s->tile_mf;
   {
     PhaseScope ps (2, st, timed);
     if (fold)
@@ -2393,14 +2393,15 @@ int plan_field_solve_direct (BatchPlan& P, const sx_msys* s, int nz, int stride,
   }
   P.phase++;
   const int rnr = 2, roff = 0;
+  const RhsTo to = rhs_in (s, s->tree != nullptr);
   batch_rec<256, FnAssemble> (P, dim3 (gb, npl), 256, 0, m->nglobal, (const int*) m->d_gptr,
                               (const int*) m->d_gsrc, (const int*) m->d_nptr,
                               (const int*) m->d_nidx, (const double*) m->d_nw,
                               (const double*) d_f, stride, lines, lstride,
-                              (const int*) s->d_nsolve, s->d_rhs, s->nmax, nz, s->base_mode,
-                              rnr, roff, (const int*) nullptr);
+                              (const int*) s->d_nsolve, to.p, to.ld, nz, s->base_mode,
+                              rnr, roff, to.perm);
   P.phase++;
-  if (int rc = plan_band_solve (P, s, 2)) return rc;
+  if (int rc = s->tree ? plan_tree_solve (P, s) : plan_band_solve (P, s, 2)) return rc;
   auto rec_r = [&] (auto fn) {
     batch_rec<CT_THREADS, decltype (fn)> (
         P, tg, CT_THREADS, reg_lds (m, true), m->np, m->nclass, (const int*) m->d_ttab,
@@ -2474,7 +2475,7 @@ int field_solve_group (sx_msys* s, int nf, int nz, int stride, double* const* d_
   const int npl = n_solved_planes (nz, s->base_mode), nr = 2 * nf;
   const int lstride = m->nbound * m->np;
   const size_t gstride = (size_t) 2 * s->nmodes * m->nglobal;
-  const RhsTo to = rhs_in (s);
+  const RhsTo to = rhs_in (s, by_tree (s));
   // the register-operand element kernels take up to three fields per launch
   const bool grouped = nf <= 3 && tiled_ok (m) && s->tile_mf;
   const int npmr = reg_npm (m->np);
@@ -2639,7 +2640,7 @@ extern "C" int sx_field_solve_weak (sx_msys_t s, int nz, int stride, double* d_w
   hipLaunchKernelGGL (k_essential, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_ess, nullptr, 0, s->d_G, nz, s->base_mode);
   if ((rc = condense (s, nz, stride, d_w, s->d_G, st, 1))) return rc;
-  const RhsTo to = rhs_in (s);
+  const RhsTo to = rhs_in (s, by_tree (s));
   hipLaunchKernelGGL (k_assemble, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw, d_w,
                       stride, nullptr, 0, s->d_nsolve, to.p, to.ld, nz, s->base_mode, 2, 0, to.perm);

@@ -282,7 +282,7 @@ enum { T_UP = 0, T_DOWN = 1, T_ROOT = 2 };
 // solution at the boundary nodes.  Every load of a round is issued before
 // any of it is used.
 template <int DIR, int W>
-__global__ __launch_bounds__(256) void k_tree_level (TreeArgs T)
+__device__ __forceinline__ void tree_level_body (const TreeArgs& T)
 {
   extern __shared__ double sm[];
   // a mode's work stays on one XCD where the modes fill all eight: its
@@ -460,6 +460,16 @@ __global__ __launch_bounds__(256) void k_tree_level (TreeArgs T)
     }
   }
 }
+
+template <int DIR, int W>
+__global__ __launch_bounds__(256) void k_tree_level (TreeArgs T)
+{
+  tree_level_body<DIR, W> (T);
+}
+template <int DIR, int W> struct FnTreeLevel {
+  __device__ __forceinline__ void operator() (const TreeArgs& T) const
+  { tree_level_body<DIR, W> (T); }
+};
 
 // Entries of a mode's assembled matrix, each pair (row <= column) summed
 // over its elements in the band assembly's order
@@ -647,43 +657,88 @@ static int factor (const TreeDev* t, const sx_mesh* m, int nm, const int* d_nsol
   return SX_OK;
 }
 
-// The launches of a solve: up to the root's children, down from the root
-static int sweep (const TreeDev* t, TreeArgs T, int nm, int nr, hipStream_t st)
+// The arguments of a level's launch that the plan gives
+struct LevelLaunch { int dir, W, blocks; size_t lds; };
+static LevelLaunch level_launch (const TreeDev* t, TreeArgs& T, int j, int down, int nm, int nr)
 {
   const TreePlan& P = t->P;
-  const int q = nr / 2 - 1, nl = (int) P.lev.size ();
+  const TreeLevel& L = P.lev[j];
+  const int q = nr / 2 - 1;
   T.gk = t->gk; T.gb = t->gb; T.tgt = t->tgt;
   T.os = P.ops;
   T.nsp = P.nsolve; T.slots = P.slots; T.nr = nr;
   T.nmodes = nm;
   T.xcd = nm >= 32 || (nm >= 8 && nm % 8 == 0);
-  auto launch = [&] (auto kern, int first, int count, size_t lds) {
-    if (!count) return (int) SX_OK;
-    if (int rc = lds_limit ((const void*) kern, lds)) return rc;
-    T.item = t->item + first;
-    T.nitem = count;
-    const int blocks = count * (T.xcd ? (nm + 7) / 8 * 8 : nm);
-    hipLaunchKernelGGL (kern, dim3 (blocks), dim3 (256), lds, st, T);
-    SX_HIP (hipGetLastError ());
-    return (int) SX_OK;
+  T.item = t->item + (down ? L.it_b[q] : L.it_f[q]);
+  T.nitem = down ? L.nit_b[q] : L.nit_f[q];
+  return {down ? (j ? T_DOWN : T_ROOT) : T_UP, P.W,
+          T.nitem * (T.xcd ? (nm + 7) / 8 * 8 : nm), down ? L.lds_b[q] : L.lds_f[q]};
+}
+
+// f (DIR, W) with the launch's kernel instance
+template <typename F> static int tree_instance (const LevelLaunch& l, F f)
+{
+  auto dir = [&] (auto w) {
+    return l.dir == T_UP     ? f (std::integral_constant<int, T_UP> {}, w)
+           : l.dir == T_DOWN ? f (std::integral_constant<int, T_DOWN> {}, w)
+                             : f (std::integral_constant<int, T_ROOT> {}, w);
   };
-  auto level = [&] (int j, int dir) {
-    const TreeLevel& L = P.lev[j];
-    const int first = dir ? L.it_b[q] : L.it_f[q], count = dir ? L.nit_b[q] : L.nit_f[q];
-    const size_t lds = dir ? L.lds_b[q] : L.lds_f[q];
-    auto with = [&] (auto w) {
-      constexpr int W = decltype (w)::value;
-      return dir == 0 ? launch (k_tree_level<T_UP, W>, first, count, lds)
-             : j      ? launch (k_tree_level<T_DOWN, W>, first, count, lds)
-                      : launch (k_tree_level<T_ROOT, W>, first, count, lds);
-    };
-    return P.W == 4 ? with (std::integral_constant<int, 4> {})
-                    : with (std::integral_constant<int, 8> {});
+  return l.W == 4 ? dir (std::integral_constant<int, 4> {}) : dir (std::integral_constant<int, 8> {});
+}
+
+// The launches of a solve: up to the root's children, down from the root
+static int sweep (const TreeDev* t, TreeArgs T, int nm, int nr, hipStream_t st)
+{
+  const int nl = (int) t->P.lev.size ();
+  auto level = [&] (int j, int down) {
+    const LevelLaunch l = level_launch (t, T, j, down, nm, nr);
+    if (!l.blocks) return (int) SX_OK;
+    return tree_instance (l, [&] (auto d, auto w) {
+      auto kern = k_tree_level<decltype (d)::value, decltype (w)::value>;
+      if (int rc = lds_limit ((const void*) kern, l.lds)) return rc;
+      hipLaunchKernelGGL (kern, dim3 (l.blocks), dim3 (256), l.lds, st, T);
+      SX_HIP (hipGetLastError ());
+      return (int) SX_OK;
+    });
   };
   for (int j = nl - 1; j > 0; j--)
     if (int rc = level (j, 0)) return rc;
   for (int j = 0; j < nl; j++)
     if (int rc = level (j, 1)) return rc;
+  return SX_OK;
+}
+
+static TreeArgs tree_args (const sx_msys* s)
+{
+  TreeArgs T {};
+  T.ops = s->d_tops;
+  T.in = s->d_tb; T.rhs = s->d_rhs; T.v = s->d_tv; T.cb = s->d_tc;
+  T.nmax = s->nmax;
+  T.nsolve = s->d_nsolve;
+  return T;
+}
+
+// The same launches recorded into a batch's plan, the roots of all its
+// systems in one phase (trees of up to TREE_PLAN_LEVELS levels end level)
+constexpr int TREE_PLAN_LEVELS = 5;
+int plan_tree_solve (BatchPlan& P, const sx_msys* s)
+{
+  const TreeDev* t = s->tree;
+  const int nl = (int) t->P.lev.size (), root = P.phase + std::max (nl, TREE_PLAN_LEVELS) - 1;
+  auto level = [&] (int j, int down) {
+    TreeArgs T = tree_args (s);
+    const LevelLaunch l = level_launch (t, T, j, down, s->nmodes, 2);
+    P.phase = down ? root + j : root - j;
+    if (!l.blocks) return (int) SX_OK;
+    return tree_instance (l, [&] (auto d, auto w) {
+      batch_rec<256, FnTreeLevel<decltype (d)::value, decltype (w)::value>> (
+          P, dim3 (l.blocks), 256, l.lds, T);
+      return (int) SX_OK;
+    });
+  };
+  for (int j = nl - 1; j > 0; j--) level (j, 0);
+  for (int j = 0; j < nl; j++) level (j, 1);
+  P.phase = root + std::max (nl, TREE_PLAN_LEVELS);
   return SX_OK;
 }
 
@@ -751,7 +806,7 @@ int tree_workspace (sx_msys* s, int nr)
   };
   const size_t n = (size_t) s->nmodes * nr;
   int rc;
-  if (s->use_tree && nr > s->rhs_cap) {
+  if (s->tree && nr > s->rhs_cap) {
     const TreePlan& P = s->tree->P;
     if ((rc = grow (&s->d_tb, n * P.nsolve)) || (rc = grow (&s->d_tv, n * P.nsolve)) ||
         (rc = grow (&s->d_tc, n * P.slots)))
@@ -768,7 +823,7 @@ int tree_workspace (sx_msys* s, int nr)
   return SX_OK;
 }
 
-const int* tree_perm (const sx_msys* s) { return s->use_tree ? s->tree->perm : nullptr; }
+const int* tree_perm (const sx_msys* s) { return s->tree->perm; }
 
 int tree_factor (sx_msys* s, const double* Sel, double* buf, hipStream_t st, int* d_status)
 {
@@ -844,13 +899,8 @@ int tree_solve (const sx_msys* s, int nr, hipStream_t st)
   }
   s->last_kernel = 4;
   s->last_nr = nr;
-  TreeArgs T {};
-  T.ops = s->d_tops;
-  T.in = s->d_tb; T.rhs = s->d_rhs; T.v = s->d_tv; T.cb = s->d_tc;
-  T.nmax = s->nmax;
-  T.nsolve = s->d_nsolve;
   const TreeDev* t = s->tree;
-  if (int rc = sweep (t, T, s->nmodes, nr, st)) return rc;
+  if (int rc = sweep (t, tree_args (s), s->nmodes, nr, st)) return rc;
   if (!s->sing) return SX_OK;
   const int nsp = t->P.nsolve;
   return refine (s, nr, s->d_tb + (size_t) s->sing->mode * nr * nsp, nsp, t->perm, st);
