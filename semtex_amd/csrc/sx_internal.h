@@ -71,15 +71,17 @@ namespace sx {
 // tree_solve: from the assembled right-hand sides in rhs_in (s) to d_rhs.
 struct TreeDev;
 struct TreeSing;
-int    tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always = false);
+int    tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always = false, int share = 1);
 void   tree_free (TreeDev* t);
 void   tree_sing_free (TreeSing* g);
-int    tree_workspace (sx_msys* s, int nr);
+int    tree_workspace (sx_msys* s, int nr, bool always = false);
 size_t tree_ops (const TreeDev* t);                 // doubles per mode of d_tops
 size_t tree_slots (const TreeDev* t);               // and per right-hand side of d_tc
 size_t tree_scratch (const TreeDev* t, int nm);     // doubles
 int    tree_factor (sx_msys* s, const double* Sel, double* buf, hipStream_t st, int* d_status);
 int    tree_solve (const sx_msys* s, int nr, hipStream_t st);
+// The system's dissection cut again for a batch (many solves side by side).
+int    tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_status);
 // A singular mode's refinement: its set-up (s->sing), and around a band
 // solve the right-hand sides kept before and the correction after.
 int    tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_status);

@@ -1753,6 +1753,7 @@ int msys_hold (sx_msys* s)
   } else {
     rc = elem_sc (m, s->nmodes, s->lambda2, s->d_betak2, buf, buf + nws, buf + nws + nS,
                   buf + nws + nS + nB, d_status + s->nmodes, nullptr);
+    if (!rc) rc = tree_for_batch (s, buf + nws, nullptr, d_status);
     if (!rc) rc = band_build (s, buf + nws, nullptr, d_status);
   }
   (void) hipFree (buf);

@@ -75,7 +75,9 @@ struct TreePlan {
 constexpr size_t TREE_LDS_MAX = 96 * 1024;   // a workgroup's column operand
 
 // false when the mesh does not suit it (an element holding one node twice,
-// a node no element holds, operators past the size bound)
-bool tree_plan (const sx_mesh* m, int nmodes, TreePlan& P);
+// a node no element holds, operators past the size bound).  share: solves
+// of this size that run side by side (a batch): a level's launches cost a
+// share-th each, so more and smaller levels pay.
+bool tree_plan (const sx_mesh* m, int nmodes, int share, TreePlan& P);
 
 }  // namespace sx

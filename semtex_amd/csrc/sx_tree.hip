@@ -533,10 +533,10 @@ template <typename V> int upload (V** d, const std::vector<V>& h)
 
 }  // namespace
 
-// A mesh's plan for one mode count with its tables on the device
+// A mesh's plan for one mode count and share with its tables on the device
 struct TreeDev {
   TreePlan P;
-  int nmodes = 0;
+  int nmodes = 0, share = 1;
   bool ok = false;
   TreeClass* cls = nullptr;
   TreeChild* child = nullptr;
@@ -567,21 +567,22 @@ static bool band_forced ()
 // that chooses a band layout.
 constexpr size_t TREE_OPS_MAX = (size_t) 3 << 30;      // doubles
 
-int tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always)
+int tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always, int share)
 {
   *out = nullptr;
   if ((!always && band_forced ()) || m->nband > 768) return SX_OK;
   std::lock_guard<std::mutex> lock (m->tree_mu);
   for (TreeDev* t : m->trees)
-    if (t->nmodes == nmodes) {
+    if (t->nmodes == nmodes && t->share == share) {
       *out = t->ok ? t : nullptr;
       return SX_OK;
     }
   TreeDev* t = new TreeDev;
   t->nmodes = nmodes;
+  t->share = share;
   m->trees.push_back (t);
   size_t f = 0;
-  t->ok = tree_plan (m, nmodes, t->P);
+  t->ok = tree_plan (m, nmodes, share, t->P);
   for (const TreeLevel& L : t->P.lev) f = std::max (f, L.fsize);
   t->ok = t->ok && t->P.ops * nmodes <= TREE_OPS_MAX && f * nmodes <= TREE_OPS_MAX;
   if (!t->ok) { t->P = TreePlan (); return SX_OK; }
@@ -794,7 +795,7 @@ void tree_sing_free (TreeSing* g)
 
 // Workspace of a solve with nr right-hand sides per mode, grown from the one
 // the system was created with (2)
-int tree_workspace (sx_msys* s, int nr)
+int tree_workspace (sx_msys* s, int nr, bool always)
 {
   auto grow = [&] (double** p, size_t n) {
     double* q = nullptr;
@@ -806,7 +807,7 @@ int tree_workspace (sx_msys* s, int nr)
   };
   const size_t n = (size_t) s->nmodes * nr;
   int rc;
-  if (s->tree && nr > s->rhs_cap) {
+  if (s->tree && (always || nr > s->rhs_cap)) {
     const TreePlan& P = s->tree->P;
     if ((rc = grow (&s->d_tb, n * P.nsolve)) || (rc = grow (&s->d_tv, n * P.nsolve)) ||
         (rc = grow (&s->d_tc, n * P.slots)))
@@ -828,6 +829,32 @@ const int* tree_perm (const sx_msys* s) { return s->tree->perm; }
 int tree_factor (sx_msys* s, const double* Sel, double* buf, hipStream_t st, int* d_status)
 {
   return factor (s->tree, s->m, s->nmodes, s->d_nsolve, Sel, s->d_tops, buf, st, d_status);
+}
+
+int tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_status)
+{
+  // (64 uneven problems: 309 us at 4, 318 at 8, 359 at 32, 360 with the
+  // systems' own cuts)
+  constexpr int BATCH_SHARE = 4;
+  TreeDev* t = nullptr;
+  if (int rc = tree_prepare (s->m, s->nmodes, &t, true, std::max (1, BATCH_SHARE / s->nmodes)))
+    return rc;
+  if (!t || t == s->tree) return SX_OK;
+  double *ops = nullptr, *buf = nullptr;
+  SX_HIP (hipMalloc (&ops, sizeof (double) * std::max<size_t> (t->P.ops * s->nmodes, 2)));
+  int rc = hipMalloc (&buf, sizeof (double) * tree_scratch (t, s->nmodes)) == hipSuccess
+               ? factor (t, s->m, s->nmodes, s->d_nsolve, Sel, ops, buf, st, d_status)
+               : hip_fail (hipErrorOutOfMemory, "tree_for_batch");
+  if (rc == SX_OK) rc = hipStreamSynchronize (st) == hipSuccess ? SX_OK : SX_ERR_HIP;
+  (void) hipFree (buf);
+  if (rc) {
+    (void) hipFree (ops);
+    return rc;
+  }
+  msys_free (s, s->d_tops);
+  s->d_tops = ops;
+  s->tree = t;
+  return tree_workspace (s, s->rhs_cap, true);
 }
 
 int tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_status)
