@@ -20,6 +20,8 @@
 // workgroup per plane.
 #include <algorithm>
 #include <cmath>
+#include <mutex>
+#include <utility>
 #include <vector>
 
 #include "sx_internal.h"
@@ -211,7 +213,7 @@ __device__ __forceinline__ double assemble_at (size_t idx, int nglobal, int npnp
 }
 
 struct PcgState {
-  double *x, *r, *p, *q, *z;        // [npl][npts]
+  double *x, *r, *p, *q;            // [npl][npts]
   double *rho, *eps, *r2;           // [npl]
   int *it, *active;                 // [npl]
 };
@@ -289,7 +291,7 @@ __global__ __launch_bounds__(PV_THREADS) void k_pcg_resid0 (
   }
 }
 
-// z = pc r, rho = r.z, p = z (+ rho/rho_old p)
+// the first direction: rho = r.z, p = z = pc r
 __global__ __launch_bounds__(PV_THREADS) void k_pcg_dir (
     const double* __restrict__ pc, size_t npts, PcgState st, int nz, int base_mode)
 {
@@ -297,63 +299,138 @@ __global__ __launch_bounds__(PV_THREADS) void k_pcg_dir (
   const int y = blockIdx.x, k = solved_plane (y, nz, base_mode);
   if (!st.active[y]) return;
   const double* pcm = pc + (size_t) (k >> 1) * npts;
-  double* r = st.r + (size_t) y * npts;
-  double* z = st.z + (size_t) y * npts;
+  const double* r = st.r + (size_t) y * npts;
   double* p = st.p + (size_t) y * npts;
   double rz = 0.0;
   for (size_t i = threadIdx.x; i < npts; i += PV_THREADS) {
     const double zi = pcm[i] * r[i];
-    z[i] = zi;
+    p[i] = zi;
     rz += r[i] * zi;
   }
   rz = block_sum (rz, red);
-  const bool first = st.it[y] == 0;
-  const double beta = first ? 0.0 : rz / st.rho[y];
-  for (size_t i = threadIdx.x; i < npts; i += PV_THREADS)
-    p[i] = first ? z[i] : beta * p[i] + z[i];
-  __syncthreads ();
   if (threadIdx.x == 0) st.rho[y] = rz;
 }
 
-// q = A p (masked); alpha = rho / p.q; x += alpha p; r -= alpha q; r2;
-// the next iteration runs while r2 > eps and ++i < STEP_MAX
-__global__ __launch_bounds__(PV_THREADS) void k_pcg_update (
+// q = A p (masked); alpha = rho / p.q; x += alpha p; r -= alpha q; r2; the
+// next iteration runs while r2 > eps and ++i < STEP_MAX, and its direction
+// z = pc r, rho' = r.z, p = z + rho'/rho p follows in the same launch (both
+// need the whole plane, one workgroup's).  R > 0: the plane's values stay in
+// registers, R a thread (npts <= R PV_THREADS), so a launch is its gather's
+// three rounds of loads and three sums; R = 0: any size, through memory.
+// 14.5 us as two launches walking memory, 6x8 elements at N_P=8.
+template <int R>
+__global__ __launch_bounds__(PV_THREADS) void k_pcg_step (
     int nglobal, int npnp, int next, const int* __restrict__ gptr,
     const int* __restrict__ gsrc, const int* __restrict__ nsolve,
-    const double* __restrict__ L, size_t lstride, PcgState st, size_t npts, int step_max,
-    int nz, int base_mode)
+    const double* __restrict__ L, size_t lstride, const double* __restrict__ pc, PcgState st,
+    size_t npts, int step_max, int nz, int base_mode)
 {
   __shared__ double red[PV_THREADS / 64];
   const int y = blockIdx.x, k = solved_plane (y, nz, base_mode), ns = nsolve[k >> 1];
   if (!st.active[y]) return;
   const double* Ly = L + (size_t) y * lstride;
+  const double* pcm = pc + (size_t) (k >> 1) * npts;
   double* p = st.p + (size_t) y * npts;
   double* q = st.q + (size_t) y * npts;
-  double pq = 0.0;
-  for (size_t i = threadIdx.x; i < npts; i += PV_THREADS) {
-    double v = 0.0;
-    if (!(i < (size_t) nglobal && (int) i >= ns))
-      v = assemble_at (i, nglobal, npnp, next, gptr, gsrc, Ly);
-    q[i] = v;
-    pq += p[i] * v;
-  }
-  pq = block_sum (pq, red);
-  const double alpha = st.rho[y] / pq;
   double* x = st.x + (size_t) y * npts;
   double* r = st.r + (size_t) y * npts;
-  double rr = 0.0;
-  for (size_t i = threadIdx.x; i < npts; i += PV_THREADS) {
-    x[i] += alpha * p[i];
-    const double ri = r[i] - alpha * q[i];
-    r[i] = ri;
-    rr += ri * ri;
+  const double rho = st.rho[y], eps = st.eps[y];
+  const int it = st.it[y] + 1;
+  constexpr int RR = R > 0 ? R : 1;
+  double pv[RR], qv[RR], xv[RR], rv[RR], cv[RR];
+  double pq = 0.0;
+  if constexpr (R > 0) {
+    const int nint = npnp - next;
+    int at[RR][4], n[RR], c0[RR];
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+      const int i = threadIdx.x + u * PV_THREADS;
+      n[u] = 0;
+      c0[u] = 0;
+      pv[u] = xv[u] = rv[u] = cv[u] = 0.0;
+      if (i < (int) npts) {
+        if (i < ns) { c0[u] = gptr[i]; n[u] = gptr[i + 1] - c0[u]; }
+        pv[u] = p[i];
+        xv[u] = x[i];
+        rv[u] = r[i];
+        cv[u] = pcm[i];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+      const int i = threadIdx.x + u * PV_THREADS;
+#pragma unroll
+      for (int c = 0; c < 4; c++) at[u][c] = c < n[u] ? gsrc[c0[u] + c] : -1;
+      if (i >= nglobal && i < (int) npts) {
+        const int e = i - nglobal;
+        at[u][0] = (e / nint) * npnp + next + e % nint;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+      double w[4], v = 0.0;
+#pragma unroll
+      for (int c = 0; c < 4; c++) w[c] = at[u][c] >= 0 ? Ly[at[u][c]] : 0.0;
+#pragma unroll
+      for (int c = 0; c < 4; c++) v += w[c];
+      for (int c = 4; c < n[u]; c++) v += Ly[gsrc[c0[u] + c]];
+      qv[u] = v;
+    }
+#pragma unroll
+    for (int u = 0; u < R; u++) pq += pv[u] * qv[u];
+  } else {
+    for (size_t i = threadIdx.x; i < npts; i += PV_THREADS) {
+      double v = 0.0;
+      if (!(i < (size_t) nglobal && (int) i >= ns))
+        v = assemble_at (i, nglobal, npnp, next, gptr, gsrc, Ly);
+      q[i] = v;
+      pq += p[i] * v;
+    }
+  }
+  pq = block_sum (pq, red);
+  const double alpha = rho / pq;
+  double rr = 0.0, rz = 0.0;
+  if constexpr (R > 0) {
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+      const int i = threadIdx.x + u * PV_THREADS;
+      rv[u] = rv[u] - alpha * qv[u];
+      rr += rv[u] * rv[u];
+      rz += rv[u] * (cv[u] * rv[u]);
+      if (i < (int) npts) {
+        x[i] = xv[u] + alpha * pv[u];
+        r[i] = rv[u];
+      }
+    }
+  } else {
+    for (size_t i = threadIdx.x; i < npts; i += PV_THREADS) {
+      x[i] += alpha * p[i];
+      const double ri = r[i] - alpha * q[i];
+      r[i] = ri;
+      rr += ri * ri;
+      rz += ri * (pcm[i] * ri);
+    }
   }
   rr = block_sum (rr, red);
+  const bool more = (rr > eps) && (it + 1 < step_max);
+  if (more) {
+    rz = block_sum (rz, red);
+    const double beta = rz / rho;
+    if constexpr (R > 0) {
+#pragma unroll
+      for (int u = 0; u < R; u++) {
+        const int i = threadIdx.x + u * PV_THREADS;
+        if (i < (int) npts) p[i] = beta * pv[u] + cv[u] * rv[u];
+      }
+    } else {
+      for (size_t i = threadIdx.x; i < npts; i += PV_THREADS) p[i] = beta * p[i] + pcm[i] * r[i];
+    }
+  }
   if (threadIdx.x == 0) {
-    const int it = st.it[y] + 1;
     st.it[y] = it;
     st.r2[y] = rr;
-    st.active[y] = (rr > st.eps[y]) && (it + 1 < step_max);
+    st.active[y] = more;
+    if (more) st.rho[y] = rz;
   }
 }
 
@@ -422,6 +499,58 @@ int pcg_setup (sx_msys* s, hipStream_t st)
 
 }  // namespace sx
 
+namespace {
+// Pinned copies of the planes' flags and their events.  One set (a few hundred
+// bytes) is kept for the next solve, a second thread's solve makes its own: a
+// pinned allocation costs more than the solve of a small system.
+struct PcgHostBuf {
+  int dev = -1, cap = 0;
+  int* mem = nullptr;
+  hipEvent_t ev[2] = {};
+  void drop ()
+  {
+    if (mem) (void) hipHostFree (mem);
+    for (hipEvent_t& e : ev)
+      if (e) { (void) hipEventDestroy (e); e = nullptr; }
+    mem = nullptr;
+    cap = 0;
+  }
+};
+struct PcgHost {
+  PcgHostBuf b;
+  int* flags[2];
+  hipEvent_t ev[2];
+  static std::mutex mu;
+  static PcgHostBuf kept;
+  int open (int npl)
+  {
+    int dev = 0;
+    SX_HIP (hipGetDevice (&dev));
+    {
+      std::lock_guard<std::mutex> lock (mu);
+      if (kept.mem && kept.dev == dev) std::swap (b, kept);
+    }
+    if (b.cap < npl) {
+      b.drop ();
+      b.dev = dev;
+      SX_HIP (hipHostMalloc ((void**) &b.mem, sizeof (int) * 2 * npl, hipHostMallocDefault));
+      b.cap = npl;
+      for (hipEvent_t& e : b.ev) SX_HIP (hipEventCreateWithFlags (&e, hipEventDisableTiming));
+    }
+    for (int i = 0; i < 2; i++) { flags[i] = b.mem + i * b.cap; ev[i] = b.ev[i]; }
+    return SX_OK;
+  }
+  ~PcgHost ()
+  {
+    std::lock_guard<std::mutex> lock (mu);
+    if (!kept.mem) std::swap (b, kept);
+    else b.drop ();
+  }
+};
+std::mutex PcgHost::mu;
+PcgHostBuf PcgHost::kept;
+}  // namespace
+
 extern "C" int sx_field_solve_pcg (sx_msys_t s, int nz, int stride, double* d_f, double* d_u,
                                    const double* d_lines, double tol_rel, int step_max,
                                    int* iters, void* stream)
@@ -442,8 +571,8 @@ extern "C" int sx_field_solve_pcg (sx_msys_t s, int nz, int stride, double* d_f,
   const size_t lstride = (size_t) m->nel * m->npnp;
   const int lstride_lines = m->nbound * m->np;
   const double* lines = (d_lines && m->nbound) ? d_lines : nullptr;
-  // workspace: L [npl][lstride], x r p q z [npl][npts], scalars
-  const size_t need = (size_t) npl * (lstride + 5 * npts) + 3 * (size_t) npl + 2 * (size_t) npl;
+  // workspace: L [npl][lstride], x r p q [npl][npts], scalars
+  const size_t need = (size_t) npl * (lstride + 4 * npts) + 3 * (size_t) npl + 2 * (size_t) npl;
   if (s->work_doubles < need) {
     if (s->d_work) (void) hipFree (s->d_work);
     s->d_work = nullptr;
@@ -457,8 +586,7 @@ extern "C" int sx_field_solve_pcg (sx_msys_t s, int nz, int stride, double* d_f,
   ps.r = ps.x + (size_t) npl * npts;
   ps.p = ps.r + (size_t) npl * npts;
   ps.q = ps.p + (size_t) npl * npts;
-  ps.z = ps.q + (size_t) npl * npts;
-  ps.rho = ps.z + (size_t) npl * npts;
+  ps.rho = ps.q + (size_t) npl * npts;
   ps.eps = ps.rho + npl;
   ps.r2 = ps.eps + npl;
   ps.it = (int*) (ps.r2 + npl);
@@ -485,33 +613,44 @@ extern "C" int sx_field_solve_pcg (sx_msys_t s, int nz, int stride, double* d_f,
                       m->npnp, m->next, m->d_gptr, m->d_gsrc, s->d_nsolve, L, lstride, ps,
                       npts, step_max, nz, s->base_mode);
   SX_HIP (hipGetLastError ());
-  std::vector<int> act (npl);
-  for (int iter = 1; iter < step_max; iter++) {
-    hipLaunchKernelGGL (k_pcg_dir, dim3 (npl), dim3 (PV_THREADS), 0, st, s->d_pc, npts, ps, nz,
-                        s->base_mode);
-    hipLaunchKernelGGL (k_pcg_op, dim3 (m->nel, npl), dim3 (64), 0, st, m->np, m->cyl,
-                        s->lambda2, s->d_betak2, m->d_geo, m->d_D, m->d_emap, m->d_btog,
-                        m->nglobal, ps.p, npts, L, lstride, ps.active, nz, s->base_mode);
-    hipLaunchKernelGGL (k_pcg_update, dim3 (npl), dim3 (PV_THREADS), 0, st, m->nglobal,
-                        m->npnp, m->next, m->d_gptr, m->d_gsrc, s->d_nsolve, L, lstride, ps,
-                        npts, step_max, nz, s->base_mode);
+  // The planes' active flags come back every GROUP iterations, and the next
+  // group is launched before the last one's are waited for: its launches
+  // find nothing active when those were the last iterations (a wait every
+  // four iterations idled the GPU for a quarter of the solve).
+  constexpr int GROUP = 4;
+  PcgHost H;
+  if (int rc = H.open (npl)) return rc;
+  const int regs = (int) ((npts + PV_THREADS - 1) / PV_THREADS);
+  auto step = regs <= 2 ? k_pcg_step<2> : regs <= 4 ? k_pcg_step<4> : regs <= 8 ? k_pcg_step<8>
+                                                                              : k_pcg_step<0>;
+  hipLaunchKernelGGL (k_pcg_dir, dim3 (npl), dim3 (PV_THREADS), 0, st, s->d_pc, npts, ps, nz,
+                      s->base_mode);
+  bool done = false;
+  for (int iter = 1, g = 0; iter < step_max && !done; g++) {
+    for (int i = 0; i < GROUP && iter < step_max; i++, iter++) {
+      hipLaunchKernelGGL (k_pcg_op, dim3 (m->nel, npl), dim3 (64), 0, st, m->np, m->cyl,
+                          s->lambda2, s->d_betak2, m->d_geo, m->d_D, m->d_emap, m->d_btog,
+                          m->nglobal, ps.p, npts, L, lstride, ps.active, nz, s->base_mode);
+      hipLaunchKernelGGL (step, dim3 (npl), dim3 (PV_THREADS), 0, st, m->nglobal, m->npnp,
+                          m->next, m->d_gptr, m->d_gsrc, s->d_nsolve, L, lstride, s->d_pc, ps,
+                          npts, step_max, nz, s->base_mode);
+    }
     SX_HIP (hipGetLastError ());
-    if (iter % 4 == 0 || iter + 1 >= step_max) {
-      SX_HIP (hipMemcpyAsync (act.data (), ps.active, sizeof (int) * npl,
-                              hipMemcpyDeviceToHost, st));
-      SX_HIP (hipStreamSynchronize (st));
-      if (std::none_of (act.begin (), act.end (), [] (int a) { return a != 0; })) break;
+    SX_HIP (hipMemcpyAsync (H.flags[g & 1], ps.active, sizeof (int) * npl, hipMemcpyDeviceToHost, st));
+    SX_HIP (hipEventRecord (H.ev[g & 1], st));
+    if (g) {
+      SX_HIP (hipEventSynchronize (H.ev[(g - 1) & 1]));
+      const int* f = H.flags[(g - 1) & 1];
+      done = std::none_of (f, f + npl, [] (int a) { return a != 0; });
     }
   }
   hipLaunchKernelGGL (k_pcg_finish, dim3 (m->nel, npl), dim3 (64), 0, st, m->np, m->d_emap,
                       m->d_btog, m->d_bmask, m->d_emask, s->d_G, m->nglobal, ps.x, npts, d_u,
                       stride, nz, s->base_mode);
   SX_HIP (hipGetLastError ());
-  if (iters) {
-    std::vector<int> its (npl);
-    SX_HIP (hipMemcpyAsync (its.data (), ps.it, sizeof (int) * npl, hipMemcpyDeviceToHost, st));
-    SX_HIP (hipStreamSynchronize (st));
-    *iters = *std::max_element (its.begin (), its.end ());
-  }
+  // (the flags' last copy ends before H goes)
+  SX_HIP (hipMemcpyAsync (H.flags[0], ps.it, sizeof (int) * npl, hipMemcpyDeviceToHost, st));
+  SX_HIP (hipStreamSynchronize (st));
+  if (iters) *iters = *std::max_element (H.flags[0], H.flags[0] + npl);
   return SX_OK;
 }
