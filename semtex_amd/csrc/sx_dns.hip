@@ -19,8 +19,8 @@
 //   k_gradz      Fourier z derivative (AuxField::gradient(2))
 //   k_ew_*       element-wise field algebra (the unfused z terms)
 //   k_smooth_*   mass-averaged direct stiffness sum on element boundaries
-//   k_hopbc      -d(u.n)/dt + n.N - nu n.curlcurl u on boundary segments
-//   k_plines     extrapolated dp/dn line data for the pressure solve
+//   k_hopbc      -d(u.n)/dt + n.N - nu n.curlcurl u on boundary segments, and
+//                from it the extrapolated dp/dn line data for the pressure
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -76,18 +76,21 @@ __global__ __launch_bounds__(64) void k_grad (int np, const double* __restrict__
 // Cartesian branches :162-193, :342-380, with Element::grad for every
 // derivative):
 //   N = -[conv (ux d_x u + uy d_y u) + cons (d_x (u ux) + d_y (u uy))]
-// written, not accumulated: the z terms are subtracted afterwards.
+// written, not accumulated: the z terms are subtracted afterwards.  A field
+// of one plane has none: scale (1/2 skew-symmetric) and the component's
+// constant force are applied here.
 // per-component arguments of a launch over up to three components
 // (blockIdx.z selects one)
 struct Comp3 {
   const double* in[3];
   double* out[3];
+  double add[3];
 };
 __global__ __launch_bounds__(64) void k_adv_xy (int np, const double* __restrict__ geo,
                                                 const double* __restrict__ Dg,
                                                 const double* __restrict__ ux,
                                                 const double* __restrict__ uy, Comp3 cmp,
-                                                int stride, int conv, int cons)
+                                                int stride, int conv, int cons, double scale)
 {
   const double* __restrict__ ui = cmp.in[blockIdx.z];
   double* N = cmp.out[blockIdx.z];
@@ -132,7 +135,7 @@ __global__ __launch_bounds__(64) void k_adv_xy (int np, const double* __restrict
     double v = 0.0;
     if (conv) v += ax[t] * (ur * rx[t] + us * sx[t]) + ay[t] * (ur * ry[t] + us * sy[t]);
     if (cons) v += (xr * rx[t] + xs * sx[t]) + (yr * ry[t] + ys * sy[t]);
-    N[off + ij] = -v;
+    N[off + ij] = -v * scale + cmp.add[blockIdx.z];
   }
 }
 
@@ -418,7 +421,8 @@ __global__ __launch_bounds__(64) void k_hopbc (
     const double* __restrict__ U2, const double* __restrict__ N0,
     const double* __restrict__ N1, double* hop_new, double* un_new,
     const double* __restrict__ un1, int Je, double a0, Coef3 acoef, double inv_dt, double nu,
-    double beta, int nz, int nline, int S)
+    double beta, int nz, int nline, int S, double* lines, Levels hop, int Jb,
+    const int* __restrict__ kind)
 {
   const int npnp = np * np, b = blockIdx.x, m = blockIdx.y, lane = threadIdx.x;
   const int e = seg_elmt[b];
@@ -538,21 +542,18 @@ __global__ __launch_bounds__(64) void k_hopbc (
       hop_new[orr] += -nu * yr * ny[q0];
       hop_new[oi] += -nu * yi * ny[q0];
     }
+    // evaluateCNBCp: lines[k] = sum_q beta_q hop[q][k], hop[0] the level just
+    // formed; essential pressure segments zero
+    for (int pl = 0; pl < (three ? 2 : 1); pl++) {
+      const size_t o = (size_t) (pl ? ki : kr) * nline + jl;
+      double v = 0.0;
+      if (kind[b] == SX_NATURAL) {
+        v += hop.c[0] * hop_new[o];
+        for (int q = 1; q < Jb; q++) v += hop.c[q] * hop.f[q][o];
+      }
+      lines[o] = v;
+    }
   }
-}
-
-// evaluateCNBCp: lines[k] = sum_q beta_q hop[q][k]; Nyquist plane and
-// essential pressure segments zero.
-__global__ void k_plines (double* lines, Levels hop, int Je, int nz, int nline, int np,
-                          const int* __restrict__ kind)
-{
-  const size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t) nz * nline) return;
-  const int k = (int) (i / nline), j = (int) (i % nline);
-  double v = 0.0;
-  if (!(nz > 1 && k == 1) && kind[j / np] == SX_NATURAL)
-    for (int q = 0; q < Je; q++) v += hop.c[q] * hop.f[q][i];
-  lines[i] = v;
 }
 
 inline unsigned nb256 (size_t n) { return (unsigned) ((n + 255) / 256); }
@@ -660,7 +661,7 @@ void adv_xy (sx_dns* d, double* const* ui, double* const* N, int nf, bool conv, 
     c.out[i] = N[i];
   }
   hipLaunchKernelGGL (k_adv_xy, dim3 (m->nel, d->nz, nf), dim3 (64), 0, st, m->np, m->d_geo,
-                      m->d_D, d->phys[0], d->phys[1], c, d->S, (int) conv, (int) cons);
+                      m->d_D, d->phys[0], d->phys[1], c, d->S, (int) conv, (int) cons, 1.0);
 }
 
 #define EW(kern, ...) \
@@ -709,7 +710,7 @@ int advection32 (sx_dns* d, double** U, double** N, hipStream_t st)
     c.in[0] = d->physM[i];
     c.out[0] = d->tmpM;
     hipLaunchKernelGGL (k_adv_xy, dim3 (m->nel, M), dim3 (64), 0, st, m->np, m->d_geo, m->d_D,
-                        d->physM[0], d->physM[1], c, d->S, 1, 1);
+                        d->physM[0], d->physM[1], c, d->S, 1, 1, 1.0);
     if ((rc = zgemm (d, U[i], d->Wdz, d->tmpM2, nz, M, 1.0))) return rc;
     hipLaunchKernelGGL (k_ew_submul, dim3 (gM), dim3 (256), 0, st, d->tmpM, d->physM[2],
                         d->tmpM2, d->nM);
@@ -776,6 +777,23 @@ int advection (sx_dns* d, double** U, double** N, hipStream_t st)
     if ((rc = smooth_n (d, N, 3, st))) return rc;
     if (d->advection == SX_ALTSKEW) d->toggle = 1 - d->toggle;
     SX_HIP (hipGetLastError ());
+    return SX_OK;
+  }
+  if (d->nz == 1) {
+    // one plane is its own transform and has no z terms: both components'
+    // terms, factor and force in one launch, the smoothing in another
+    Comp3 c {};
+    for (int i = 0; i < nc; i++) {
+      c.in[i] = U[i];
+      c.out[i] = N[i];
+      c.add[i] = std::fabs (d->cf[i]) > EPSDP ? d->cf[i] : 0.0;
+    }
+    hipLaunchKernelGGL (k_adv_xy, dim3 (m->nel, 1, nc), dim3 (64), 0, st, m->np, m->d_geo, m->d_D,
+                        U[0], U[1], c, d->S, (int) conv, (int) cons,
+                        d->advection == SX_SKEW ? 0.5 : 1.0);
+    SX_HIP (hipGetLastError ());
+    if ((rc = smooth_n (d, N, nc, st))) return rc;
+    if (d->advection == SX_ALTSKEW) d->toggle = 1 - d->toggle;
     return SX_OK;
   }
   for (int i = 0; i < nc; i++)
@@ -856,22 +874,19 @@ int dns_step (sx_dns* d, hipStream_t st)
     // (the plane padding is never written and stays zero)
     const int nmodes = std::max (1, d->nz / 2);
     Coef3 ac = {{SSc[Je][1], SSc[Je][2], SSc[Je][3]}};
-    hipLaunchKernelGGL (k_hopbc, dim3 (d->nb, nmodes), dim3 (64), 0, st, d->mu->np,
-                        d->seg_elmt, d->seg_idx, d->seg_nx, d->seg_ny, d->mu->d_geo,
-                        d->mu->d_D, U[0], U[1], nc == 3 ? U[2] : U[0], N[0], N[1], hnew,
-                        unnew, un1, Je, SSc[Je][0], ac, 1.0 / d->dt, d->nu, d->beta, d->nz,
-                        d->nline, d->S);
-    SX_HIP (hipGetLastError ());
-    d->un_head = 1 - d->un_head;
     const int Jb = std::min (d->step, nord);
     Levels hl = {};
     for (int q = 0; q < Jb; q++) {
       hl.f[q] = d->hop[(d->hop_head + q) % nord];
       hl.c[q] = EXc[Jb][q];
     }
-    hipLaunchKernelGGL (k_plines, dim3 (nb256 ((size_t) d->nz * d->nline)), dim3 (256), 0,
-                        st, d->plines, hl, Jb, d->nz, d->nline, d->mu->np, d->seg_kind);
+    hipLaunchKernelGGL (k_hopbc, dim3 (d->nb, nmodes), dim3 (64), 0, st, d->mu->np,
+                        d->seg_elmt, d->seg_idx, d->seg_nx, d->seg_ny, d->mu->d_geo,
+                        d->mu->d_D, U[0], U[1], nc == 3 ? U[2] : U[0], N[0], N[1], hnew,
+                        unnew, un1, Je, SSc[Je][0], ac, 1.0 / d->dt, d->nu, d->beta, d->nz,
+                        d->nline, d->S, d->plines, hl, Jb, d->seg_kind);
     SX_HIP (hipGetLastError ());
+    d->un_head = 1 - d->un_head;
     plines = d->plines;
   }
   // -- waveProp
@@ -1075,7 +1090,8 @@ extern "C" int sx_dns_create (sx_mesh_t mu, sx_mesh_t mp, int nz, double beta,
         hipMemcpy (d->seg_nx, nxv.data (), sizeof (double) * nxv.size (), hipMemcpyHostToDevice) ||
         hipMemcpy (d->seg_ny, nyv.data (), sizeof (double) * nyv.size (), hipMemcpyHostToDevice))
       return fail (hip_fail (hipErrorUnknown, "sx_dns_create copy"));
-    for (double* q : {d->hop[0], d->hop[1], d->hop[2], d->un[0], d->un[1]})
+    // (the Nyquist plane of the line data is never written)
+    for (double* q : {d->hop[0], d->hop[1], d->hop[2], d->un[0], d->un[1], d->plines})
       if (q && hipMemsetAsync (q, 0, sizeof (double) * nz * d->nline, st))
         return fail (hip_fail (hipErrorUnknown, "sx_dns_create memset"));
   }
