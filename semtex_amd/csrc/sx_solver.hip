@@ -242,36 +242,68 @@ __global__ __launch_bounds__(256) void k_elem_sc_lds (
     return helm_entry (np, emap[a], emap[b], G, G + npnp, G + 2 * npnp, G + 3 * npnp,
                        G + 4 * npnp, D, lambda2, bk2, cyl, hasQ3);
   };
+  // this block's workspace: hbi, hii and a residual (2 next nint <= npnp^2)
+  double* Hb = ws + (size_t) blk * (npnp * npnp + nint * nint);
+  double* Hc = Hb + next * nint;
+  double* Rg = Hc + nint * nint;
   for (int i = tid; i < N * N; i += 256) {
     const int a = i / N, b = i % N;
-    P[a * LD + b] = a < nint && b < nint ? entry (next + a, next + b) : a == b ? 1.0 : 0.0;
+    const bool in = a < nint && b < nint;
+    const double h = in ? entry (next + a, next + b) : a == b ? 1.0 : 0.0;
+    P[a * LD + b] = h;
+    if (in) Hc[a * nint + b] = h;
   }
-  // hbi, kept in this block's workspace
-  double* Hb = ws + (size_t) blk * (npnp * npnp + nint * nint);
   for (int i = tid; i < next * nint; i += 256) Hb[i] = entry (i / nint, next + i % nint);
   __syncthreads ();
   spd_invert (P, LD, N / 16, W, Di, &s_bad);
   if (s_bad) { if (tid == 0) atomicExch (status, 1); return; }
   double* Hi = Hinv + ((size_t) mode * nclass + cls) * nint * nint;
   for (int i = tid; i < nint * nint; i += 256) Hi[i] = P[(i / nint) * LD + i % nint];
-  // Bm = hbi inv(hii), then S = hbb - Bm hbi^T, 16x16 tiles
+  // Bm = hbi inv(hii), corrected once by its residual, and S = hbb - Bm
+  // hbi^T, 16x16 tiles.  (The inverse's rounding is the same in every element
+  // of a class: without the correction its row sums in S, a spurious constant
+  // term, moved the pure-Neumann pressure by 6e-10 in five channel steps.)
   double* B = Bm + ((size_t) mode * nclass + cls) * next * nint;
   const int ne = (next + 15) / 16, nk = N / 4, lr = lane & 15, lq = lane >> 4;
-  for (int t = wave; t < ne * (N / 16); t += 4) {
-    const int i0 = 16 * (t % ne), j0 = 16 * (t / ne), row = min (i0 + lr, next - 1);
-    v4d acc = {};
-    for (int s = 0; s < nk; s++) {
-      const int kk = 4 * s + lq;
-      const double h = kk < nint ? Hb[(size_t) row * nint + kk] : 0.0;
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64 (h, P[kk * LD + j0 + lr], acc, 0, 0, 0);
-    }
+  for (int pass = 0; pass < 2; pass++) {
+    const double* X = pass ? Rg : Hb;      // B (+)= X inv(hii)
+    for (int t = wave; t < ne * (N / 16); t += 4) {
+      const int i0 = 16 * (t % ne), j0 = 16 * (t / ne), row = min (i0 + lr, next - 1);
+      v4d acc = {};
+      for (int s = 0; s < nk; s++) {
+        const int kk = 4 * s + lq;
+        const double h = kk < nint ? X[(size_t) row * nint + kk] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64 (h, P[kk * LD + j0 + lr], acc, 0, 0, 0);
+      }
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int a = i0 + 4 * r + lq, b = j0 + lr;
-      if (a < next && b < nint) B[(size_t) a * nint + b] = acc[r];
+      for (int r = 0; r < 4; r++) {
+        const int a = i0 + 4 * r + lq, b = j0 + lr;
+        if (a < next && b < nint) {
+          double* o = B + (size_t) a * nint + b;
+          *o = pass ? *o + acc[r] : acc[r];
+        }
+      }
     }
+    __syncthreads ();
+    if (pass) break;
+    // R = hbi - B hii
+    for (int t = wave; t < ne * (N / 16); t += 4) {
+      const int i0 = 16 * (t % ne), j0 = 16 * (t / ne), row = min (i0 + lr, next - 1),
+                col = min (j0 + lr, nint - 1);
+      v4d acc = {};
+      for (int s = 0; s < nk; s++) {
+        const int kk = min (4 * s + lq, nint - 1);
+        const double h = 4 * s + lq < nint ? B[(size_t) row * nint + kk] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64 (h, Hc[(size_t) kk * nint + col], acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int a = i0 + 4 * r + lq, b = j0 + lr;
+        if (a < next && b < nint) Rg[(size_t) a * nint + b] = Hb[(size_t) a * nint + b] - acc[r];
+      }
+    }
+    __syncthreads ();
   }
-  __syncthreads ();
   double* So = S + ((size_t) mode * nclass + cls) * next * next;
   for (int t = wave; t < ne * ne; t += 4) {
     const int i0 = 16 * (t % ne), j0 = 16 * (t / ne);
