@@ -33,6 +33,7 @@ using namespace sx;
 
 namespace {
 
+typedef double v4d __attribute__ ((ext_vector_type (4)));
 constexpr double EPSDP = 6.0e-14;
 
 // x or y derivative of every element of every plane (Element::grad,
@@ -588,6 +589,9 @@ struct sx_dns {
   size_t nM = 0;                       // M * S
   double *physM[3] = {}, *tmpM = nullptr, *tmpM2 = nullptr;
   double *Wi = nullptr, *Wdz = nullptr, *Wf = nullptr;   // [N][M], [N][M], [M][N]
+  // the same transforms on own MFMA tiles (zmat_ok): operators in fragment
+  // order, one dealiased product field per component
+  double *Zi = nullptr, *Zdz = nullptr, *Zf = nullptr, *prodM[3] = {};
   rocblas_handle blas = nullptr;
 
   double* alloc (size_t cnt)
@@ -686,6 +690,141 @@ int zgemm (sx_dns* d, const double* X, const double* W, double* out, int inner, 
   return SX_OK;
 }
 
+// The dealiased z transforms as FP64 MFMA products of a fixed matrix W (rows x
+// K, fragment order: per 16-row block and pair of k steps [lane][2]) with
+// the columns of a field, fused with what surrounds them; all components in
+// one launch (blockIdx.z), 32 columns a workgroup, the columns staged
+// through LDS ZK rows at a time while the outputs stay in registers.
+//   EPI 0: out = W x            (velocity onto M planes)
+//   EPI 1: out -= mul .* (W x)  (convective z term, w d_z u)
+//   EPI 2: out = W [x; y .* mul], add on plane 0 (back to N planes: the
+//          summed products and, differentiated, the conservative z term)
+// A step's dealiasing is 4 launches instead of 27 (12 library products with
+// element-wise launches between them, ~5 us each at 48 planes).
+struct ZMat {
+  const double* W;
+  int rows, K, kx;                     // kx: k rows from x, the rest from y .* mul
+  const double *x[3], *y[3], *mul;
+  double* out[3];
+  double add[3];
+  int S;
+};
+constexpr int ZC = 32, ZK = 96, ZLD = ZC + 2, ZRB = 3;
+bool zmat_ok (int nz) { return 3 * nz / 2 <= 64 * ZRB; }
+
+template <int RB, int EPI>
+__global__ __launch_bounds__(256) void k_zmat (ZMat Z)
+{
+  __shared__ double X[ZK * ZLD];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = blockIdx.z;
+  const int col0 = blockIdx.x * ZC, S = Z.S, np = (Z.K + 7) / 8;
+  v4d acc[RB][2] = {};
+  const double2* A = (const double2*) Z.W + lane;
+  for (int k0 = 0; k0 < Z.K; k0 += ZK) {
+    // (S even: the last tile's pairs of columns end with it)
+    double2 v[ZK / 16], w[ZK / 16];
+#pragma unroll
+    for (int u = 0; u < ZK / 16; u++) {
+      const int k = min (k0 + 16 * u + (tid >> 4), Z.K - 1), cl = min (col0 + 2 * (tid & 15), S - 2);
+      const bool first = EPI != 2 || k < Z.kx;
+      const size_t at = (size_t) (first ? k : k - Z.kx) * S + cl;
+      v[u] = *(const double2*) ((first ? Z.x[c] : Z.y[c]) + at);
+      w[u] = make_double2 (1.0, 1.0);
+      if (EPI == 2 && !first) w[u] = *(const double2*) (Z.mul + at);
+    }
+    if (k0) __syncthreads ();
+#pragma unroll
+    for (int u = 0; u < ZK / 16; u++) {
+      const int kl = 16 * u + (tid >> 4);
+      const bool in = k0 + kl < Z.K;
+      X[kl * ZLD + 2 * (tid & 15)] = in ? v[u].x * w[u].x : 0.0;
+      X[kl * ZLD + 2 * (tid & 15) + 1] = in ? v[u].y * w[u].y : 0.0;
+    }
+    __syncthreads ();
+    const int p0 = k0 / 8, p1 = min (p0 + ZK / 8, np);
+#pragma unroll
+    for (int r = 0; r < RB; r++) {
+      const int rb = wave + 4 * r;
+      if (16 * rb >= Z.rows) continue;
+#pragma unroll 4
+      for (int p = p0; p < p1; p++) {
+        const double2 a = A[((size_t) rb * np + p) * 64];
+        const double* b = X + (8 * (p - p0) + (lane >> 4)) * ZLD + (lane & 15);
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+          acc[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a.x, b[16 * t], acc[r][t], 0, 0, 0);
+          acc[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64 (a.y, b[4 * ZLD + 16 * t], acc[r][t], 0,
+                                                            0, 0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RB; r++)
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int row = 16 * (wave + 4 * r) + 4 * q + (lane >> 4), col = col0 + 16 * t + (lane & 15);
+        if (row >= Z.rows || col >= S) continue;
+        double* o = Z.out[c] + (size_t) row * S + col;
+        if (EPI == 0) *o = acc[r][t][q];
+        else if (EPI == 1) *o -= Z.mul[(size_t) row * S + col] * acc[r][t][q];
+        else *o = acc[r][t][q] + (row == 0 ? Z.add[c] : 0.0);
+      }
+}
+
+template <int EPI> int zmat (const ZMat& Z, int nc, hipStream_t st)
+{
+  const dim3 grid ((Z.S + ZC - 1) / ZC, 1, nc);
+  const int rb = (Z.rows + 63) / 64;
+  if (rb <= 1) hipLaunchKernelGGL ((k_zmat<1, EPI>), grid, dim3 (256), 0, st, Z);
+  else if (rb == 2) hipLaunchKernelGGL ((k_zmat<2, EPI>), grid, dim3 (256), 0, st, Z);
+  else hipLaunchKernelGGL ((k_zmat<ZRB, EPI>), grid, dim3 (256), 0, st, Z);
+  SX_HIP (hipGetLastError ());
+  return SX_OK;
+}
+
+// skewSymmetric with dealiased products, as advection32 below, on k_zmat
+int advection32_z (sx_dns* d, double** U, double** N, hipStream_t st)
+{
+  const int nz = d->nz, M = d->M;
+  const sx_mesh* m = d->mu;
+  int rc;
+  ZMat Z {};
+  Comp3 c {};
+  Z.S = d->S;
+  for (int i = 0; i < 3; i++) {
+    Z.x[i] = U[i];
+    Z.out[i] = d->physM[i];
+    c.in[i] = d->physM[i];
+    c.out[i] = d->prodM[i];
+  }
+  Z.rows = M;
+  Z.K = Z.kx = nz;
+  Z.W = d->Zi;
+  if ((rc = zmat<0> (Z, 3, st))) return rc;
+  hipLaunchKernelGGL (k_adv_xy, dim3 (m->nel, M, 3), dim3 (64), 0, st, m->np, m->d_geo, m->d_D,
+                      d->physM[0], d->physM[1], c, d->S, 1, 1, 1.0);
+  SX_HIP (hipGetLastError ());
+  Z.W = d->Zdz;
+  Z.mul = d->physM[2];
+  for (int i = 0; i < 3; i++) Z.out[i] = d->prodM[i];
+  if ((rc = zmat<1> (Z, 3, st))) return rc;
+  Z.W = d->Zf;
+  Z.rows = nz;
+  Z.K = 2 * M;
+  Z.kx = M;
+  for (int i = 0; i < 3; i++) {
+    Z.x[i] = d->prodM[i];
+    Z.y[i] = d->physM[i];
+    Z.out[i] = N[i];
+    Z.add[i] = std::fabs (d->cf[i]) > EPSDP ? d->cf[i] : 0.0;
+  }
+  if ((rc = zmat<2> (Z, 3, st))) return rc;
+  return smooth_n (d, N, 3, st);
+}
+
 // skewSymmetric (dns/nonlinear.cpp:162-193) with every product in z formed
 // on M = 3N/2 physical planes (AuxField::transform32,
 // src/auxfield.cpp:1197-1258, with the 3/2 rule): the velocity and its z
@@ -695,6 +834,7 @@ int zgemm (sx_dns* d, const double* X, const double* W, double* out, int inner, 
 // from the truncated product.
 int advection32 (sx_dns* d, double** U, double** N, hipStream_t st)
 {
+  if (d->Zi) return advection32_z (d, U, N, st);
   const int nc = d->ncom, nz = d->nz, M = d->M;
   const sx_mesh* m = d->mu;
   int rc;
@@ -1157,19 +1297,23 @@ extern "C" int sx_dns_set_dealias (sx_dns_t d, int on, void* stream)
     return SX_ERR_ARG;
   }
   (void) stream;
-  if (on && !d->blas) {
+  if (on && !d->M) {
     const int N = d->nz, M = 3 * N / 2;
-    d->M = M;
-    d->nM = (size_t) M * d->S;
-    if (rocblas_create_handle (&d->blas) != rocblas_status_success) {
+    // N past 128 (more than 192 rows, the three blocks a wavefront k_zmat
+    // keeps in registers): library products.  A step of 12x24 N_P=8 N_Z=128
+    // 1518 -> 1045 us on k_zmat, 4x6 N_P=6 N_Z=256 369 -> 464 us.
+    const bool own = zmat_ok (N);
+    if (!own && !d->blas && rocblas_create_handle (&d->blas) != rocblas_status_success) {
       set_error ("rocblas_create_handle failed");
       return SX_ERR_HIP;
     }
+    d->nM = (size_t) M * d->S;
     for (int i = 0; i < 3; i++)
-      if (!(d->physM[i] = d->alloc (d->nM))) return hip_fail (hipErrorOutOfMemory, "dealias");
-    if (!(d->tmpM = d->alloc (d->nM)) || !(d->tmpM2 = d->alloc (d->nM)) ||
-        !(d->Wi = d->alloc ((size_t) N * M)) || !(d->Wdz = d->alloc ((size_t) N * M)) ||
-        !(d->Wf = d->alloc ((size_t) N * M)))
+      if (!(d->physM[i] = d->alloc (d->nM)) || (own && !(d->prodM[i] = d->alloc (d->nM))))
+        return hip_fail (hipErrorOutOfMemory, "dealias");
+    if (!own && (!(d->tmpM = d->alloc (d->nM)) || !(d->tmpM2 = d->alloc (d->nM)) ||
+                 !(d->Wi = d->alloc ((size_t) N * M)) || !(d->Wdz = d->alloc ((size_t) N * M)) ||
+                 !(d->Wf = d->alloc ((size_t) N * M))))
       return hip_fail (hipErrorOutOfMemory, "dealias");
     // packed real DFT matrices (femlib/fourier.c packing, the Nyquist plane
     // of the N planes dropped): Wi (N x M, ld N) evaluates modes 0..N/2-1
@@ -1192,10 +1336,41 @@ extern "C" int sx_dns_set_dealias (sx_dns_t d, int on, void* stream)
         wf[(size_t) (2 * k + 1) * M + j] = -sn / M;
       }
     }
-    if (hipMemcpy (d->Wi, wi.data (), sizeof (double) * wi.size (), hipMemcpyHostToDevice) ||
+    if (own) {
+      // (the padding of the product planes is never written)
+      for (int i = 0; i < 3; i++) SX_HIP (hipMemset (d->prodM[i], 0, sizeof (double) * d->nM));
+      SX_HIP (hipStreamSynchronize (nullptr));
+      // fragment order (k_zmat); the way back takes the summed products
+      // through Wf / 2 and u w through its z derivative, -d_z Wf / 2
+      auto upload_frag = [&] (int rows, int K, auto at, double** dev) -> int {
+        const int np = (K + 7) / 8, nb = (rows + 15) / 16;
+        std::vector<double> f ((size_t) nb * np * 128, 0.0);
+        for (size_t q = 0; q < f.size (); q++) {
+          const int l = (int) ((q >> 1) & 63), row = 16 * (int) ((q >> 7) / np) + (l & 15),
+                    k = 4 * (2 * (int) ((q >> 7) % np) + (int) (q & 1)) + (l >> 4);
+          if (row < rows && k < K) f[q] = at (row, k);
+        }
+        if (!(*dev = d->alloc (f.size ()))) return hip_fail (hipErrorOutOfMemory, "dealias");
+        SX_HIP (hipMemcpy (*dev, f.data (), sizeof (double) * f.size (), hipMemcpyHostToDevice));
+        return SX_OK;
+      };
+      auto back = [&] (int r, int k) {
+        if (k < M) return 0.5 * wf[(size_t) r * M + k];
+        const double bk = d->beta * (r >> 1);
+        if (r < 2) return 0.0;
+        return (r & 1) ? -0.5 * bk * wf[(size_t) (r - 1) * M + k - M]
+                       : 0.5 * bk * wf[(size_t) (r + 1) * M + k - M];
+      };
+      int rc;
+      if ((rc = upload_frag (M, N, [&] (int r, int k) { return wi[(size_t) r * N + k]; }, &d->Zi)) ||
+          (rc = upload_frag (M, N, [&] (int r, int k) { return wdz[(size_t) r * N + k]; }, &d->Zdz)) ||
+          (rc = upload_frag (N, 2 * M, back, &d->Zf)))
+        return rc;
+    } else if (hipMemcpy (d->Wi, wi.data (), sizeof (double) * wi.size (), hipMemcpyHostToDevice) ||
         hipMemcpy (d->Wdz, wdz.data (), sizeof (double) * wdz.size (), hipMemcpyHostToDevice) ||
         hipMemcpy (d->Wf, wf.data (), sizeof (double) * wf.size (), hipMemcpyHostToDevice))
       return hip_fail (hipErrorUnknown, "dealias matrices");
+    d->M = M;
   }
   d->dealias = on ? 1 : 0;
   return SX_OK;
