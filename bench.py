@@ -16,9 +16,8 @@ splitting with skew-symmetric advection, Poiseuille + seeded 1e-2
 perturbation; 100 steps timed.
 
 Prints ONE JSON line: the Helmholtz rate as `value`, both precision
-variants, the DNS rate, a roofline entry for the dominant kernel (the
-banded FP64 triangular sweeps, HBM-bound) measured with HIP events on the
-solve stream, and the CPU oracle timed on bounded samples of the same
+variants, the DNS rate, a roofline entry for the condensed FP64 solve (the
+dissection's levels) measured with HIP events on the solve stream, and the CPU oracle timed on bounded samples of the same
 workloads.
 """
 from __future__ import annotations
@@ -68,21 +67,6 @@ def parse():
                    help="only copy 256 MiB device to device 3 times (the reference "
                         "kernel for scaling rocprofv3 FETCH_SIZE / WRITE_SIZE)")
     return p.parse_args()
-
-
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "band_sweep_hbm_traffic.json")
-
-
-def measured_traffic(workload):
-    """HBM bytes per band-solve launch from the committed rocprofv3 counter
-    summary of this workload (FETCH_SIZE + WRITE_SIZE, copy-calibrated), or
-    None when there is none for it."""
-    try:
-        with open(TRAFFIC_FILE) as f:
-            t = json.load(f)
-    except (OSError, ValueError):
-        return None
-    return t.get("traffic_bytes_per_launch") if t.get("workload") == workload else None
 
 
 def copy_calibration(torch):
@@ -268,21 +252,23 @@ FIELDS = ("u", "v", "w", "p")
 
 def dns_roofline(dn):
     """Algorithmic HBM bytes of one DNS step over its time: every mode's
-    velocity and pressure band factor read once (the grouped velocity solve
-    reads the velocity factor once for u, v, w), plus 40 passes over an
+    velocity and pressure solve operators read once (the grouped velocity
+    solve reads the velocity's once for u, v, w), plus 40 passes over an
     [nz][S] field: advection 6 (u in, N out), waveProp 15 (4 history levels
     of 3 fields in, H out), divergence 4, pressure solve 2, projection 7,
     velocity solves 6."""
+    from semtex_amd.solver import ModalMatrixSys
     P, D = dn["P"], dn["D"]
-    mu, mp = P["mesh_u"], P["mesh_p"]
     nm = P["nz"] // 2
-    band = 8 * nm * (mu.nsolve * mu.nband + mp.nsolve * mp.nband)
+    lam2 = 1.5 / (P["dt"] * P["kinvis"])
+    band = 8 * nm * sum(ModalMatrixSys(lam, P["beta"], 0, nm, g).layout()["operators"]
+                        for lam, g in ((lam2, D.gu), (0.0, D.gp)))
     fields = 40 * 8 * P["nz"] * D.stride
     total = band + fields
     achieved = total / (dn["ms_per_step"] * 1e-3) / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "algorithmic_bytes": total,
-            "band_bytes": band, "field_bytes": fields}
+            "operator_bytes": band, "field_bytes": fields}
 
 
 def dns_parity(dn, torch):
@@ -537,21 +523,24 @@ def main():
             value, chosen = mx["value"], "mixed"
         del mx
 
-    # algorithmic bytes of one band-solve launch: every mode's factor once
-    # (8 nsolve nband) + its right-hand sides read and solutions written
+    # bytes of one condensed solve: the dissection's operators of every mode
+    # once (the band factor, 8 nsolve nband, where a system solves by it) and
+    # its right-hand sides read and solutions written
     M = f64["M"]
+    lay = M.layout()
     band_bytes = 0
     for md in range(nmodes):
         ns = M.nsolve(md)
         nrhs = 1 if md == 0 else 2
-        band_bytes += 8 * ns * m.nband + 16 * ns * nrhs
+        factor = 8 * lay["operators"] if lay["kernel"] == 4 else 8 * ns * m.nband
+        band_bytes += factor + 16 * ns * nrhs
     phases = f64["phases"]
     band_ms = phases["band_solve"]
     achieved = band_bytes / (band_ms * 1e-3) / 1e9
 
     workload = ("batched 2.5D Helmholtz, 16x16 elements on [0,2pi]x[-1,1], N_P=10, "
                 "N_Z=64 (32 modes, beta=1, lambda2=1+k^2), Dirichlet y=+-1, periodic x, "
-                "seeded Gaussian forcing ~(1+k)^-2; static condensation + banded Cholesky")
+                "seeded Gaussian forcing ~(1+k)^-2; static condensation + direct solve by dissection")
     out = {
         "metric": METRIC,
         "value": round(value, 2),
@@ -574,13 +563,13 @@ def main():
         },
         "variants": variants,
         "roofline": {
-            "kernel": "k_band_solve",
+            "kernel": "k_tree_level" if lay["kernel"] == 4 else "k_band_solve",
             "bound": "hbm",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": measured_traffic(workload),
+            "traffic": None,
             "algorithmic_bytes": band_bytes,
             "avg_ms": round(band_ms, 5),
         },

@@ -145,8 +145,10 @@ int sx_msys_nsolve (sx_msys_t s, int mode);
  * info[3] band width nband; info[4] 1 = unit-diagonal panels (W = T_J U);
  * info[5] kernel of the last band solve: 0 none yet, 1 panel sweeps with
  * the triangle in the chain, 2 unit-diagonal sweeps, 3 split sweeps (two
- * workgroups per chain); info[6] its right-hand sides per workgroup.
- * Fills min(n, 7) entries. */
+ * workgroups per chain); info[6] its right-hand sides per workgroup; info[5]
+ * 4: the dissection solve, info[6] its right-hand sides per mode; info[7]
+ * doubles per mode of the dissection's operators (0: band only).
+ * Fills min(n, 8) entries. */
 int sx_msys_layout (sx_msys_t s, int* info, int n);
 
 /* Field::solve (src/field.cpp:598-709, DIRECT branch) over nz planes.

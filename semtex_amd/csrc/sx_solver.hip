@@ -2,19 +2,21 @@
 // Helmholtz solver (semtex ModalMatrixSys + Field::solve, DIRECT).
 //
 // Set-up (once per system, not timed):
-//   k_elem_sc       elemental Helmholtz matrix + static condensation per
-//                   (mode, element class)  [Element::HelmholtzSC]
-//   k_band_assemble deterministic direct-stiffness assembly of the band
-//   band_factor     FP64 banded Cholesky + inverted diagonal blocks (sx_band.hip)
+//   k_elem_sc_lds   elemental Helmholtz matrix + static condensation per
+//                   (mode, element class)  [Element::HelmholtzSC] (N_P > 12: k_elem_sc)
+//   tree_factor     dissection of the condensed system (sx_tree.hip), or
+//   k_band_assemble, band_factor  its banded Cholesky (sx_band.hip)
 // Solve (the timed path, per call):
 //   k_essential     essential BC values into global numbering (k_ess_weak:
 //                   with the essential elements' -(M f + H g) in one launch)
 //   k_condense      -(M f + H g), emap gather, F_b -= hbi hii^-1 F_i
 //   k_assemble      direct-stiffness sum of F_b (+ natural BC integrals)
-//   band_solve      FP64 U^T U x = b, one workgroup per mode (sx_band.hip)
+//   band_solve      the condensed FP64 systems: dissection levels (sx_tree.hip) or
+//                   band sweeps (sx_band.hip)
 //   k_recover       u_i = hii^-1 F_i - (hbi hii^-1)^T u_b, essential insert
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstring>
 #include <vector>
 
@@ -1712,9 +1714,9 @@ extern "C" int sx_msys_layout (sx_msys_t s, int* info, int n)
     sx::set_error ("sx_msys_layout: null system or output");
     return SX_ERR_ARG;
   }
-  const int v[7] = {s->sw_panel, s->sw_D, s->tw, s->m->nband, s->sw_unit, s->last_kernel,
-                    s->last_nr};
-  for (int i = 0; i < n && i < 7; i++) info[i] = v[i];
+  const int v[8] = {s->sw_panel, s->sw_D, s->tw, s->m->nband, s->sw_unit, s->last_kernel,
+                    s->last_nr, s->tree ? (int) std::min<size_t> (tree_ops (s->tree), INT32_MAX) : 0};
+  for (int i = 0; i < n && i < 8; i++) info[i] = v[i];
   return SX_OK;
 }
 

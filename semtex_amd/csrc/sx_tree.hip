@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void k_tree_panel (
 // with s_i = -1 for unknowns already eliminated (i < p0), +1 otherwise: the
 // matrix stays symmetric up to that sign, so only upper tiles are formed.
 // R and W are padded to whole tiles, so every load is unconditional and
-// issued before the products (46 -> 12 us a step at 96 fronts of 370).
+// issued before the products (46 -> 25 us a step at 96 fronts of 370, 17 with upper tiles only).
 __global__ __launch_bounds__(256) void k_tree_update (
     const TreeClass* __restrict__ cls, int cls0, double* F, size_t fs,
     const double* __restrict__ RW, int ldw, int step, int nt)

@@ -84,13 +84,15 @@ class ModalMatrixSys:
         return _lib.load().sx_msys_nsolve(self.handle, mode)
 
     def layout(self):
-        """{"panels", "D", "twisted", "nband", "unit", "kernel", "nr"} of the
-        factor's solve copies and of the last band solve (kernel: 0 none yet,
-        1 panel sweeps, 2 unit-diagonal sweeps, 3 split sweeps; nr:
-        right-hand sides per workgroup)."""
-        info = (C.c_int * 7)()
-        _lib.check(_lib.load().sx_msys_layout(self.handle, info, 7), "sx_msys_layout")
-        keys = ("panels", "D", "twisted", "nband", "unit", "kernel", "nr")
+        """{"panels", "D", "twisted", "nband", "unit", "kernel", "nr",
+        "operators"} of the factor and of the last solve (kernel: 0 none yet,
+        1 panel sweeps, 2 unit-diagonal sweeps, 3 split sweeps -- nr:
+        right-hand sides per workgroup; 4 dissection -- nr: right-hand sides
+        per mode; operators: doubles per mode of the dissection's operators,
+        0 without one)."""
+        info = (C.c_int * 8)()
+        _lib.check(_lib.load().sx_msys_layout(self.handle, info, 8), "sx_msys_layout")
+        keys = ("panels", "D", "twisted", "nband", "unit", "kernel", "nr", "operators")
         return dict(zip(keys, info))
 
     def status(self):
