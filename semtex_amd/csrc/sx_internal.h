@@ -275,6 +275,7 @@ struct sx_msys {
   int use_tree = 0;            //   solves run it
   int held = 0;                //   a batch holds the system (msys_hold)
   sx::TreeSing* sing = nullptr;  // the singular mode's refinement, or null
+  sx::TreeSing* sing_kept = nullptr;  // the same, out of use since a batch holds the system
   double* d_tops = nullptr;    //   operators [nmodes][ops]
   double* d_tb = nullptr;      //   assembled right-hand sides by position [nmodes][nr][nsolve]
   double* d_tv = nullptr;      //   fronts' eliminated parts [nmodes][nr][nsolve]

@@ -1698,6 +1698,7 @@ extern "C" int sx_msys_destroy (sx_msys_t s)
     block_free (s->block, s->block_bytes, s->block_dev);
   }
   tree_sing_free (s->sing);
+  tree_sing_free (s->sing_kept);
   delete s;
   return SX_OK;
 }
@@ -1766,8 +1767,9 @@ namespace sx {
 int msys_hold (sx_msys* s)
 {
   if (s->held) return SX_OK;
-  // (neither refines a singular mode in a batch)
-  tree_sing_free (s->sing);
+  // Neither refines a singular mode in a batch.  The buffers stay until the
+  // system goes: a graph the caller captured of its own solve still uses them
+  s->sing_kept = s->sing;
   s->sing = nullptr;
   if (!s->use_tree) { s->held = 1; return SX_OK; }
   const sx_mesh* m = s->m;

@@ -132,3 +132,37 @@ def test_element_holding_a_node_twice_keeps_the_band(torch_cuda, oracle):
     assert kernel != 4
     uo = oracle.solve_modes(m, 1.0, 1.0, F[:, :m.nel * m.npnp], lines)[0]
     assert np.linalg.norm(ug[0] - uo) < TOL * np.linalg.norm(uo)
+
+
+def test_captured_singular_solve_outlives_a_batch(torch_cuda):
+    """A graph captured of a pure Neumann solve replays to the same solution
+    after a batch has taken its system."""
+    from semtex_amd.mesh import rect_mesh
+    from semtex_amd.solver import Batch, Field, GpuMesh, ModalMatrixSys
+    torch = torch_cuda
+    print("case: captured singular solve, then a batch", flush=True)
+    m = rect_mesh(4, 3, 6, 0.0, 2 * np.pi, -1.0, 1.0, bc=("N", "N", "N", "N"), periodic_x=True)
+    F = np.zeros((1, m.plane_size))
+    F[0, :m.nel * m.npnp] = np.sin(m.x.ravel()) * m.y.ravel()
+    gm = GpuMesh(m)
+    M = ModalMatrixSys(0.0, 1.0, 0, 1, gm)
+    u, v = Field(gm, 1), Field(gm, 1)
+    src = torch.tensor(F, device="cuda")
+    f = src.clone()
+    u.solve(f, M)
+    torch.cuda.synchronize()
+    expect = u.data.clone()
+    f.copy_(src)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        u.solve(f, M)
+    B = Batch([(M, v, src)])
+    for _ in range(3):
+        f.copy_(src)
+        u.data.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.linalg.norm(u.data - expect) <= TOL * torch.linalg.norm(expect)
+        B.run()
+        torch.cuda.synchronize()
