@@ -2469,15 +2469,16 @@ static int band_factor_twisted (sx_msys* s, const std::vector<int>& tw, hipStrea
   }
   SX_HIP (hipMalloc (&s->d_tw, sizeof (int) * tw.size ()));
   SX_HIP (hipMemcpy (s->d_tw, tw.data (), sizeof (int) * tw.size (), hipMemcpyHostToDevice));
-  int* d_aux = nullptr;
-  SX_HIP (hipMalloc (&d_aux, sizeof (int) * aux.size ()));
+  DevTmp taux, tR, tV;
+  SX_HIP (hipMalloc (&taux.p, sizeof (int) * aux.size ()));
+  int* d_aux = (int*) taux.p;
   SX_HIP (hipMemcpy (d_aux, aux.data (), sizeof (int) * aux.size (), hipMemcpyHostToDevice));
   const int *d_ntop = d_aux, *d_nbot = d_aux + nm, *d_nelim = d_aux + 2 * nm;
   const size_t rstride = (size_t) nbbm * PB * ld;
-  double *R = nullptr, *V = nullptr;
   const size_t vstride = std::max (rstride, s->band_stride);
-  SX_HIP (hipMalloc (&R, sizeof (double) * nm * rstride));
-  SX_HIP (hipMalloc (&V, sizeof (double) * nm * vstride));
+  SX_HIP (hipMalloc (&tR.p, sizeof (double) * nm * rstride));
+  SX_HIP (hipMalloc (&tV.p, sizeof (double) * nm * vstride));
+  double *R = (double*) tR.p, *V = (double*) tV.p;
   SX_HIP (hipMemsetAsync (V, 0, sizeof (double) * nm * vstride, st));
   hipLaunchKernelGGL (k_twist_rbuild, dim3 ((unsigned) ((rstride + 255) / 256), nm),
                       dim3 (256), 0, st, s->d_bandU, s->band_stride, R, rstride, ld, s->d_tw);
@@ -2508,9 +2509,6 @@ static int band_factor_twisted (sx_msys* s, const std::vector<int>& tw, hipStrea
   SX_HIP (hipMalloc (&s->d_rhsb, sizeof (double) * nb_rhs));
   SX_HIP (hipMemsetAsync (s->d_rhsb, 0, sizeof (double) * nb_rhs, st));
   SX_HIP (hipStreamSynchronize (st));
-  (void) hipFree (R);
-  (void) hipFree (V);
-  (void) hipFree (d_aux);
   return SX_OK;
 }
 
@@ -2529,9 +2527,11 @@ int band_factor (sx_msys* s, hipStream_t st, int* d_status)
     s->sw_unit = use_unit (panel_D (ld));
   }
   const bool rev = !panels || reversed_panels (s);
+  DevTmp tV;
   double* V = nullptr;
   if (rev) {
-    SX_HIP (hipMalloc (&V, sizeof (double) * s->nmodes * s->band_stride));
+    SX_HIP (hipMalloc (&tV.p, sizeof (double) * s->nmodes * s->band_stride));
+    V = (double*) tV.p;
     SX_HIP (hipMemsetAsync (V, 0, sizeof (double) * s->nmodes * s->band_stride, st));
     hipLaunchKernelGGL (k_band_reverse,
                         dim3 ((unsigned) ((s->band_stride + 255) / 256), s->nmodes),
@@ -2563,7 +2563,6 @@ int band_factor (sx_msys* s, hipStream_t st, int* d_status)
     }
     SX_HIP (hipGetLastError ());
     SX_HIP (hipStreamSynchronize (st));
-    (void) hipFree (V);
     return SX_OK;
   }
   s->sw_panel = 0;
@@ -2586,8 +2585,20 @@ int band_factor (sx_msys* s, hipStream_t st, int* d_status)
                       s->d_swR, s->band_stride, s->sw_stride, ld, B, s->d_nsolve);
   SX_HIP (hipGetLastError ());
   SX_HIP (hipStreamSynchronize (st));
-  (void) hipFree (V);
   return SX_OK;
+}
+
+void band_drop (sx_msys* s)
+{
+  for (void* p : {(void*) s->d_bandU, (void*) s->d_swF, (void*) s->d_swR, (void*) s->d_tw,
+                  (void*) s->d_rhsb, (void*) s->d_xch, (void*) s->d_xep})
+    if (p) (void) hipFree (p);
+  s->d_bandU = s->d_swF = s->d_swR = s->d_rhsb = nullptr;
+  s->d_tw = nullptr;
+  s->d_xch = nullptr;
+  s->d_xep = nullptr;
+  s->sw_block = s->sw_panel = s->sw_D = s->sw_unit = s->tw = s->tw_S = s->nmaxb = 0;
+  s->sw_stride = s->tw_boff = 0;
 }
 
 static int band_sweeps (const sx_msys* s, int nr, hipStream_t st, int moves)

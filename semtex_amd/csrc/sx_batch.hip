@@ -265,11 +265,16 @@ extern "C" int sx_batch_create (int n, const sx_msys_t* systems, const int* nz,
       return SX_ERR_ARG;
     }
   *out = nullptr;
-  for (int i = 0; i < n; i++)
-    if (int rc = msys_hold (systems[i])) return rc;
+  std::vector<Held> held (n);
   sx_batch* b = new sx_batch;
   b->n = n;
-  auto fail = [&] (int r) { sx_batch_destroy (b); return r; };
+  auto fail = [&] (int r) {            // (the graph goes before what it uses)
+    sx_batch_destroy (b);
+    for (Held& h : held) msys_release (h);
+    return r;
+  };
+  for (int i = 0; i < n; i++)
+    if (int rc = msys_hold (systems[i], held[i])) return fail (rc);
   if (hipStreamCreate (&b->cap) != hipSuccess) return fail (hip_fail (hipErrorUnknown, "hipStreamCreate"));
   // lanes: 4, as many as the hardware queues a process gets by default
   // (measured: 4 lanes 2.9 ms FP64 / 7.4 ms mixed per 64-problem batch, 8
@@ -301,6 +306,7 @@ extern "C" int sx_batch_create (int n, const sx_msys_t* systems, const int* nz,
     const int rc = fused_record (b);
     if (rc == SX_OK) {
       b->fused = 1;
+      for (Held& h : held) msys_keep (h);
       *out = b;
       return SX_OK;
     }
@@ -335,6 +341,7 @@ extern "C" int sx_batch_create (int n, const sx_msys_t* systems, const int* nz,
   if (ec != hipSuccess) return fail (hip_fail (ec, "hipStreamEndCapture"));
   hipError_t ei = hipGraphInstantiate (&b->exec, b->graph, nullptr, nullptr, 0);
   if (ei != hipSuccess) return fail (hip_fail (ei, "hipGraphInstantiate"));
+  for (Held& h : held) msys_keep (h);
   *out = b;
   return SX_OK;
 }

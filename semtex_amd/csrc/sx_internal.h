@@ -74,14 +74,17 @@ struct TreeSing;
 int    tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always = false, int share = 1);
 void   tree_free (TreeDev* t);
 void   tree_sing_free (TreeSing* g);
-int    tree_workspace (sx_msys* s, int nr, bool always = false);
+struct Grow;
+int    tree_grow (Grow& G, sx_msys* s, TreeDev* t, int nr);
 size_t tree_ops (const TreeDev* t);                 // doubles per mode of d_tops
 size_t tree_slots (const TreeDev* t);               // and per right-hand side of d_tc
 size_t tree_scratch (const TreeDev* t, int nm);     // doubles
 int    tree_factor (sx_msys* s, const double* Sel, double* buf, hipStream_t st, int* d_status);
 int    tree_solve (const sx_msys* s, int nr, hipStream_t st);
-// The system's dissection cut again for a batch (many solves side by side).
-int    tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_status);
+// The system's dissection cut again for a batch (many solves side by side):
+// the plan, its operators and its workspace; the system is not changed.
+struct Held;
+int    tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_status, Held& h);
 // A singular mode's refinement: its set-up (s->sing), and around a band
 // solve the right-hand sides kept before and the correction after.
 int    tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_status);
@@ -92,9 +95,31 @@ int    sing_refine (const sx_msys* s, int nr, hipStream_t st);
 // factor is built here), as systems of a batch always did, unless
 // SX_BAND_SPLIT=0 asks for no split sweeps, when they run what the batch
 // records.
-int    msys_hold (sx_msys* s);
+// h: what the system had before; msys_keep gives that up once the batch is
+// made, msys_release puts it back when the batch fails.
+int    msys_hold (sx_msys* s, Held& h);
+void   msys_keep (Held& h);
+void   msys_release (Held& h);
 // Frees a device array of the system unless it lies in its block.
 void   msys_free (sx_msys* s, void* p);
+// A device temporary, freed where its scope ends.
+struct DevTmp {
+  void* p = nullptr;
+  DevTmp () = default;
+  DevTmp (const DevTmp&) = delete;
+  ~DevTmp () { if (p) (void) hipFree (p); }
+};
+// Device arrays of a system replaced together: all the new ones are allocated
+// and cleared before an old one is given up, so a failure changes nothing.
+struct Grow {
+  struct Item { double **at, *p; };
+  std::vector<Item> items;
+  int add (double** at, size_t doubles);
+  int install (sx_msys* s);
+  Grow () = default;
+  Grow (const Grow&) = delete;
+  ~Grow ();
+};
 // Banded FP64 Cholesky of every mode's band, the offset-major sweep copies
 // of the factor and of its reversal (with inverted diagonal blocks), and
 // the two-sweep solve of the right-hand sides in d_rhs ([mode][2][nmax])
@@ -102,6 +127,7 @@ void   msys_free (sx_msys* s, void* p);
 int    band_block (int nband);
 size_t band_sweep_bytes_per_mode (int nmax, int nband);
 int    band_factor (sx_msys* s, hipStream_t st, int* d_status);
+void   band_drop (sx_msys* s);       // gives the factor (or a part of one) up
 // nr RHS per mode; moves (twisted systems): 1 gather the bottom piece's
 // right-hand side, 2 scatter its solution (3: both; 0 when the caller's
 // assembly and recovery address the bottom piece themselves)
@@ -286,6 +312,13 @@ struct sx_msys {
   double* d_work = nullptr;    // mixed-precision / PCG workspace
   double* d_pc = nullptr;      // SX_JACPCG: [nmodes][npts] inverse assembled diagonal
   size_t work_doubles = 0;
+};
+// What msys_hold replaces of a system (s null: nothing)
+struct sx::Held {
+  sx_msys* s = nullptr;
+  sx::TreeDev* tree = nullptr;         // null: the plan stayed
+  double *ops = nullptr, *tb = nullptr, *tv = nullptr, *tc = nullptr;
+  int use_tree = 0;
 };
 // where the assembly writes a solve's right-hand sides: [mode][nr][ld], node
 // g at perm[g] (perm null: at g).  The dissection solve reads them by

@@ -19,6 +19,9 @@ void set_error (const std::string& msg) { g_err = msg; }
 int hip_fail (hipError_t e, const char* what)
 {
   set_error (std::string ("HIP error ") + hipGetErrorString (e) + " in " + what);
+  // the runtime keeps the error for hipGetLastError as well: reported here, it
+  // must not fail the next call's launch check
+  (void) hipGetLastError ();
   return SX_ERR_HIP;
 }
 

@@ -1764,40 +1764,102 @@ static int band_build (sx_msys* s, const double* d_S, hipStream_t st, int* d_sta
 
 namespace sx {
 
-int msys_hold (sx_msys* s)
+int Grow::add (double** at, size_t doubles)
 {
+  double* p = nullptr;
+  const size_t bytes = sizeof (double) * std::max<size_t> (doubles, 1);
+  SX_HIP (hipMalloc (&p, bytes));
+  items.push_back ({at, p});
+  SX_HIP (hipMemset (p, 0, bytes));
+  return SX_OK;
+}
+
+int Grow::install (sx_msys* s)
+{
+  SX_HIP (hipStreamSynchronize (nullptr));      // the clears
+  for (Item& i : items) {
+    msys_free (s, *i.at);
+    *i.at = i.p;
+  }
+  items.clear ();
+  return SX_OK;
+}
+
+Grow::~Grow ()
+{
+  for (Item& i : items) (void) hipFree (i.p);
+}
+
+int msys_hold (sx_msys* s, Held& h)
+{
+  h = Held {};
   if (s->held) return SX_OK;
-  // Neither refines a singular mode in a batch.  The buffers stay until the
-  // system goes: a graph the caller captured of its own solve still uses them
+  Held was;
+  was.s = s;
+  was.use_tree = s->use_tree;
+  if (s->use_tree) {
+    const sx_mesh* m = s->m;
+    const int next = m->next, nint = m->nint, npnp = m->npnp;
+    const size_t nmc = (size_t) s->nmodes * m->nclass;
+    const size_t nws = nmc * ((size_t) npnp * npnp + (size_t) nint * nint), nS = nmc * next * next,
+                 nB = nmc * next * nint, nH = nmc * nint * nint;
+    // the condensed element matrices again (k_elem_sc forms them with the
+    // element operators, which the system holds already)
+    DevTmp tbuf, tstat;
+    SX_HIP (hipMalloc (&tbuf.p, sizeof (double) * (nws + nS + nB + nH + 1)));
+    SX_HIP (hipMalloc (&tstat.p, sizeof (int) * (s->nmodes + 1)));
+    double* buf = (double*) tbuf.p;
+    int* d_status = (int*) tstat.p;
+    SX_HIP (hipMemset (d_status, 0, sizeof (int) * (s->nmodes + 1)));
+    int rc = elem_sc (m, s->nmodes, s->lambda2, s->d_betak2, buf, buf + nws, buf + nws + nS,
+                      buf + nws + nS + nB, d_status + s->nmodes, nullptr);
+    Held now;
+    if (!rc) rc = tree_for_batch (s, buf + nws, nullptr, d_status, now);
+    if (!rc && (rc = band_build (s, buf + nws, nullptr, d_status))) band_drop (s);
+    if (rc) {
+      for (double* p : {now.ops, now.tb, now.tv, now.tc}) if (p) (void) hipFree (p);
+      return rc;
+    }
+    if (now.tree) {
+      was.tree = s->tree;
+      was.ops = s->d_tops; was.tb = s->d_tb; was.tv = s->d_tv; was.tc = s->d_tc;
+      s->tree = now.tree;
+      s->d_tops = now.ops; s->d_tb = now.tb; s->d_tv = now.tv; s->d_tc = now.tc;
+    }
+  }
+  // Neither the batch nor the system's own solves refine a singular mode from
+  // here on.  The buffers stay until the system goes: a graph the caller
+  // captured of its own solve still uses them
   s->sing_kept = s->sing;
   s->sing = nullptr;
-  if (!s->use_tree) { s->held = 1; return SX_OK; }
-  const sx_mesh* m = s->m;
-  const int next = m->next, nint = m->nint, npnp = m->npnp;
-  const size_t nmc = (size_t) s->nmodes * m->nclass;
-  const size_t nws = nmc * ((size_t) npnp * npnp + (size_t) nint * nint), nS = nmc * next * next,
-               nB = nmc * next * nint, nH = nmc * nint * nint;
-  // the condensed element matrices again (k_elem_sc forms them with the
-  // element operators, which the system holds already)
-  double* buf = nullptr;
-  int* d_status = nullptr;
-  SX_HIP (hipMalloc (&buf, sizeof (double) * (nws + nS + nB + nH + 1)));
-  int rc = SX_OK;
-  if (hipMalloc (&d_status, sizeof (int) * (s->nmodes + 1)) != hipSuccess ||
-      hipMemset (d_status, 0, sizeof (int) * (s->nmodes + 1)) != hipSuccess) {
-    rc = hip_fail (hipErrorOutOfMemory, "msys_use_band");
-  } else {
-    rc = elem_sc (m, s->nmodes, s->lambda2, s->d_betak2, buf, buf + nws, buf + nws + nS,
-                  buf + nws + nS + nB, d_status + s->nmodes, nullptr);
-    if (!rc) rc = tree_for_batch (s, buf + nws, nullptr, d_status);
-    if (!rc) rc = band_build (s, buf + nws, nullptr, d_status);
-  }
-  (void) hipFree (buf);
-  (void) hipFree (d_status);
-  if (rc) return rc;
   s->use_tree = 0;
   s->held = 1;
+  h = was;
   return SX_OK;
+}
+
+void msys_keep (Held& h)
+{
+  if (h.s && h.tree)
+    for (double* p : {h.ops, h.tb, h.tv, h.tc}) msys_free (h.s, p);
+  h = Held {};
+}
+
+void msys_release (Held& h)
+{
+  sx_msys* s = h.s;
+  if (!s) return;
+  if (h.tree) {
+    for (double* p : {s->d_tops, s->d_tb, s->d_tv, s->d_tc}) msys_free (s, p);
+    s->tree = h.tree;
+    s->d_tops = h.ops; s->d_tb = h.tb; s->d_tv = h.tv; s->d_tc = h.tc;
+  }
+  if (h.use_tree) band_drop (s);
+  s->sing = s->sing_kept;
+  s->sing_kept = nullptr;
+  s->use_tree = h.use_tree;
+  s->held = 0;
+  h = Held {};
 }
 
 }  // namespace sx
@@ -2285,26 +2347,16 @@ int msys_reserve_rhs (sx_msys* s, int nr)
                "sweeps with at most 6 off-diagonal blocks (band offsets kd <= 447)");
     return SX_ERR_LIMIT;
   }
-  double *r = nullptr, *g = nullptr;
-  if (s->tw) {
-    double* rb = nullptr;
-    const size_t nb = sizeof (double) * s->nmodes * nr * s->nmaxb;
-    SX_HIP (hipMalloc (&rb, nb));
-    SX_HIP (hipMemset (rb, 0, nb));
-    (void) hipFree (s->d_rhsb);
-    s->d_rhsb = rb;
-  }
-  SX_HIP (hipMalloc (&r, sizeof (double) * s->nmodes * nr * std::max (s->nmax, 1)));
-  SX_HIP (hipMalloc (&g, sizeof (double) * (nr / 2) * 2 * s->nmodes * s->m->nglobal));
-  SX_HIP (hipMemset (r, 0, sizeof (double) * s->nmodes * nr * std::max (s->nmax, 1)));
-  SX_HIP (hipMemset (g, 0, sizeof (double) * (nr / 2) * 2 * s->nmodes * s->m->nglobal));
-  msys_free (s, s->d_rhs);
-  msys_free (s, s->d_G);
-  s->d_rhs = r;
-  s->d_G = g;
-  const int rc = tree_workspace (s, nr);
+  const size_t nm = s->nmodes;
+  Grow G;
+  int rc;
+  if ((rc = G.add (&s->d_rhs, nm * nr * std::max (s->nmax, 1))) ||
+      (rc = G.add (&s->d_G, nr * nm * s->m->nglobal)) ||
+      (s->tw && (rc = G.add (&s->d_rhsb, nm * nr * s->nmaxb))) ||
+      (rc = tree_grow (G, s, s->tree, nr)) || (rc = G.install (s)))
+    return rc;
   s->rhs_cap = nr;
-  return rc;
+  return SX_OK;
 }
 
 int condense32_tiled (const sx_msys* s, int nz, int stride, const double* X, double* Fp,

@@ -793,34 +793,22 @@ void tree_sing_free (TreeSing* g)
   delete g;
 }
 
-// Workspace of a solve with nr right-hand sides per mode, grown from the one
-// the system was created with (2)
-int tree_workspace (sx_msys* s, int nr, bool always)
+// The workspace of solves with nr right-hand sides per mode by plan t (null:
+// none) and of the singular mode's refinement, added to what G replaces
+int tree_grow (Grow& G, sx_msys* s, TreeDev* t, int nr)
 {
-  auto grow = [&] (double** p, size_t n) {
-    double* q = nullptr;
-    SX_HIP (hipMalloc (&q, sizeof (double) * std::max<size_t> (n, 1)));
-    SX_HIP (hipMemset (q, 0, sizeof (double) * n));
-    msys_free (s, *p);
-    *p = q;
-    return (int) SX_OK;
-  };
   const size_t n = (size_t) s->nmodes * nr;
   int rc;
-  if (s->tree && (always || nr > s->rhs_cap)) {
-    const TreePlan& P = s->tree->P;
-    if ((rc = grow (&s->d_tb, n * P.nsolve)) || (rc = grow (&s->d_tv, n * P.nsolve)) ||
-        (rc = grow (&s->d_tc, n * P.slots)))
-      return rc;
-  }
+  if (t && ((rc = G.add (&s->d_tb, n * t->P.nsolve)) || (rc = G.add (&s->d_tv, n * t->P.nsolve)) ||
+            (rc = G.add (&s->d_tc, n * t->P.slots))))
+    return rc;
   if (TreeSing* g = s->sing) {
     const TreePlan& P = g->t->P;
-    if ((rc = grow (&g->b, (size_t) nr * s->nmax)) || (rc = grow (&g->dx, (size_t) nr * s->nmax)) ||
-        (rc = grow (&g->v, (size_t) nr * P.nsolve)) || (rc = grow (&g->cb, nr * P.slots)) ||
-        (rc = grow (&g->r, (size_t) nr * P.nsolve)))
+    if ((rc = G.add (&g->b, (size_t) nr * s->nmax)) || (rc = G.add (&g->dx, (size_t) nr * s->nmax)) ||
+        (rc = G.add (&g->v, (size_t) nr * P.nsolve)) || (rc = G.add (&g->cb, nr * P.slots)) ||
+        (rc = G.add (&g->r, (size_t) nr * P.nsolve)))
       return rc;
   }
-  SX_HIP (hipStreamSynchronize (nullptr));
   return SX_OK;
 }
 
@@ -831,7 +819,7 @@ int tree_factor (sx_msys* s, const double* Sel, double* buf, hipStream_t st, int
   return factor (s->tree, s->m, s->nmodes, s->d_nsolve, Sel, s->d_tops, buf, st, d_status);
 }
 
-int tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_status)
+int tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_status, Held& h)
 {
   // (64 uneven problems: 309 us at 4, 318 at 8, 359 at 32, 360 with the
   // systems' own cuts)
@@ -840,21 +828,25 @@ int tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_status
   if (int rc = tree_prepare (s->m, s->nmodes, &t, true, std::max (1, BATCH_SHARE / s->nmodes)))
     return rc;
   if (!t || t == s->tree) return SX_OK;
-  double *ops = nullptr, *buf = nullptr;
-  SX_HIP (hipMalloc (&ops, sizeof (double) * std::max<size_t> (t->P.ops * s->nmodes, 2)));
-  int rc = hipMalloc (&buf, sizeof (double) * tree_scratch (t, s->nmodes)) == hipSuccess
-               ? factor (t, s->m, s->nmodes, s->d_nsolve, Sel, ops, buf, st, d_status)
-               : hip_fail (hipErrorOutOfMemory, "tree_for_batch");
-  if (rc == SX_OK) rc = hipStreamSynchronize (st) == hipSuccess ? SX_OK : SX_ERR_HIP;
-  (void) hipFree (buf);
-  if (rc) {
-    (void) hipFree (ops);
+  const size_t n = (size_t) s->nmodes * s->rhs_cap;
+  Held now;
+  Grow G;
+  DevTmp buf;
+  int rc;
+  if ((rc = G.add (&now.ops, std::max<size_t> (t->P.ops * s->nmodes, 2))) ||
+      (rc = G.add (&now.tb, n * t->P.nsolve)) || (rc = G.add (&now.tv, n * t->P.nsolve)) ||
+      (rc = G.add (&now.tc, n * t->P.slots)))
     return rc;
-  }
-  msys_free (s, s->d_tops);
-  s->d_tops = ops;
-  s->tree = t;
-  return tree_workspace (s, s->rhs_cap, true);
+  SX_HIP (hipMalloc (&buf.p, sizeof (double) * tree_scratch (t, s->nmodes)));
+  // (the arrays are now's once installed)
+  if ((rc = factor (t, s->m, s->nmodes, s->d_nsolve, Sel, G.items[0].p, (double*) buf.p, st,
+                    d_status)))
+    return rc;
+  SX_HIP (hipStreamSynchronize (st));
+  if ((rc = G.install (s))) return rc;
+  now.tree = t;
+  h = now;
+  return SX_OK;
 }
 
 int tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_status)
@@ -879,7 +871,9 @@ int tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_statu
     hipLaunchKernelGGL (k_tree_entries, dim3 ((m->npairs + 255) / 256), dim3 (256), 0, st,
                         m->npairs, m->d_pptr, m->d_psrc, S, g->val);
     SX_HIP (hipGetLastError ());
-    return tree_workspace (s, 2);      // at most mode 0 has a zero constant
+    Grow G;
+    int rc = tree_grow (G, s, nullptr, 2);
+    return rc ? rc : G.install (s);    // at most mode 0 has a zero constant
   }
   return SX_OK;
 }

@@ -1,0 +1,161 @@
+"""Device allocations that fail, on the CPU: the library's host code runs on
+tests/hip_stub.cpp (host memory for device memory, launches counted and not
+run), which makes any chosen allocation fail.  A call that fails for memory
+must leave the system it was given as it was -- the same plan, operators,
+refinement and reserved right-hand sides -- hold no memory it did not hold
+before, and succeed when it is called again with memory there."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SRC = os.path.join(ROOT, "tests", "hip_stub.cpp")
+STUB = os.path.join(ROOT, "tests", "_bin", "libhip_stub.so")
+
+PRELUDE = textwrap.dedent("""
+    import ctypes as C, os, sys
+    import numpy as np
+    from semtex_amd import _lib
+    from semtex_amd.mesh import rect_mesh
+    from semtex_amd import solver
+    solver._stream = lambda: None
+    from semtex_amd.solver import GpuMesh, ModalMatrixSys
+    L = _lib.load()
+    S = C.CDLL(os.environ["LD_PRELOAD"])
+    S.stub_bytes.restype = C.c_size_t
+    S.stub_limit.argtypes = [C.c_size_t]
+    for f in ("stub_allocs", "stub_live", "stub_launches", "stub_bad_pointers"): getattr(S, f).restype = C.c_long
+    S.stub_fail.argtypes = [C.c_long, C.c_long]
+    S.stub_device.argtypes = [C.c_long]
+    launches = lambda name: S.stub_launches(name.encode())
+
+    class Buf:                       # a device array
+        def __init__(self, n):
+            self.p = C.c_void_p()
+            assert S.hipMalloc(C.byref(self.p), C.c_size_t(8 * n)) == 0
+            C.memset(self.p, 0, 8 * n)
+        def free(self): S.hipFree(self.p)
+
+    def reserve(M, nr): return L._ZN2sx16msys_reserve_rhsEP7sx_msysi(M.handle, nr)
+    def solve_nr(M, nr): return L._ZN2sx10band_solveEPK7sx_msysiP12ihipStream_ti(M.handle, nr, None, 3)
+
+    class RawBatch:
+        def __init__(self, Ms, nz=1):
+            n = len(Ms)
+            self.bufs = [[Buf(nz * M.gmesh.plane_size) for _ in range(3)] for M in Ms]
+            pp = lambda j: (C.c_void_p * n)(*[b[j].p for b in self.bufs])
+            self.args = (n, (C.c_void_p * n)(*[M.handle for M in Ms]), (C.c_int * n)(*[nz] * n),
+                         (C.c_int * n)(*[M.gmesh.plane_size for M in Ms]), pp(0), pp(1), pp(2), None, 1)
+            self.h = None
+        def create(self):
+            h = C.c_void_p()
+            rc = L.sx_batch_create(*self.args, C.byref(h))
+            self.h = h if rc == 0 else None
+            return rc
+        def destroy(self):
+            if self.h: L.sx_batch_destroy(self.h)
+            self.h = None
+        def free(self):
+            for b in self.bufs:
+                for x in b: x.free()
+
+    def own_solve(M, nz=1):
+        b = [Buf(nz * M.gmesh.plane_size) for _ in range(2)]
+        rc = L.sx_field_solve(M.handle, nz, M.gmesh.plane_size, b[0].p, b[1].p, None, None)
+        for x in b: x.free()
+        return rc
+""")
+
+
+def run(body, **env):
+    if not os.path.exists(STUB) or os.path.getmtime(STUB) < os.path.getmtime(SRC):
+        os.makedirs(os.path.dirname(STUB), exist_ok=True)
+        subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__",
+                        "-I/opt/rocm/include", SRC, "-o", STUB + ".tmp"], check=True)
+        os.replace(STUB + ".tmp", STUB)
+    e = {k: v for k, v in os.environ.items() if not k.startswith("SX_")}
+    e.update(LD_PRELOAD=STUB, PYTHONPATH=ROOT, **env)
+    r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body)], env=e, cwd=ROOT,
+                       capture_output=True, text=True, timeout=240)
+    assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout[-2000:] + r.stderr[-4000:]
+
+
+def test_failed_reservation_keeps_the_reserved_count():
+    """msys_reserve_rhs: whichever allocation fails, a solve of more
+    right-hand sides than the arrays hold is refused afterwards."""
+    run("""
+    m = rect_mesh(12, 10, 6, 0.0, 6.0, -1.0, 1.0, bc=("D", "N", "D", "N"), periodic_x=True)
+    for bc in (("D", "N", "D", "N"), ("N", "N", "N", "N")):       # the second with a singular mode
+        m = rect_mesh(12, 10, 6, 0.0, 6.0, -1.0, 1.0, bc=bc, periodic_x=True)
+        M = ModalMatrixSys(0.0, 1.0, 0, 4, GpuMesh(m))
+        assert M.layout()["operators"] > 0
+        k = 0
+        while True:
+            held = S.stub_bytes()
+            S.stub_fail(k, 1)
+            rc = reserve(M, 6)
+            failed = S.stub_allocs() > k
+            S.stub_fail(-1, 0)
+            if not failed: break
+            assert rc == _lib.SX_ERR_HIP, rc
+            assert solve_nr(M, 6) == _lib.SX_ERR_ARG, k
+            assert solve_nr(M, 2) == 0
+            assert S.stub_bytes() == held, (k, S.stub_bytes(), held)
+            k += 1
+        assert rc == 0 and k >= 5, (rc, k)
+        assert solve_nr(M, 6) == 0
+    assert S.stub_bad_pointers() == 0
+    print("ok")
+    """)
+
+
+@pytest.mark.parametrize("bc", ["DNDN", "NNNN"])
+def test_failed_batch_leaves_its_systems_as_they_were(bc):
+    """sx_batch_create over two systems: whichever allocation fails, both keep
+    their own plan, operators and refinement and solve as before."""
+    run(f"""
+    ms = [rect_mesh(nx, ny, 6, 0.0, 6.0, -1.0, 1.0, bc=tuple("{bc}"), periodic_x=True)
+          for nx, ny in ((16, 12), (9, 7))]
+    Ms = [ModalMatrixSys(0.0, 1.0, 0, 1, GpuMesh(m)) for m in ms]
+    B = RawBatch(Ms)
+    keys = ("panels", "D", "twisted", "unit", "operators")
+    def state():
+        out = []
+        for M in Ms:
+            a, r = launches("k_tree_level"), launches("k_tree_residual")
+            assert own_solve(M) == 0
+            out.append((launches("k_tree_level") - a, launches("k_tree_residual") - r,
+                        [M.layout()[k] for k in keys], M.layout()["kernel"]))
+        return out
+    was = state()
+    # (plans and row lists stay with their meshes: made by a batch that works)
+    Ms2 = [ModalMatrixSys(0.0, 1.0, 0, 1, M.gmesh) for M in Ms]
+    B2 = RawBatch(Ms2)
+    S.stub_fail(0, 0); assert B2.create() == 0
+    total = S.stub_allocs()
+    B2.destroy(); B2.free()
+    del Ms2
+    assert [w[2][4] > 0 for w in was] == [True, True] and total > 4
+    assert all(w[1] == ("{bc}" == "NNNN") for w in was)
+    k = 0
+    while True:
+        held = S.stub_bytes()
+        S.stub_fail(k, 1)
+        rc = B.create()
+        failed = S.stub_allocs() > k
+        S.stub_fail(-1, 0)
+        if not failed: break
+        assert rc == _lib.SX_ERR_HIP, (k, rc, L.sx_last_error())
+        assert S.stub_bytes() == held, (k, S.stub_bytes(), held)
+        assert state() == was, (k, state(), was)
+        k += 1
+    assert rc == 0 and k > 4, (rc, k)
+    B.destroy(); B.free()
+    del Ms
+    assert S.stub_live() == 0, S.stub_live()
+    assert S.stub_bad_pointers() == 0
+    print("ok")
+    """)
