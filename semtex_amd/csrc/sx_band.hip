@@ -2716,13 +2716,20 @@ static int band_sweeps (const sx_msys* s, int nr, hipStream_t st, int moves)
   return SX_ERR_LIMIT;
 }
 
-int band_solve (const sx_msys* s, int nr, hipStream_t st, int moves)
+int band_solve (const sx_msys* s, bool tree, int nr, hipStream_t st, int moves)
 {
-  if (by_tree (s)) return tree_solve (s, nr, st);
+  if (tree) return tree_solve (s, nr, st);
   if (!s->sing) return band_sweeps (s, nr, st, moves);
   int rc;
   if ((rc = sing_keep (s, nr, st)) || (rc = band_sweeps (s, nr, st, 3))) return rc;
   return sing_refine (s, nr, st);
+}
+
+bool band_splits (const sx_msys* s)
+{
+  std::vector<int> tw;
+  const int ld = s->m->nband;
+  return use_panels (ld, s->nmax) && use_unit (panel_D (ld)) && twist_split (s, tw);
 }
 
 // ---------------------------------------------------------------------------
@@ -2807,9 +2814,18 @@ int plan_sweep (BatchPlan& P, const sx_msys* s, int G, int stage)
 // The right-hand sides per sweep workgroup: P.tune when it divides nr and
 // the kernel takes it, else band_solve's default (the fewest that keep one
 // workgroup per CU, at most 2 for the unit-diagonal sweeps).
+static int plan_band_sweeps (BatchPlan& P, const sx_msys* s, int nr);
 int plan_band_solve (BatchPlan& P, const sx_msys* s, int nr)
 {
   if (!s->sw_panel || nr != 2) return SX_ERR_LIMIT;
+  if (!s->sing) return plan_band_sweeps (P, s, nr);
+  int rc;
+  if ((rc = plan_sing_keep (P, s)) || (rc = plan_band_sweeps (P, s, nr))) return rc;
+  return plan_sing_refine (P, s);
+}
+
+static int plan_band_sweeps (BatchPlan& P, const sx_msys* s, int nr)
+{
   const int pieces = s->tw ? 2 : 1, slots = (s->nmodes + 7) / 8 * 8 * pieces;
   int per = nr;
   for (int c : {1, 2})

@@ -90,11 +90,8 @@ int    tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_sta
 int    tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_status);
 int    sing_keep (const sx_msys* s, int nr, hipStream_t st);
 int    sing_refine (const sx_msys* s, int nr, hipStream_t st);
-// A system taken into a batch (sx_solver.hip): the batch records the
-// dissection; the system's own solves run band sweeps from then on (their
-// factor is built here), as systems of a batch always did, unless
-// SX_BAND_SPLIT=0 asks for no split sweeps, when they run what the batch
-// records.
+// A system taken into a batch (sx_solver.hip): its dissection is cut again
+// for many solves side by side, which the batch records.
 // h: what the system had before; msys_keep gives that up once the batch is
 // made, msys_release puts it back when the batch fails.
 int    msys_hold (sx_msys* s, Held& h);
@@ -131,7 +128,8 @@ void   band_drop (sx_msys* s);       // gives the factor (or a part of one) up
 // nr RHS per mode; moves (twisted systems): 1 gather the bottom piece's
 // right-hand side, 2 scatter its solution (3: both; 0 when the caller's
 // assembly and recovery address the bottom piece themselves)
-int    band_solve (const sx_msys* s, int nr, hipStream_t st, int moves = 3);
+int    band_solve (const sx_msys* s, bool tree, int nr, hipStream_t st, int moves = 3);
+bool   band_splits (const sx_msys* s);   // the band layout would have split sweeps
 // per-mode split of a twisted system (d_tw): TW ints per mode
 constexpr int TW = 8;
 enum { TW_NBT = 0, TW_NBB, TW_PAD, TW_M, TW_NTOP, TW_NBOT, TW_N };
@@ -298,10 +296,10 @@ struct sx_msys {
   size_t block_bytes = 0;
   int block_dev = 0;
   sx::TreeDev* tree = nullptr; // dissection solve: the mesh's plan, null: band only
-  int use_tree = 0;            //   solves run it
   int held = 0;                //   a batch holds the system (msys_hold)
+  int own_band = 0;            //   and the band factor of its own solves: 1 built, -1 not
+                               //   wanted or failed, 0 not asked for yet (by_tree)
   sx::TreeSing* sing = nullptr;  // the singular mode's refinement, or null
-  sx::TreeSing* sing_kept = nullptr;  // the same, out of use since a batch holds the system
   double* d_tops = nullptr;    //   operators [nmodes][ops]
   double* d_tb = nullptr;      //   assembled right-hand sides by position [nmodes][nr][nsolve]
   double* d_tv = nullptr;      //   fronts' eliminated parts [nmodes][nr][nsolve]
@@ -318,19 +316,20 @@ struct sx::Held {
   sx_msys* s = nullptr;
   sx::TreeDev* tree = nullptr;         // null: the plan stayed
   double *ops = nullptr, *tb = nullptr, *tv = nullptr, *tc = nullptr;
-  int use_tree = 0;
 };
 // where the assembly writes a solve's right-hand sides: [mode][nr][ld], node
 // g at perm[g] (perm null: at g).  The dissection solve reads them by
 // position and writes the solution to d_rhs by node.
 namespace sx {
 const int* tree_perm (const sx_msys* s);
-inline bool by_tree (const sx_msys* s)
-{
-  if (s->use_tree || !s->held || !s->tree) return s->use_tree;
-  const char* e = std::getenv ("SX_BAND_SPLIT");
-  return s->no_split || (e && std::atoi (e) == 0);
-}
+// Whether a solve on st runs the dissection.  A system without a plan never
+// does, one with a plan does unless a batch holds it: the own solves of such
+// a system run the split band sweeps where its band layout has them, as the
+// systems of batches always did (SX_BAND_SPLIT=0 turns split sweeps off and
+// so gives the dissection, what the batch records).  The first such solve
+// builds the band factor; under capture, or where that fails, it is the
+// dissection.
+bool by_tree (const sx_msys* s, hipStream_t st);
 struct RhsTo { double* p; int ld; const int* perm; };
 inline RhsTo rhs_in (const sx_msys* s, bool tree)
 {
@@ -462,9 +461,12 @@ int plan_field_solve_direct (BatchPlan& P, const sx_msys* s, int nz, int stride,
                              double* d_u, const double* d_lines);
 int plan_band_solve (BatchPlan& P, const sx_msys* s, int nr);
 int plan_tree_solve (BatchPlan& P, const sx_msys* s);
+// around a band solve of a system with a singular mode: its two right-hand
+// sides kept before, the refinement after
+int plan_sing_keep (BatchPlan& P, const sx_msys* s);
+int plan_sing_refine (BatchPlan& P, const sx_msys* s);
 int plan_mixed_passes (BatchPlan& P, sx_msys* s, int nz, int stride, double* d_f,
                        double* d_u, const double* d_lines, int passes);
-int plan_copy (BatchPlan& P, double* dst, const double* src, size_t n);
 int plan_condense32_tiled (BatchPlan& P, const sx_msys* s, int nz, int stride, const double* X,
                            double* Fp);
 int plan_recover32_tiled (BatchPlan& P, const sx_msys* s, int nz, int stride, const double* Fp,

@@ -346,13 +346,14 @@ int inner_solve (sx_msys* s, int nz, int stride, const double* X, double* Fp,
     hipLaunchKernelGGL (k_condense32, dim3 (m->nel, npl), dim3 (64), 0, st, m->np, m->nclass,
                         m->d_emap, m->d_cls, s->d_Bm32, X, Fp, stride, nz, s->base_mode);
   }
-  const RhsTo to = rhs_in (s, by_tree (s));
+  const bool tree = by_tree (s, st);
+  const RhsTo to = rhs_in (s, tree);
   hipLaunchKernelGGL (k_assemble_m, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw, Fp,
                       stride, lines, lstride, s->d_nsolve, to.p, to.ld, nz, s->base_mode,
                       to.perm);
   SX_HIP (hipGetLastError ());
-  int rc = band_solve (s, 2, st);
+  int rc = band_solve (s, tree, 2, st);
   if (rc) return rc;
   if (s->d_Mrec32) {
     if ((rc = recover32_tiled (s, nz, stride, Fp, V, st))) return rc;

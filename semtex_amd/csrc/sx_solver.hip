@@ -1698,7 +1698,6 @@ extern "C" int sx_msys_destroy (sx_msys_t s)
     block_free (s->block, s->block_bytes, s->block_dev);
   }
   tree_sing_free (s->sing);
-  tree_sing_free (s->sing_kept);
   delete s;
   return SX_OK;
 }
@@ -1790,36 +1789,40 @@ Grow::~Grow ()
   for (Item& i : items) (void) hipFree (i.p);
 }
 
+// The system's condensed element matrices, formed once more with its element
+// operators (buf: the allocation that holds them; S in it); d_status:
+// [nmodes + 1] cleared status words behind them
+static int condensed_again (const sx_msys* s, DevTmp& buf, double** S, int** d_status,
+                            hipStream_t st)
+{
+  const sx_mesh* m = s->m;
+  const int next = m->next, nint = m->nint, npnp = m->npnp;
+  const size_t nmc = (size_t) s->nmodes * m->nclass;
+  const size_t nws = nmc * ((size_t) npnp * npnp + (size_t) nint * nint), nS = nmc * next * next,
+               nB = nmc * next * nint, nH = nmc * nint * nint, nd = nws + nS + nB + nH;
+  SX_HIP (hipMalloc (&buf.p, sizeof (double) * (nd + s->nmodes + 1)));
+  double* d = (double*) buf.p;
+  *S = d + nws;
+  *d_status = (int*) (d + nd);
+  SX_HIP (hipMemsetAsync (*d_status, 0, sizeof (int) * (s->nmodes + 1), st));
+  return elem_sc (m, s->nmodes, s->lambda2, s->d_betak2, d, d + nws, d + nws + nS,
+                  d + nws + nS + nB, *d_status + s->nmodes, st);
+}
+
 int msys_hold (sx_msys* s, Held& h)
 {
   h = Held {};
   if (s->held) return SX_OK;
   Held was;
   was.s = s;
-  was.use_tree = s->use_tree;
-  if (s->use_tree) {
-    const sx_mesh* m = s->m;
-    const int next = m->next, nint = m->nint, npnp = m->npnp;
-    const size_t nmc = (size_t) s->nmodes * m->nclass;
-    const size_t nws = nmc * ((size_t) npnp * npnp + (size_t) nint * nint), nS = nmc * next * next,
-                 nB = nmc * next * nint, nH = nmc * nint * nint;
-    // the condensed element matrices again (k_elem_sc forms them with the
-    // element operators, which the system holds already)
-    DevTmp tbuf, tstat;
-    SX_HIP (hipMalloc (&tbuf.p, sizeof (double) * (nws + nS + nB + nH + 1)));
-    SX_HIP (hipMalloc (&tstat.p, sizeof (int) * (s->nmodes + 1)));
-    double* buf = (double*) tbuf.p;
-    int* d_status = (int*) tstat.p;
-    SX_HIP (hipMemset (d_status, 0, sizeof (int) * (s->nmodes + 1)));
-    int rc = elem_sc (m, s->nmodes, s->lambda2, s->d_betak2, buf, buf + nws, buf + nws + nS,
-                      buf + nws + nS + nB, d_status + s->nmodes, nullptr);
+  if (s->tree) {
+    DevTmp buf;
+    double* S = nullptr;
+    int* d_status = nullptr;
     Held now;
-    if (!rc) rc = tree_for_batch (s, buf + nws, nullptr, d_status, now);
-    if (!rc && (rc = band_build (s, buf + nws, nullptr, d_status))) band_drop (s);
-    if (rc) {
-      for (double* p : {now.ops, now.tb, now.tv, now.tc}) if (p) (void) hipFree (p);
-      return rc;
-    }
+    int rc = condensed_again (s, buf, &S, &d_status, nullptr);
+    if (!rc) rc = tree_for_batch (s, S, nullptr, d_status, now);
+    if (rc) return rc;
     if (now.tree) {
       was.tree = s->tree;
       was.ops = s->d_tops; was.tb = s->d_tb; was.tv = s->d_tv; was.tc = s->d_tc;
@@ -1827,12 +1830,6 @@ int msys_hold (sx_msys* s, Held& h)
       s->d_tops = now.ops; s->d_tb = now.tb; s->d_tv = now.tv; s->d_tc = now.tc;
     }
   }
-  // Neither the batch nor the system's own solves refine a singular mode from
-  // here on.  The buffers stay until the system goes: a graph the caller
-  // captured of its own solve still uses them
-  s->sing_kept = s->sing;
-  s->sing = nullptr;
-  s->use_tree = 0;
   s->held = 1;
   h = was;
   return SX_OK;
@@ -1854,12 +1851,40 @@ void msys_release (Held& h)
     s->tree = h.tree;
     s->d_tops = h.ops; s->d_tb = h.tb; s->d_tv = h.tv; s->d_tc = h.tc;
   }
-  if (h.use_tree) band_drop (s);
-  s->sing = s->sing_kept;
-  s->sing_kept = nullptr;
-  s->use_tree = h.use_tree;
   s->held = 0;
   h = Held {};
+}
+
+// The band factor of a system that solves by dissection
+static int own_band (sx_msys* s, hipStream_t st)
+{
+  DevTmp buf;
+  double* S = nullptr;
+  int* d_status = nullptr;
+  int rc = condensed_again (s, buf, &S, &d_status, st);
+  if (!rc) rc = band_build (s, S, st, d_status);
+  std::vector<int> status (s->nmodes + 1, 1);
+  if (!rc && hipMemcpy (status.data (), d_status, sizeof (int) * status.size (),
+                        hipMemcpyDeviceToHost) == hipSuccess &&
+      std::all_of (status.begin (), status.end (), [] (int e) { return e == 0; }))
+    return SX_OK;
+  band_drop (s);
+  return rc ? rc : (int) SX_ERR_FACTOR;
+}
+
+bool by_tree (const sx_msys* s, hipStream_t st)
+{
+  if (!s->tree || !s->held || s->no_split) return s->tree != nullptr;
+  const char* e = std::getenv ("SX_BAND_SPLIT");
+  if (e && std::atoi (e) == 0) return true;
+  if (!s->own_band) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing (st, &c) != hipSuccess) { (void) hipGetLastError (); return true; }
+    if (c != hipStreamCaptureStatusNone) return true;
+    sx_msys* sm = const_cast<sx_msys*> (s);
+    sm->own_band = band_splits (s) && own_band (sm, st) == SX_OK ? 1 : -1;
+  }
+  return s->own_band < 0;
 }
 
 }  // namespace sx
@@ -1921,7 +1946,6 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
     return SX_OK;
   }
   if ((rc = tree_prepare (m, num_modes, &s->tree))) return fail (rc);
-  s->use_tree = s->tree != nullptr;
   // The system's arrays in one block and the set-up's scratch in another
   // (block_alloc): two dozen allocations and frees of 10-20 us, and the
   // unmapping of the large ones, took longer than the GPU did.  The arrays
@@ -1939,13 +1963,13 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
     return o;
   };
   const size_t o_rhs = take (n, nrhs * std::max (s->nmax, 1));
-  const size_t o_tb = take (n, s->use_tree ? nrhs * m->nsolve : 0),
-               o_tc = take (n, s->use_tree ? nrhs * tree_slots (s->tree) : 0), nzero = n;
+  const size_t o_tb = take (n, s->tree ? nrhs * m->nsolve : 0),
+               o_tc = take (n, s->tree ? nrhs * tree_slots (s->tree) : 0), nzero = n;
   const size_t o_par = take (n, 2 * (size_t) num_modes), o_G = take (n, nrhs * m->nglobal),
                o_Bm = take (n, nmc * next * nint), o_Hi = take (n, nmc * nint * nint),
                o_rec = take (n, nmc * nrec), o_con = take (n, nmc * ncon),
-               o_tv = take (n, s->use_tree ? nrhs * m->nsolve : 0),
-               o_ops = take (n, s->use_tree ? tree_ops (s->tree) * num_modes : 0);
+               o_tv = take (n, s->tree ? nrhs * m->nsolve : 0),
+               o_ops = take (n, s->tree ? tree_ops (s->tree) * num_modes : 0);
   if ((rc = block_alloc ((void**) &s->block, sizeof (double) * n, &s->block_bytes, &s->block_dev)))
     return fail (rc);
   double* base = (double*) s->block;
@@ -1959,7 +1983,7 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
     s->d_Mrec = base + o_rec;
     s->d_Mcon = base + o_con;
   }
-  if (s->use_tree) {
+  if (s->tree) {
     s->d_tb = base + o_tb;
     s->d_tc = base + o_tc;
     s->d_tv = base + o_tv;
@@ -1976,7 +2000,7 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
   size_t nt = 0;
   const size_t o_st = take (nt, num_modes + 1), o_ws = take (nt, nmc * ws_per),
                o_S = take (nt, nmc * next * next),
-               o_f = take (nt, s->use_tree ? tree_scratch (s->tree, num_modes) : 0);
+               o_f = take (nt, s->tree ? tree_scratch (s->tree, num_modes) : 0);
   if ((rc = block_alloc ((void**) &d_ws, sizeof (double) * nt, &ws_bytes, &ws_dev))) return fail (rc);
   double* d_S = d_ws + o_S;
   int* d_status = (int*) (d_ws + o_st);
@@ -1992,7 +2016,7 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
                         s->d_Mrec, s->d_Mcon);
     TRY (hipGetLastError ());
   }
-  rc = s->use_tree ? tree_factor (s, d_S, d_ws + o_f, st, d_status)
+  rc = s->tree ? tree_factor (s, d_S, d_ws + o_f, st, d_status)
                    : band_build (s, d_S, st, d_status);
   if (rc || (rc = tree_sing_setup (s, d_S, st, d_status))) return fail (rc);
   std::vector<int> status (num_modes + 1);
@@ -2260,7 +2284,8 @@ int field_solve_direct (const sx_msys* s, int nz, int stride, double* d_f, doubl
   const int npl = n_solved_planes (nz, s->base_mode);
   const int lstride = m->nbound * m->np;
   const double* lines = (d_lines && m->nbound) ? d_lines : nullptr;
-  const RhsTo to = rhs_in (s, by_tree (s));
+  const bool tree = by_tree (s, st);
+  const RhsTo to = rhs_in (s, tree);
   // the essential values and the essential elements' weak form in one
   // launch where the tiled condensation follows
   const bool ew = tiled_ok (m) && m->ness;
@@ -2287,7 +2312,7 @@ int field_solve_direct (const sx_msys* s, int nz, int stride, double* d_f, doubl
   }
   // a twisted system's bottom piece addressed by the assembly and the
   // recovery themselves (no gather and scatter launches around the sweeps)
-  const bool fold = !by_tree (s) && !s->sing && s->tw && s->sw_panel && tiled_ok (m) && s->tile_mf;
+  const bool fold = !tree && !s->sing && s->tw && s->sw_panel && tiled_ok (m) && s->tile_mf;
   {
     PhaseScope ps (2, st, timed);
     if (fold)
@@ -2304,7 +2329,7 @@ int field_solve_direct (const sx_msys* s, int nz, int stride, double* d_f, doubl
   SX_HIP (hipGetLastError ());
   {
     PhaseScope ps (3, st, timed);
-    if ((rc = band_solve (s, 2, st, fold ? 0 : 3))) return rc;
+    if ((rc = band_solve (s, tree, 2, st, fold ? 0 : 3))) return rc;
   }
   {
     PhaseScope ps (4, st, timed);
@@ -2342,7 +2367,7 @@ int msys_reserve_rhs (sx_msys* s, int nr)
     return SX_ERR_ARG;
   }
   if (nr <= s->rhs_cap) return SX_OK;
-  if (!s->use_tree && (!s->sw_panel || s->sw_D > 6)) {
+  if (!s->tree && (!s->sw_panel || s->sw_D > 6)) {
     set_error ("msys_reserve_rhs: more than 2 right-hand sides per mode need the panel "
                "sweeps with at most 6 off-diagonal blocks (band offsets kd <= 447)");
     return SX_ERR_LIMIT;
@@ -2564,7 +2589,8 @@ int field_solve_group (sx_msys* s, int nf, int nz, int stride, double* const* d_
   const int npl = n_solved_planes (nz, s->base_mode), nr = 2 * nf;
   const int lstride = m->nbound * m->np;
   const size_t gstride = (size_t) 2 * s->nmodes * m->nglobal;
-  const RhsTo to = rhs_in (s, by_tree (s));
+  const bool tree = by_tree (s, st);
+  const RhsTo to = rhs_in (s, tree);
   // the register-operand element kernels take up to three fields per launch
   const bool grouped = nf <= 3 && tiled_ok (m) && s->tile_mf;
   const int npmr = reg_npm (m->np);
@@ -2603,7 +2629,7 @@ int field_solve_group (sx_msys* s, int nf, int nz, int stride, double* const* d_
                         2 * f, to.perm);
   }
   SX_HIP (hipGetLastError ());
-  if (int rc = band_solve (s, nr, st)) return rc;
+  if (int rc = band_solve (s, tree, nr, st)) return rc;
   if (grouped) {
     FieldCPtrs F {}, G {};
     FieldPtrs U {};
@@ -2729,12 +2755,13 @@ extern "C" int sx_field_solve_weak (sx_msys_t s, int nz, int stride, double* d_w
   hipLaunchKernelGGL (k_essential, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_ess, nullptr, 0, s->d_G, nz, s->base_mode);
   if ((rc = condense (s, nz, stride, d_w, s->d_G, st, 1))) return rc;
-  const RhsTo to = rhs_in (s, by_tree (s));
+  const bool tree = by_tree (s, st);
+  const RhsTo to = rhs_in (s, tree);
   hipLaunchKernelGGL (k_assemble, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw, d_w,
                       stride, nullptr, 0, s->d_nsolve, to.p, to.ld, nz, s->base_mode, 2, 0, to.perm);
   SX_HIP (hipGetLastError ());
-  if ((rc = band_solve (s, 2, st))) return rc;
+  if ((rc = band_solve (s, tree, 2, st))) return rc;
   return recover (s, nz, stride, d_w, d_u, s->d_G, 2, 0, st);
 }
 

@@ -487,7 +487,7 @@ __global__ __launch_bounds__(256) void k_tree_entries (int npairs, const int* __
 // out = b - A x for one mode's nr right-hand sides (b by bperm, out by
 // operm: the positions of their dissections), accumulated in twice
 // the working precision (error-free products and sums); a wavefront per row
-__global__ __launch_bounds__(256) void k_tree_residual (
+__device__ __forceinline__ void k_tree_residual_body (
     int ns, int nmax, int nr, const int* __restrict__ ptr, const int* __restrict__ col,
     const int* __restrict__ pair, const double* __restrict__ val, const double* __restrict__ b,
     int ldb, const int* __restrict__ bperm, const double* __restrict__ x, double* out, int ldo,
@@ -521,6 +521,26 @@ __global__ __launch_bounds__(256) void k_tree_residual (
     }
   }
 }
+
+__global__ __launch_bounds__(256) void k_tree_residual (
+    int ns, int nmax, int nr, const int* __restrict__ ptr, const int* __restrict__ col,
+    const int* __restrict__ pair, const double* __restrict__ val, const double* __restrict__ b,
+    int ldb, const int* __restrict__ bperm, const double* __restrict__ x, double* out, int ldo,
+    const int* __restrict__ operm)
+{
+  k_tree_residual_body (ns, nmax, nr, ptr, col, pair, val, b, ldb, bperm, x, out, ldo, operm);
+}
+struct FnTreeResidual {
+  template <typename... A> __device__ __forceinline__ void operator() (A... a) const
+  { k_tree_residual_body (a...); }
+};
+struct FnTreeKeep {
+  __device__ __forceinline__ void operator() (double* to, const double* from, int n) const
+  {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) to[i] = from[i];
+  }
+};
 
 template <typename V> int upload (V** d, const std::vector<V>& h)
 {
@@ -722,13 +742,12 @@ static TreeArgs tree_args (const sx_msys* s)
 // The same launches recorded into a batch's plan, the roots of all its
 // systems in one phase (trees of up to TREE_PLAN_LEVELS levels end level)
 constexpr int TREE_PLAN_LEVELS = 5;
-int plan_tree_solve (BatchPlan& P, const sx_msys* s)
+static void plan_levels (BatchPlan& P, const TreeDev* t, const TreeArgs& args, int nm)
 {
-  const TreeDev* t = s->tree;
   const int nl = (int) t->P.lev.size (), root = P.phase + std::max (nl, TREE_PLAN_LEVELS) - 1;
   auto level = [&] (int j, int down) {
-    TreeArgs T = tree_args (s);
-    const LevelLaunch l = level_launch (t, T, j, down, s->nmodes, 2);
+    TreeArgs T = args;
+    const LevelLaunch l = level_launch (t, T, j, down, nm, 2);
     P.phase = down ? root + j : root - j;
     if (!l.blocks) return (int) SX_OK;
     return tree_instance (l, [&] (auto d, auto w) {
@@ -740,7 +759,6 @@ int plan_tree_solve (BatchPlan& P, const sx_msys* s)
   for (int j = nl - 1; j > 0; j--) level (j, 0);
   for (int j = 0; j < nl; j++) level (j, 1);
   P.phase = root + std::max (nl, TREE_PLAN_LEVELS);
-  return SX_OK;
 }
 
 // Refinement of a singular mode's solution (pure Neumann, its last unknown
@@ -878,37 +896,91 @@ int tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_statu
   return SX_OK;
 }
 
-static int refine (const sx_msys* s, int nr, const double* b, int ldb, const int* bperm,
-                   hipStream_t st)
+// A refinement's right-hand sides as they were before the solve, by node
+// (band solves) or by position of the solve's dissection
+struct Kept { const double* b; int ld; const int* perm; };
+static Kept kept (const sx_msys* s, int nr, bool tree)
+{
+  const TreeSing* g = s->sing;
+  if (!tree) return {g->b, s->nmax, nullptr};
+  const int nsp = s->tree->P.nsolve;
+  return {s->d_tb + (size_t) g->mode * nr * nsp, nsp, s->tree->perm};
+}
+static double* sing_x (const sx_msys* s, int nr)
+{
+  return s->d_rhs + (size_t) s->sing->mode * nr * s->nmax;
+}
+static TreeArgs sing_args (const sx_msys* s, int nr)
+{
+  const TreeSing* g = s->sing;
+  TreeArgs T {};
+  T.ops = g->ops;
+  T.in = g->r; T.rhs = g->dx; T.v = g->v; T.cb = g->cb;
+  T.sum = sing_x (s, nr);
+  T.nmax = s->nmax;
+  T.nsolve = s->d_nsolve + g->mode;
+  return T;
+}
+
+static int refine (const sx_msys* s, int nr, bool tree, hipStream_t st)
 {
   const TreeSing* g = s->sing;
   const sx_mesh* m = s->m;
   const int ns = s->nsolve[g->mode];
-  double* x = s->d_rhs + (size_t) g->mode * nr * s->nmax;
+  const Kept k = kept (s, nr, tree);
   hipLaunchKernelGGL (k_tree_residual, dim3 ((ns + 3) / 4), dim3 (256), 0, st, ns, s->nmax, nr,
-                      m->d_sptr, m->d_scol, m->d_spair, g->val, b, ldb, bperm, x, g->r,
-                      g->t->P.nsolve, g->t->perm);
+                      m->d_sptr, m->d_scol, m->d_spair, g->val, k.b, k.ld, k.perm, sing_x (s, nr),
+                      g->r, g->t->P.nsolve, g->t->perm);
   SX_HIP (hipGetLastError ());
-  TreeArgs T {};
-  T.ops = g->ops;
-  T.in = g->r; T.rhs = g->dx; T.v = g->v; T.cb = g->cb;
-  T.sum = x;
-  T.nmax = s->nmax;
-  T.nsolve = s->d_nsolve + g->mode;
-  return sweep (g->t, T, 1, nr, st);
+  return sweep (g->t, sing_args (s, nr), 1, nr, st);
 }
 
 int sing_keep (const sx_msys* s, int nr, hipStream_t st)
 {
-  const TreeSing* g = s->sing;
-  SX_HIP (hipMemcpyAsync (g->b, s->d_rhs + (size_t) g->mode * nr * s->nmax,
-                          sizeof (double) * nr * s->nmax, hipMemcpyDeviceToDevice, st));
+  SX_HIP (hipMemcpyAsync (s->sing->b, sing_x (s, nr), sizeof (double) * nr * s->nmax,
+                          hipMemcpyDeviceToDevice, st));
   return SX_OK;
 }
 
-int sing_refine (const sx_msys* s, int nr, hipStream_t st)
+int sing_refine (const sx_msys* s, int nr, hipStream_t st) { return refine (s, nr, false, st); }
+
+// The same recorded (two right-hand sides per mode)
+static void plan_refine (BatchPlan& P, const sx_msys* s, bool tree)
 {
-  return refine (s, nr, s->sing->b, s->nmax, nullptr, st);
+  const TreeSing* g = s->sing;
+  const sx_mesh* m = s->m;
+  const int ns = s->nsolve[g->mode], nr = 2;
+  const Kept k = kept (s, nr, tree);
+  batch_rec<256, FnTreeResidual> (P, dim3 ((ns + 3) / 4), 256, 0, ns, s->nmax, nr,
+                                  (const int*) m->d_sptr, (const int*) m->d_scol,
+                                  (const int*) m->d_spair, (const double*) g->val, k.b, k.ld,
+                                  k.perm, (const double*) sing_x (s, nr), g->r,
+                                  g->t->P.nsolve, (const int*) g->t->perm);
+  P.phase++;
+  plan_levels (P, g->t, sing_args (s, nr), 1);
+}
+
+int plan_sing_keep (BatchPlan& P, const sx_msys* s)
+{
+  const int n = 2 * s->nmax;
+  batch_rec<256, FnTreeKeep> (P, dim3 ((n + 255) / 256), 256, 0, s->sing->b,
+                              (const double*) sing_x (s, 2), n);
+  P.phase++;
+  return SX_OK;
+}
+
+int plan_sing_refine (BatchPlan& P, const sx_msys* s)
+{
+  plan_refine (P, s, false);
+  return SX_OK;
+}
+
+// A system's solve recorded into a batch's plan
+int plan_tree_solve (BatchPlan& P, const sx_msys* s)
+{
+  plan_levels (P, s->tree, tree_args (s), s->nmodes);
+  if (s->sing) plan_refine (P, s, true);
+  return SX_OK;
 }
 
 // Solve of the nr (2, 4, 6) right-hand sides per mode from d_tb to d_rhs.
@@ -922,9 +994,7 @@ int tree_solve (const sx_msys* s, int nr, hipStream_t st)
   s->last_nr = nr;
   const TreeDev* t = s->tree;
   if (int rc = sweep (t, tree_args (s), s->nmodes, nr, st)) return rc;
-  if (!s->sing) return SX_OK;
-  const int nsp = t->P.nsolve;
-  return refine (s, nr, s->d_tb + (size_t) s->sing->mode * nr * nsp, nsp, t->perm, st);
+  return s->sing ? refine (s, nr, true, st) : (int) SX_OK;
 }
 
 }  // namespace sx

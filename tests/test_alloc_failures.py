@@ -40,7 +40,7 @@ PRELUDE = textwrap.dedent("""
         def free(self): S.hipFree(self.p)
 
     def reserve(M, nr): return L._ZN2sx16msys_reserve_rhsEP7sx_msysi(M.handle, nr)
-    def solve_nr(M, nr): return L._ZN2sx10band_solveEPK7sx_msysiP12ihipStream_ti(M.handle, nr, None, 3)
+    def solve_nr(M, nr): return L._ZN2sx10tree_solveEPK7sx_msysiP12ihipStream_t(M.handle, nr, None)
 
     class RawBatch:
         def __init__(self, Ms, nz=1):
@@ -157,5 +157,52 @@ def test_failed_batch_leaves_its_systems_as_they_were(bc):
     del Ms
     assert S.stub_live() == 0, S.stub_live()
     assert S.stub_bad_pointers() == 0
+    print("ok")
+    """)
+
+
+def test_held_system_keeps_its_refinement_and_builds_a_band_only_when_asked():
+    """A batch factorises no band for its systems and records the singular
+    mode's refinement; a held system's own solves keep the refinement, run
+    split band sweeps only where its layout has them, and the dissection where
+    the band factor does not fit."""
+    run("""
+    def held(nx, ny, np_, bc, **kw):
+        m = rect_mesh(nx, ny, np_, 0.0, 6.0, -1.0, 1.0, bc=tuple(bc), **kw)
+        M = ModalMatrixSys(0.0, 1.0, 0, 1, GpuMesh(m))
+        B = RawBatch([M])
+        bands, res = launches("k_band_factor"), launches("FnTreeResidual")
+        assert B.create() == 0
+        assert launches("k_band_factor") == bands
+        assert (launches("FnTreeResidual") > res) == (bc == "NNNN")
+        return M, B
+    # a layout with split sweeps, its mode singular
+    M, B = held(16, 12, 8, "NNNN", periodic_x=True)
+    r = launches("k_tree_residual")
+    assert own_solve(M) == 0 and M.layout()["kernel"] == 3
+    bands = launches("k_band_factor")
+    assert bands > 0 and launches("k_tree_residual") == r + 1
+    assert own_solve(M) == 0 and launches("k_band_factor") == bands
+    B.destroy(); B.free(); del M, B
+    # the band factor does not fit: the dissection, and nothing kept
+    M, B = held(16, 12, 8, "NNNN", periodic_x=True)
+    bytes_, r = S.stub_bytes(), launches("k_tree_residual")
+    k = 0
+    b = [Buf(M.gmesh.plane_size) for _ in range(2)]
+    S.stub_fail(0, 1 << 30)
+    assert L.sx_field_solve(M.handle, 1, M.gmesh.plane_size, b[0].p, b[1].p, None, None) == 0
+    S.stub_fail(-1, 0)
+    for x in b: x.free()
+    assert M.layout()["kernel"] == 4 and S.stub_bytes() == bytes_
+    assert launches("k_tree_residual") == r + 1
+    B.destroy(); B.free(); del M, B
+    # a band past the panel sweeps
+    M, B = held(48, 40, 9, "DDDN")
+    assert M.layout()["nband"] > 513
+    bands = launches("k_band_factor")
+    assert own_solve(M) == 0 and M.layout()["kernel"] == 4
+    assert launches("k_band_factor") == bands
+    B.destroy(); B.free(); del M, B
+    assert S.stub_live() == 0 and S.stub_bad_pointers() == 0
     print("ok")
     """)
