@@ -2725,6 +2725,21 @@ int band_solve (const sx_msys* s, bool tree, int nr, hipStream_t st, int moves)
   return sing_refine (s, nr, st);
 }
 
+// Time of a band solve (two right-hand sides per mode) of more than 32 modes,
+// us: single-piece panel sweeps, a chain of 64-row block steps forward and
+// back whose latency counts while few modes run, their panels' bytes with
+// many (past 128 modes a workgroup takes both right-hand sides).  The fit to
+// 320 traced solves (bands of 1 to 6 off-diagonal blocks, 48 to 512 modes),
+// within 20 %.  Offset-major sweeps: not worth comparing.
+double band_us (const sx_mesh* m, int nmodes)
+{
+  if (!use_panels (m->nband, m->nsolve)) return 1e30;
+  const int D = panel_D (m->nband), nblk = (m->nsolve + PB - 1) / PB;
+  const double step = D <= 2 ? 2.45 + (nmodes <= 128 ? 0.003 : 0.0065) * D * nmodes
+                             : 2.3 + 0.6 * (D - 2) + 0.006 * D * nmodes;
+  return 4.0 + nblk * step;
+}
+
 bool band_splits (const sx_msys* s)
 {
   std::vector<int> tw;

@@ -129,6 +129,7 @@ void   band_drop (sx_msys* s);       // gives the factor (or a part of one) up
 // right-hand side, 2 scatter its solution (3: both; 0 when the caller's
 // assembly and recovery address the bottom piece themselves)
 int    band_solve (const sx_msys* s, bool tree, int nr, hipStream_t st, int moves = 3);
+double band_us (const sx_mesh* m, int nmodes);   // estimated time of a solve
 bool   band_splits (const sx_msys* s);   // the band layout would have split sweeps
 // per-mode split of a twisted system (d_tw): TW ints per mode
 constexpr int TW = 8;

@@ -73,6 +73,7 @@ struct TreePlan {
 };
 
 constexpr size_t TREE_LDS_MAX = 96 * 1024;   // a workgroup's column operand
+constexpr int TREE_FEW_MODES = 32;           // all workgroups of a level resident at once
 
 // false when the mesh does not suit it (an element holding one node twice,
 // a node no element holds, operators past the size bound).  share: solves

@@ -542,12 +542,18 @@ struct FnTreeKeep {
   }
 };
 
+// h on the device, unless it is there already
 template <typename V> int upload (V** d, const std::vector<V>& h)
 {
-  *d = nullptr;
-  if (h.empty ()) return SX_OK;
-  SX_HIP (hipMalloc (d, sizeof (V) * h.size ()));
-  SX_HIP (hipMemcpy (*d, h.data (), sizeof (V) * h.size (), hipMemcpyHostToDevice));
+  if (*d || h.empty ()) return SX_OK;
+  V* p = nullptr;
+  SX_HIP (hipMalloc (&p, sizeof (V) * h.size ()));
+  const hipError_t e = hipMemcpy (p, h.data (), sizeof (V) * h.size (), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    (void) hipFree (p);
+    return hip_fail (e, "hipMemcpy");
+  }
+  *d = p;
   return SX_OK;
 }
 
@@ -557,7 +563,7 @@ template <typename V> int upload (V** d, const std::vector<V>& h)
 struct TreeDev {
   TreePlan P;
   int nmodes = 0, share = 1;
-  bool ok = false;
+  bool ok = false, slower = false;     // slower: the band solve is the faster one
   TreeClass* cls = nullptr;
   TreeChild* child = nullptr;
   TreeItem* item = nullptr;
@@ -586,34 +592,42 @@ static bool band_forced ()
 // suit, and operators of more than 24 GB.  always: also under a variable
 // that chooses a band layout.
 constexpr size_t TREE_OPS_MAX = (size_t) 3 << 30;      // doubles
+// More than TREE_FEW_MODES modes: also where the band solve is estimated
+// faster (up to 32 modes its twisted and split sweeps lost everywhere
+// measured; with many its chain costs little next to the fronts' many
+// workgroups).  Whole solves, band / dissection: 5x5 elements N_P=6, 128
+// modes 40 / 53 us; 8x8 N_P=8, 128 modes 80 / 91 us; uniform 12x24 N_P=6, 256
+// modes, which stays, 411 / 315 us.
+constexpr double TREE_BAND = 0.95;
 
 int tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always, int share)
 {
   *out = nullptr;
   if ((!always && band_forced ()) || m->nband > 768) return SX_OK;
   std::lock_guard<std::mutex> lock (m->tree_mu);
-  for (TreeDev* t : m->trees)
-    if (t->nmodes == nmodes && t->share == share) {
-      *out = t->ok ? t : nullptr;
-      return SX_OK;
-    }
-  TreeDev* t = new TreeDev;
-  t->nmodes = nmodes;
-  t->share = share;
-  m->trees.push_back (t);
-  size_t f = 0;
-  t->ok = tree_plan (m, nmodes, share, t->P);
-  for (const TreeLevel& L : t->P.lev) f = std::max (f, L.fsize);
-  t->ok = t->ok && t->P.ops * nmodes <= TREE_OPS_MAX && f * nmodes <= TREE_OPS_MAX;
-  if (!t->ok) { t->P = TreePlan (); return SX_OK; }
+  TreeDev* t = nullptr;
+  for (TreeDev* q : m->trees)
+    if (q->nmodes == nmodes && q->share == share) t = q;
+  if (!t) {
+    t = new TreeDev;
+    t->nmodes = nmodes;
+    t->share = share;
+    m->trees.push_back (t);
+    size_t f = 0;
+    t->ok = tree_plan (m, nmodes, share, t->P);
+    for (const TreeLevel& L : t->P.lev) f = std::max (f, L.fsize);
+    t->ok = t->ok && t->P.ops * nmodes <= TREE_OPS_MAX && f * nmodes <= TREE_OPS_MAX;
+    if (!t->ok) t->P = TreePlan ();
+    t->slower = nmodes > TREE_FEW_MODES && band_us (m, nmodes) < TREE_BAND * t->P.est_us;
+  }
+  if (!t->ok || (t->slower && !always)) return SX_OK;
+  // (the tables of a plan whose upload failed are tried again)
   int rc;
   if ((rc = upload (&t->cls, t->P.cls)) || (rc = upload (&t->child, t->P.child)) ||
       (rc = upload (&t->item, t->P.item)) || (rc = upload (&t->map, t->P.map)) ||
       (rc = upload (&t->gk, t->P.gk)) || (rc = upload (&t->gb, t->P.gb)) ||
-      (rc = upload (&t->tgt, t->P.tgt)) || (rc = upload (&t->perm, t->P.perm))) {
-    t->ok = false;
+      (rc = upload (&t->tgt, t->P.tgt)) || (rc = upload (&t->perm, t->P.perm)))
     return rc;
-  }
   *out = t;
   return SX_OK;
 }

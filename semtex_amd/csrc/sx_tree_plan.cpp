@@ -202,6 +202,73 @@ void split_rows (int blocks, int pairs, long long tiles, bool batch, int* nrb, i
   *nrb = 4 / *kw;
 }
 
+// Time of a level (both directions, two right-hand sides per mode), us; the
+// cuts are chosen by it.  src: its fronts have fronts among their parts.
+// Up to TREE_FEW_MODES modes (and TREE_FEW_OPERATORS element classes times
+// modes: on a mesh graded both ways each front is a class and a tile of its
+// own) most workgroups are resident at once and a level costs its launches
+// (4.5 us each measured) and the bytes of its operators, once from memory
+// (4 TB/s) and once per tile of columns from the L2s (12 TB/s).  share:
+// solves side by side share the launches.
+// With more the workgroups queue: that of a small front is a chain of
+// load rounds, and its place on a CU, not the bytes, bounds a level of many
+// modes or many classes (cuts chosen by bytes alone took up to 1.9x the
+// solve of these or of the band at 128 to 256 modes).  The terms, a launch
+// with one workgroup's chain, every workgroup, operators, gathers and
+// stores, are the fit to 2,400 traced launches (4x4 to 32x32 elements, N_P 4
+// to 12, uniform and graded): a solve within 15 % for nine tenths of them.
+// (The fit is no better than the bytes up to 32 modes: it cut the 16x16
+// N_P=10 problem into 3 levels instead of 4, 152 us instead of 145.)
+constexpr int TREE_FEW_OPERATORS = 4096;
+struct LevelClass { int k, b, count; };
+double direction_us (const std::vector<LevelClass>& cl, int nmodes, bool down, bool src)
+{
+  long long tiles = 0;
+  for (const LevelClass& c : cl) {
+    const int nf = tile_fronts (c.k + c.b, 2);
+    tiles += (c.count + nf - 1) / nf;
+  }
+  double wg = 0.0, bytes = 0.0, in = 0.0, out = 0.0, turns = 0.0;
+  int kmax = 0;
+  for (const LevelClass& c : cl) {
+    const int nf = tile_fronts (c.k + c.b, 2), nt = (c.count + nf - 1) / nf;
+    const int K = down ? c.k + c.b : c.k, rows = down ? c.k : c.b;
+    const int blocks = (rows + 15) / 16, pairs = (K + 7) / 8;
+    if (!blocks) continue;
+    kmax = std::max (kmax, K);
+    int nrb, kw;
+    split_rows (blocks, pairs, tiles * nmodes, false, &nrb, &kw);
+    const int per = (blocks + nrb - 1) / nrb;            // workgroups of a tile
+    wg += (double) nt * per;
+    bytes += 1024.0 * nt * blocks * pairs;
+    in += 2.0 * c.count * per * K;
+    out += 2.0 * c.count * rows;
+    turns += (double) nt * per * ((nrb + 4 / kw - 1) / (4 / kw)) * ((pairs + kw - 1) / kw);
+  }
+  if (wg == 0.0) return 0.0;
+  const double chain = down ? 3.8 + 0.032 * turns / wg + 9.4e-4 * kmax + 1.5e-3 * in / wg
+                           : 2.6 + 0.26 * turns / wg + 2.3e-3 * kmax + 7.6e-4 * in / wg;
+  const double each = down ? 4.0e-3 * wg + 1.7e-7 * bytes + (src ? 6.4e-6 : 3.4e-6) * out
+                           : 4.4e-3 * wg + 2.3e-7 * bytes + (src ? 1.4e-6 * in + 2.8e-5 * out : 5.0e-6 * out);
+  return chain + nmodes * each;
+}
+
+double level_us (const std::vector<LevelClass>& cl, int nmodes, int share, bool many, bool root,
+                 bool src)
+{
+  if (many)
+    return direction_us (cl, nmodes, true, src) + (root ? 0.0 : direction_us (cl, nmodes, false, src));
+  double us = (root ? 4.5 : 9.0) / share;
+  for (const LevelClass& c : cl) {
+    const int K = c.k + c.b, nf = tile_fronts (K, 2);
+    const double bytes = 8.0 * nmodes * ((double) c.k * K + (double) c.k * c.b);
+    us += bytes / 4.0e6 + bytes * ((c.count + nf - 1) / nf) / 12.0e6;
+    // one wavefront's chain of k-step rounds, each a memory latency
+    us += 1e-3 * K / share;
+  }
+  return us;
+}
+
 }  // namespace
 
 bool tree_plan (const sx_mesh* m, int nmodes, int share, TreePlan& P)
@@ -245,39 +312,33 @@ bool tree_plan (const sx_mesh* m, int nmodes, int share, TreePlan& P)
   const int root = B.make (all, 0);
 
   // -- cut the binary tree into levels: the cheapest chain of depths
-  // 0 = d0 < d1 < ... (a level's fronts are the tree nodes at its depth).
-  // A level costs its launches (4.5 us each measured, one forward, one
-  // backward) and the bytes of its operators, once from memory (4 TB/s)
-  // and once per tile of columns from the L2s (12 TB/s).
+  // 0 = d0 < d1 < ... (a level's fronts are the tree nodes at its depth)
   const int nd = B.maxdepth + 1;
   std::vector<std::vector<int>> at (nd + 1);
   for (int i = 0; i < (int) B.node.size (); i++)
     if (B.node[i].elem < 0 || i == root) at[B.node[i].depth].push_back (i);
   auto bnd_dim = [&] (int id) { return (int) B.node[id].bnd.size (); };
+  const int last = std::max (nd - 1, 1);         // elements lie at depth <= nd - 1
+  const bool many = share == 1 && (nmodes > TREE_FEW_MODES ||
+                                   (long long) nmodes * m->nclass > TREE_FEW_OPERATORS);
   auto cost = [&] (int a, int c) {
     std::map<int, int> count;
     for (int id : at[a]) count[B.node[id].cls]++;
-    double us = (a == 0 ? 4.5 : 9.0) / share;
+    std::vector<LevelClass> cl;
     for (auto& kv : count) {
       const int id = B.rep[kv.first];
       // the representative may sit at another depth: same subtree, shifted
       const int k = B.node[id].elem >= 0 ? bnd_dim (id)
                                          : B.elim_to (id, c - a + B.node[id].depth);
       const int b = B.node[id].elem >= 0 ? 0 : bnd_dim (id);
-      const int K = k + b;
-      if (sizeof (double) * (size_t) K * 7 > TREE_LDS_MAX || K > 4096) return 1e30;
-      const double bytes = 8.0 * nmodes * ((double) k * K + (double) k * b);
-      const int nf = tile_fronts (K, 2);
-      us += bytes / 4.0e6 + bytes * ((kv.second + nf - 1) / nf) / 12.0e6;
-      // one wavefront's chain of k-step rounds, each a memory latency
-      us += 1e-3 * K / share;
+      if (sizeof (double) * (size_t) (k + b) * 7 > TREE_LDS_MAX || k + b > 4096) return 1e30;
+      cl.push_back ({k, b, kv.second});
     }
-    return us;
+    return level_us (cl, nmodes, share, many, a == 0, c < last);
   };
   std::vector<double> best (nd + 1, 1e30);
   std::vector<int> from (nd + 1, -1);
   best[0] = 0.0;
-  const int last = std::max (nd - 1, 1);         // elements lie at depth <= nd - 1
   for (int c = 1; c <= last; c++)
     for (int a = 0; a < c; a++) {
       if (best[a] >= 1e30) continue;
