@@ -316,7 +316,8 @@ __global__ __launch_bounds__(PV_THREADS) void k_pcg_dir (
 // z = pc r, rho' = r.z, p = z + rho'/rho p follows in the same launch (both
 // need the whole plane, one workgroup's).  R > 0: the plane's values stay in
 // registers, R a thread (npts <= R PV_THREADS), so a launch is its gather's
-// three rounds of loads and three sums; R = 0: any size, through memory.
+// three rounds of loads (one more at R = 8) and three sums; R = 0: any size,
+// through memory.
 // 14.5 us as two launches walking memory, 6x8 elements at N_P=8.
 template <int R>
 __global__ __launch_bounds__(PV_THREADS) void k_pcg_step (
@@ -337,6 +338,10 @@ __global__ __launch_bounds__(PV_THREADS) void k_pcg_step (
   const double rho = st.rho[y], eps = st.eps[y];
   const int it = st.it[y] + 1;
   constexpr int RR = R > 0 ? R : 1;
+  // (eight values a thread with their gathers in flight spill, 92 bytes a
+  // lane; x and pc, not needed before alpha, come once the gathers are done:
+  // 14x8 elements at N_P=7, 16 planes, 1190 -> 920 us a solve)
+  constexpr bool LATE = R > 4;
   double pv[RR], qv[RR], xv[RR], rv[RR], cv[RR];
   double pq = 0.0;
   if constexpr (R > 0) {
@@ -351,9 +356,11 @@ __global__ __launch_bounds__(PV_THREADS) void k_pcg_step (
       if (i < (int) npts) {
         if (i < ns) { c0[u] = gptr[i]; n[u] = gptr[i + 1] - c0[u]; }
         pv[u] = p[i];
-        xv[u] = x[i];
         rv[u] = r[i];
-        cv[u] = pcm[i];
+        if (!LATE) {
+          xv[u] = x[i];
+          cv[u] = pcm[i];
+        }
       }
     }
 #pragma unroll
@@ -376,6 +383,15 @@ __global__ __launch_bounds__(PV_THREADS) void k_pcg_step (
       for (int c = 4; c < n[u]; c++) v += Ly[gsrc[c0[u] + c]];
       qv[u] = v;
     }
+    if (LATE)
+#pragma unroll
+      for (int u = 0; u < R; u++) {
+        const int i = threadIdx.x + u * PV_THREADS;
+        if (i < (int) npts) {
+          xv[u] = x[i];
+          cv[u] = pcm[i];
+        }
+      }
 #pragma unroll
     for (int u = 0; u < R; u++) pq += pv[u] * qv[u];
   } else {
