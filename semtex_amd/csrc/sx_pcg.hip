@@ -21,7 +21,6 @@
 #include <algorithm>
 #include <cmath>
 #include <mutex>
-#include <utility>
 #include <vector>
 
 #include "sx_internal.h"
@@ -516,9 +515,10 @@ int pcg_setup (sx_msys* s, hipStream_t st)
 }  // namespace sx
 
 namespace {
-// Pinned copies of the planes' flags and their events.  One set (a few hundred
-// bytes) is kept for the next solve, a second thread's solve makes its own: a
-// pinned allocation costs more than the solve of a small system.
+// Pinned copies of the planes' flags and their events.  One set a device (a
+// few hundred bytes) is kept for the next solve, a second thread's solve
+// makes its own: a pinned allocation costs more than the solve of a small
+// system.
 struct PcgHostBuf {
   int dev = -1, cap = 0;
   int* mem = nullptr;
@@ -536,35 +536,47 @@ struct PcgHost {
   PcgHostBuf b;
   int* flags[2];
   hipEvent_t ev[2];
+  hipStream_t st;
   static std::mutex mu;
-  static PcgHostBuf kept;
+  static std::vector<PcgHostBuf> kept;
+  explicit PcgHost (hipStream_t stream) : st (stream) {}
   int open (int npl)
   {
     int dev = 0;
     SX_HIP (hipGetDevice (&dev));
     {
       std::lock_guard<std::mutex> lock (mu);
-      if (kept.mem && kept.dev == dev) std::swap (b, kept);
+      for (size_t i = 0; i < kept.size (); i++)
+        if (kept[i].dev == dev) {
+          b = kept[i];
+          kept.erase (kept.begin () + i);
+          break;
+        }
     }
+    b.dev = dev;
     if (b.cap < npl) {
       b.drop ();
-      b.dev = dev;
       SX_HIP (hipHostMalloc ((void**) &b.mem, sizeof (int) * 2 * npl, hipHostMallocDefault));
-      b.cap = npl;
       for (hipEvent_t& e : b.ev) SX_HIP (hipEventCreateWithFlags (&e, hipEventDisableTiming));
+      b.cap = npl;                     // complete: may be kept
     }
     for (int i = 0; i < 2; i++) { flags[i] = b.mem + i * b.cap; ev[i] = b.ev[i]; }
     return SX_OK;
   }
+  // after an error copies to the flags may still be queued: wait for them
   ~PcgHost ()
   {
+    if (b.mem && !closed) (void) hipStreamSynchronize (st);
     std::lock_guard<std::mutex> lock (mu);
-    if (!kept.mem) std::swap (b, kept);
-    else b.drop ();
+    bool have = b.cap == 0;
+    for (const PcgHostBuf& k : kept) have = have || k.dev == b.dev;
+    if (have) b.drop ();
+    else kept.push_back (b);
   }
+  bool closed = false;                 // the caller has waited for st
 };
 std::mutex PcgHost::mu;
-PcgHostBuf PcgHost::kept;
+std::vector<PcgHostBuf> PcgHost::kept;
 }  // namespace
 
 extern "C" int sx_field_solve_pcg (sx_msys_t s, int nz, int stride, double* d_f, double* d_u,
@@ -634,7 +646,7 @@ extern "C" int sx_field_solve_pcg (sx_msys_t s, int nz, int stride, double* d_f,
   // find nothing active when those were the last iterations (a wait every
   // four iterations idled the GPU for a quarter of the solve).
   constexpr int GROUP = 4;
-  PcgHost H;
+  PcgHost H (st);
   if (int rc = H.open (npl)) return rc;
   const int regs = (int) ((npts + PV_THREADS - 1) / PV_THREADS);
   auto step = regs <= 2 ? k_pcg_step<2> : regs <= 4 ? k_pcg_step<4> : regs <= 8 ? k_pcg_step<8>
@@ -664,9 +676,9 @@ extern "C" int sx_field_solve_pcg (sx_msys_t s, int nz, int stride, double* d_f,
                       m->d_btog, m->d_bmask, m->d_emask, s->d_G, m->nglobal, ps.x, npts, d_u,
                       stride, nz, s->base_mode);
   SX_HIP (hipGetLastError ());
-  // (the flags' last copy ends before H goes)
   SX_HIP (hipMemcpyAsync (H.flags[0], ps.it, sizeof (int) * npl, hipMemcpyDeviceToHost, st));
   SX_HIP (hipStreamSynchronize (st));
+  H.closed = true;
   if (iters) *iters = *std::max_element (H.flags[0], H.flags[0] + npl);
   return SX_OK;
 }

@@ -206,3 +206,30 @@ def test_held_system_keeps_its_refinement_and_builds_a_band_only_when_asked():
     assert S.stub_live() == 0 and S.stub_bad_pointers() == 0
     print("ok")
     """)
+
+
+def test_pcg_keeps_one_set_of_pinned_flags_a_device():
+    """Solves that alternate between devices allocate no pinned memory after
+    the first on each, and a solve whose events or buffer could not be made
+    leaves nothing half made for the next."""
+    run("""
+    m = rect_mesh(6, 4, 6, 0.0, 6.0, -1.0, 1.0, bc=("D", "N", "D", "N"), periodic_x=True)
+    M = []
+    for d in (0, 1):
+        S.stub_device(d)
+        M.append(ModalMatrixSys(500.0, 1.0, 0, 2, GpuMesh(m), precision=_lib.SX_JACPCG))
+    b = [Buf(4 * m.plane_size) for _ in range(2)]
+    def pcg(i):
+        S.stub_device(i)
+        return L.sx_field_solve_pcg(M[i].handle, 4, m.plane_size, b[0].p, b[1].p, None, 1e-8, 20, None, None)
+    S.stub_fail(0, 0); assert pcg(0) == 0
+    n = S.stub_allocs()                                   # workspace, flags
+    for k in range(n):
+        S.stub_fail(k, 1); rc = pcg(1); S.stub_fail(-1, 0)
+        assert rc == _lib.SX_ERR_HIP and L.sx_last_error()
+    assert pcg(1) == 0
+    S.stub_fail(-1, 0)
+    for i in (0, 1, 0, 1, 1, 0): assert pcg(i) == 0
+    assert S.stub_allocs() == 0
+    print("ok")
+    """)
