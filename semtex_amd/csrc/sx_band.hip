@@ -2288,8 +2288,8 @@ int split_alloc (sx_msys* s, hipStream_t st)
 {
   const size_t rows = (size_t) 2 * s->nmodes * XMAXR;
   s->xch_bytes = rows * SPLIT_ROLES * XR * PB * 16;  // one direction per role
-  SX_HIP (hipMalloc (&s->d_xch, s->xch_bytes));
-  SX_HIP (hipMalloc (&s->d_xep, sizeof (unsigned) * 4));
+  SX_HIP (dev_malloc (&s->d_xch, s->xch_bytes));
+  SX_HIP (dev_malloc (&s->d_xep, sizeof (unsigned) * 4));
   SX_HIP (hipMemsetAsync (s->d_xch, 0, s->xch_bytes, st));
   SX_HIP (hipMemsetAsync (s->d_xep, 0, sizeof (unsigned) * 4, st));
   return SX_OK;
@@ -2467,17 +2467,17 @@ static int band_factor_twisted (sx_msys* s, const std::vector<int>& tw, hipStrea
     nbtm = std::max (nbtm, t[TW_NTOP] / PB);
     nbbm = std::max (nbbm, t[TW_NBOT] / PB);
   }
-  SX_HIP (hipMalloc (&s->d_tw, sizeof (int) * tw.size ()));
+  SX_HIP (dev_malloc (&s->d_tw, sizeof (int) * tw.size ()));
   SX_HIP (hipMemcpy (s->d_tw, tw.data (), sizeof (int) * tw.size (), hipMemcpyHostToDevice));
   DevTmp taux, tR, tV;
-  SX_HIP (hipMalloc (&taux.p, sizeof (int) * aux.size ()));
+  SX_HIP (dev_malloc (&taux.p, sizeof (int) * aux.size ()));
   int* d_aux = (int*) taux.p;
   SX_HIP (hipMemcpy (d_aux, aux.data (), sizeof (int) * aux.size (), hipMemcpyHostToDevice));
   const int *d_ntop = d_aux, *d_nbot = d_aux + nm, *d_nelim = d_aux + 2 * nm;
   const size_t rstride = (size_t) nbbm * PB * ld;
   const size_t vstride = std::max (rstride, s->band_stride);
-  SX_HIP (hipMalloc (&tR.p, sizeof (double) * nm * rstride));
-  SX_HIP (hipMalloc (&tV.p, sizeof (double) * nm * vstride));
+  SX_HIP (dev_malloc (&tR.p, sizeof (double) * nm * rstride));
+  SX_HIP (dev_malloc (&tV.p, sizeof (double) * nm * vstride));
   double *R = (double*) tR.p, *V = (double*) tV.p;
   SX_HIP (hipMemsetAsync (V, 0, sizeof (double) * nm * vstride, st));
   hipLaunchKernelGGL (k_twist_rbuild, dim3 ((unsigned) ((rstride + 255) / 256), nm),
@@ -2498,15 +2498,15 @@ static int band_factor_twisted (sx_msys* s, const std::vector<int>& tw, hipStrea
   s->tw_S = S;
   s->tw_boff = (size_t) (nbtm + 1) * (D + 1) * PB * PB;
   s->sw_stride = s->tw_boff + (size_t) (nbbm + 1) * (D + 1) * PB * PB;
-  SX_HIP (hipMalloc (&s->d_swF, sizeof (double) * nm * s->sw_stride));
-  if (reversed_panels (s)) SX_HIP (hipMalloc (&s->d_swR, sizeof (double) * nm * s->sw_stride));
+  SX_HIP (dev_malloc (&s->d_swF, sizeof (double) * nm * s->sw_stride));
+  if (reversed_panels (s)) SX_HIP (dev_malloc (&s->d_swR, sizeof (double) * nm * s->sw_stride));
   if (int rc = build_panels (s, s->d_bandU, V, s->band_stride, d_ntop, nbtm + 1, 0, st))
     return rc;
   SX_HIP (hipMemsetAsync (V, 0, sizeof (double) * nm * vstride, st));
   if (int rc = build_panels (s, R, V, rstride, d_nbot, nbbm + 1, s->tw_boff, st)) return rc;
   s->nmaxb = nbbm * PB;
   const size_t nb_rhs = (size_t) nm * s->rhs_cap * s->nmaxb;
-  SX_HIP (hipMalloc (&s->d_rhsb, sizeof (double) * nb_rhs));
+  SX_HIP (dev_malloc (&s->d_rhsb, sizeof (double) * nb_rhs));
   SX_HIP (hipMemsetAsync (s->d_rhsb, 0, sizeof (double) * nb_rhs, st));
   SX_HIP (hipStreamSynchronize (st));
   return SX_OK;
@@ -2530,7 +2530,7 @@ int band_factor (sx_msys* s, hipStream_t st, int* d_status)
   DevTmp tV;
   double* V = nullptr;
   if (rev) {
-    SX_HIP (hipMalloc (&tV.p, sizeof (double) * s->nmodes * s->band_stride));
+    SX_HIP (dev_malloc (&tV.p, sizeof (double) * s->nmodes * s->band_stride));
     V = (double*) tV.p;
     SX_HIP (hipMemsetAsync (V, 0, sizeof (double) * s->nmodes * s->band_stride, st));
     hipLaunchKernelGGL (k_band_reverse,
@@ -2545,8 +2545,8 @@ int band_factor (sx_msys* s, hipStream_t st, int* d_status)
       if (int rc = split_alloc (s, st)) return rc;
     s->sw_block = PB;
     s->sw_stride = band_sweep_bytes_per_mode (s->nmax, ld);
-    SX_HIP (hipMalloc (&s->d_swF, sizeof (double) * s->nmodes * s->sw_stride));
-    if (rev) SX_HIP (hipMalloc (&s->d_swR, sizeof (double) * s->nmodes * s->sw_stride));
+    SX_HIP (dev_malloc (&s->d_swF, sizeof (double) * s->nmodes * s->sw_stride));
+    if (rev) SX_HIP (dev_malloc (&s->d_swR, sizeof (double) * s->nmodes * s->sw_stride));
     const double* src[2] = {s->d_bandU, V};
     double* dst[2] = {s->d_swF, s->d_swR};
     // panels 0..nblk (per-mode nb <= nblk; everything past a mode's own
@@ -2575,8 +2575,8 @@ int band_factor (sx_msys* s, hipStream_t st, int* d_status)
   SX_HIP (hipGetLastError ());
   s->sw_block = B;
   s->sw_stride = band_sweep_bytes_per_mode (s->nmax, ld);
-  SX_HIP (hipMalloc (&s->d_swF, sizeof (double) * s->nmodes * s->sw_stride));
-  SX_HIP (hipMalloc (&s->d_swR, sizeof (double) * s->nmodes * s->sw_stride));
+  SX_HIP (dev_malloc (&s->d_swF, sizeof (double) * s->nmodes * s->sw_stride));
+  SX_HIP (dev_malloc (&s->d_swR, sizeof (double) * s->nmodes * s->sw_stride));
   const unsigned gx = (unsigned) ((s->sw_stride + 255) / 256);
   hipLaunchKernelGGL (k_band_blockify, dim3 (gx, s->nmodes), dim3 (256), 0, st,
                       s->d_bandU, s->d_swF, s->band_stride, s->sw_stride, ld, B,

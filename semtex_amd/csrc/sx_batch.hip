@@ -170,7 +170,7 @@ int fused_record (sx_batch* b)
   for (auto& g : P.groups) bytes += al (g.blob.size ()) + al (sizeof (uint2) * g.grid.size ());
   if (b->d_plan) (void) hipFree (b->d_plan);
   b->d_plan = nullptr;
-  SX_HIP (hipMalloc (&b->d_plan, std::max<size_t> (bytes, 256)));
+  SX_HIP (dev_malloc (&b->d_plan, std::max<size_t> (bytes, 256)));
   char* base = (char*) b->d_plan;
   size_t off = 0;
   for (auto& g : P.groups) {

@@ -597,7 +597,7 @@ struct sx_dns {
   double* alloc (size_t cnt)
   {
     double* q = nullptr;
-    if (hipMalloc (&q, sizeof (double) * std::max<size_t> (cnt, 1)) != hipSuccess) return nullptr;
+    if (dev_malloc (&q, sizeof (double) * std::max<size_t> (cnt, 1)) != hipSuccess) return nullptr;
     bufs.push_back (q);
     return q;
   }
@@ -1211,8 +1211,8 @@ extern "C" int sx_dns_create (sx_mesh_t mu, sx_mesh_t mp, int nz, double beta,
         nyv[(size_t) b * np + k] = ny / len;
       }
     }
-    if (hipMalloc (&d->seg_elmt, sizeof (int) * d->nb) || hipMalloc (&d->seg_idx, sizeof (int) * ix.size ()) ||
-        hipMalloc (&d->seg_kind, sizeof (int) * d->nb))
+    if (dev_malloc (&d->seg_elmt, sizeof (int) * d->nb) || dev_malloc (&d->seg_idx, sizeof (int) * ix.size ()) ||
+        dev_malloc (&d->seg_kind, sizeof (int) * d->nb))
       return fail (hip_fail (hipErrorOutOfMemory, "sx_dns_create"));
     if (!(d->seg_nx = d->alloc (nxv.size ())) || !(d->seg_ny = d->alloc (nyv.size ())))
       return fail (hip_fail (hipErrorOutOfMemory, "sx_dns_create"));

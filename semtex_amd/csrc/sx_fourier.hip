@@ -419,7 +419,7 @@ int tables (int nz, Tables** out)
       const long double a = twopi * j / nz;
       h[j] = make_double2 ((double) cosl (a), (double) -sinl (a));
     }
-    SX_HIP (hipMalloc (&t.tw, sizeof (double2) * h.size ()));
+    SX_HIP (sx::dev_malloc (&t.tw, sizeof (double2) * h.size ()));
     SX_HIP (hipMemcpy (t.tw, h.data (), sizeof (double2) * h.size (), hipMemcpyHostToDevice));
   }
   if (!pow2_fft (nz) && !t.Cf) {
@@ -440,8 +440,8 @@ int tables (int nz, Tables** out)
         Ci[(size_t) n * nz + 2 * k + 1] = -2.0 * s;
       }
     }
-    SX_HIP (hipMalloc (&t.Cf, sizeof (double) * Cf.size ()));
-    SX_HIP (hipMalloc (&t.Ci, sizeof (double) * Ci.size ()));
+    SX_HIP (sx::dev_malloc (&t.Cf, sizeof (double) * Cf.size ()));
+    SX_HIP (sx::dev_malloc (&t.Ci, sizeof (double) * Ci.size ()));
     SX_HIP (hipMemcpy (t.Cf, Cf.data (), sizeof (double) * Cf.size (), hipMemcpyHostToDevice));
     SX_HIP (hipMemcpy (t.Ci, Ci.data (), sizeof (double) * Ci.size (), hipMemcpyHostToDevice));
   }

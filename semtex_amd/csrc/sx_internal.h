@@ -37,12 +37,18 @@ inline int lds_limit (const void* kern, size_t lds)
 // Device blocks of systems and their set-up kept for the next ones: unmapping
 // and mapping one costs 2-6 us a MB, which bounded the making of a system
 // (a changed time step or lambda2).  At most POOL_BYTES in POOL_BLOCKS blocks
-// a device; given back when a device runs out of memory and when the last
-// mesh goes.  block_free: nothing on the GPU uses the block any more (the
-// caller has waited, as hipFree itself would); dev: the device it was
-// allocated on.
+// a device; given back when an allocation of this library fails on it
+// (dev_malloc, which every one goes through; another allocator of the process
+// finds at most POOL_BYTES taken) and when the last mesh goes.  block_free:
+// nothing on the GPU uses the block any more (the caller has waited, as
+// hipFree itself would); dev: the device it was allocated on.
 constexpr size_t POOL_BYTES = (size_t) 512 << 20;
 constexpr int POOL_BLOCKS = 8;
+hipError_t dev_malloc_bytes (void** p, size_t bytes);
+template <typename T> hipError_t dev_malloc (T** p, size_t bytes)
+{
+  return dev_malloc_bytes ((void**) p, bytes);
+}
 int  block_alloc (void** p, size_t bytes, size_t* size, int* dev);
 void block_free (void* p, size_t size, int dev);
 void block_meshes (int delta);

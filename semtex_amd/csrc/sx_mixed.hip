@@ -440,7 +440,7 @@ int plan_mixed_passes (BatchPlan& P, sx_msys* s, int nz, int stride, double* d_f
     if (s->d_work) (void) hipFree (s->d_work);
     s->d_work = nullptr;
     s->work_doubles = 0;
-    SX_HIP (hipMalloc (&s->d_work, sizeof (double) * need));
+    SX_HIP (dev_malloc (&s->d_work, sizeof (double) * need));
     s->work_doubles = need;
   }
   double *W = s->d_work, *X = W + nplane, *Fp = X + nplane, *V = Fp + nplane,
@@ -492,7 +492,7 @@ int field_solve_mixed_passes (sx_msys* s, int nz, int stride, double* d_f, doubl
     if (s->d_work) (void) hipFree (s->d_work);
     s->d_work = nullptr;
     s->work_doubles = 0;
-    SX_HIP (hipMalloc (&s->d_work, sizeof (double) * need));
+    SX_HIP (dev_malloc (&s->d_work, sizeof (double) * need));
     s->work_doubles = need;
   }
   double *W = s->d_work, *X = W + nplane, *Fp = X + nplane, *V = Fp + nplane,
@@ -617,7 +617,7 @@ extern "C" int sx_field_solve_mixed (sx_msys_t s, int nz, int stride, double* d_
     if (s->d_work) (void) hipFree (s->d_work);
     s->d_work = nullptr;
     s->work_doubles = 0;
-    SX_HIP (hipMalloc (&s->d_work, sizeof (double) * need));
+    SX_HIP (dev_malloc (&s->d_work, sizeof (double) * need));
     s->work_doubles = need;
   }
   return field_solve_mixed_ws (s, nz, stride, d_f, d_u, d_lines, refine_tol, max_iter, iters,

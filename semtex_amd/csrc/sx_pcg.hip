@@ -498,8 +498,8 @@ int pcg_setup (sx_msys* s, hipStream_t st)
   const size_t npts = (size_t) m->nglobal + (size_t) m->nel * m->nint;
   const size_t lstride = (size_t) m->nel * m->npnp;
   double* L = nullptr;
-  SX_HIP (hipMalloc (&s->d_pc, sizeof (double) * s->nmodes * npts));
-  SX_HIP (hipMalloc (&L, sizeof (double) * s->nmodes * lstride));
+  SX_HIP (dev_malloc (&s->d_pc, sizeof (double) * s->nmodes * npts));
+  SX_HIP (dev_malloc (&L, sizeof (double) * s->nmodes * lstride));
   hipLaunchKernelGGL (k_pcg_elem_diag, dim3 (m->nel, s->nmodes), dim3 (64), 0, st, m->np,
                       m->cyl, s->lambda2, s->d_betak2, m->d_geo, m->d_D, m->d_emap, L,
                       lstride);
@@ -605,7 +605,7 @@ extern "C" int sx_field_solve_pcg (sx_msys_t s, int nz, int stride, double* d_f,
     if (s->d_work) (void) hipFree (s->d_work);
     s->d_work = nullptr;
     s->work_doubles = 0;
-    SX_HIP (hipMalloc (&s->d_work, sizeof (double) * need));
+    SX_HIP (dev_malloc (&s->d_work, sizeof (double) * need));
     s->work_doubles = need;
   }
   double* L = s->d_work;

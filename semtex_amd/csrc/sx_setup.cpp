@@ -209,7 +209,7 @@ template <typename T>
 static int upload (T** dst, const std::vector<T>& src)
 {
   const size_t n = std::max<size_t> (src.size (), 1);
-  SX_HIP (hipMalloc ((void**) dst, n * sizeof (T)));
+  SX_HIP (dev_malloc (dst, n * sizeof (T)));
   if (!src.empty ())
     SX_HIP (hipMemcpy (*dst, src.data (), src.size () * sizeof (T),
                        hipMemcpyHostToDevice));
@@ -237,6 +237,22 @@ void pool_flush (std::vector<Block>& gone, int dev)     // dev < 0: every device
 
 namespace sx {
 
+hipError_t dev_malloc_bytes (void** p, size_t bytes)
+{
+  hipError_t e = hipMalloc (p, bytes);
+  if (e == hipSuccess) return e;
+  std::vector<Block> gone;
+  int dev = 0;
+  if (hipGetDevice (&dev) == hipSuccess) {
+    std::lock_guard<std::mutex> lock (pool_mu);
+    pool_flush (gone, dev);
+  }
+  for (const Block& b : gone) (void) hipFree (b.p);
+  if (gone.empty ()) return e;
+  (void) hipGetLastError ();
+  return hipMalloc (p, bytes);
+}
+
 int block_alloc (void** p, size_t bytes, size_t* size, int* device)
 {
   int dev = 0;
@@ -257,19 +273,7 @@ int block_alloc (void** p, size_t bytes, size_t* size, int* device)
     }
   }
   *size = bytes;
-  hipError_t e = hipMalloc (p, bytes);
-  if (e != hipSuccess) {
-    std::vector<Block> gone;
-    {
-      std::lock_guard<std::mutex> lock (pool_mu);
-      pool_flush (gone, dev);
-    }
-    for (const Block& b : gone) (void) hipFree (b.p);
-    if (!gone.empty ()) {
-      (void) hipGetLastError ();
-      e = hipMalloc (p, bytes);
-    }
-  }
+  const hipError_t e = dev_malloc (p, bytes);
   return e == hipSuccess ? (int) SX_OK : hip_fail (e, "hipMalloc");
 }
 

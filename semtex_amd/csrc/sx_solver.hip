@@ -1746,7 +1746,7 @@ static int band_build (sx_msys* s, const double* d_S, hipStream_t st, int* d_sta
 {
   const sx_mesh* m = s->m;
   const size_t nb = sizeof (double) * s->nmodes * s->band_stride;
-  SX_HIP (hipMalloc (&s->d_bandU, nb));
+  SX_HIP (dev_malloc (&s->d_bandU, nb));
   SX_HIP (hipMemsetAsync (s->d_bandU, 0, nb, st));
   if (m->npairs)
     hipLaunchKernelGGL (k_band_assemble, dim3 ((m->npairs + 255) / 256, s->nmodes), dim3 (256), 0,
@@ -1767,7 +1767,7 @@ int Grow::add (double** at, size_t doubles)
 {
   double* p = nullptr;
   const size_t bytes = sizeof (double) * std::max<size_t> (doubles, 1);
-  SX_HIP (hipMalloc (&p, bytes));
+  SX_HIP (dev_malloc (&p, bytes));
   items.push_back ({at, p});
   SX_HIP (hipMemset (p, 0, bytes));
   return SX_OK;
@@ -1800,7 +1800,7 @@ static int condensed_again (const sx_msys* s, DevTmp& buf, double** S, int** d_s
   const size_t nmc = (size_t) s->nmodes * m->nclass;
   const size_t nws = nmc * ((size_t) npnp * npnp + (size_t) nint * nint), nS = nmc * next * next,
                nB = nmc * next * nint, nH = nmc * nint * nint, nd = nws + nS + nB + nH;
-  SX_HIP (hipMalloc (&buf.p, sizeof (double) * (nd + s->nmodes + 1)));
+  SX_HIP (dev_malloc (&buf.p, sizeof (double) * (nd + s->nmodes + 1)));
   double* d = (double*) buf.p;
   *S = d + nws;
   *d_status = (int*) (d + nd);
@@ -1936,11 +1936,11 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
 #define TRY(call) do { hipError_t _e = (call); if (_e != hipSuccess) return fail (hip_fail (_e, #call)); } while (0)
   const size_t nmc = (size_t) num_modes * m->nclass;
   if (precision == SX_JACPCG) {      // MatrixSys JACPCG: the preconditioner only
-    TRY (hipMalloc (&s->d_betak2, sizeof (double) * num_modes));
-    TRY (hipMalloc (&s->d_nsolve, sizeof (int) * num_modes));
+    TRY (dev_malloc (&s->d_betak2, sizeof (double) * num_modes));
+    TRY (dev_malloc (&s->d_nsolve, sizeof (int) * num_modes));
     TRY (hipMemcpy (s->d_betak2, s->betak2.data (), sizeof (double) * num_modes, hipMemcpyHostToDevice));
     TRY (hipMemcpy (s->d_nsolve, s->nsolve.data (), sizeof (int) * num_modes, hipMemcpyHostToDevice));
-    TRY (hipMalloc (&s->d_G, sizeof (double) * 2 * num_modes * m->nglobal));
+    TRY (dev_malloc (&s->d_G, sizeof (double) * 2 * num_modes * m->nglobal));
     if ((rc = pcg_setup (s, st))) return fail (rc);
     *out = s;
     return SX_OK;
@@ -1956,52 +1956,74 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
   const TileShape R = rec_shape (m->np, s->tile_mf), Cs = con_shape (m->np, s->tile_mf);
   const size_t nrec = tiled ? (size_t) R.KR * R.NA : 0, ncon = tiled ? (size_t) Cs.KR * Cs.NA : 0;
   const size_t nrhs = (size_t) num_modes * 2;
-  size_t n = 0;
   auto take = [] (size_t& at, size_t doubles) {
     const size_t o = at;
     at += (std::max<size_t> (doubles, 1) + 31) / 32 * 32;
     return o;
   };
-  const size_t o_rhs = take (n, nrhs * std::max (s->nmax, 1));
-  const size_t o_tb = take (n, s->tree ? nrhs * m->nsolve : 0),
-               o_tc = take (n, s->tree ? nrhs * tree_slots (s->tree) : 0), nzero = n;
-  const size_t o_par = take (n, 2 * (size_t) num_modes), o_G = take (n, nrhs * m->nglobal),
-               o_Bm = take (n, nmc * next * nint), o_Hi = take (n, nmc * nint * nint),
-               o_rec = take (n, nmc * nrec), o_con = take (n, nmc * ncon),
-               o_tv = take (n, s->tree ? nrhs * m->nsolve : 0),
-               o_ops = take (n, s->tree ? tree_ops (s->tree) * num_modes : 0);
-  if ((rc = block_alloc ((void**) &s->block, sizeof (double) * n, &s->block_bytes, &s->block_dev)))
-    return fail (rc);
-  double* base = (double*) s->block;
-  s->d_rhs = base + o_rhs;
-  s->d_betak2 = base + o_par;
-  s->d_nsolve = (int*) (s->d_betak2 + num_modes);
-  s->d_G = base + o_G;
-  s->d_Bm = base + o_Bm;
-  s->d_Hinv = base + o_Hi;
-  if (tiled) {
-    s->d_Mrec = base + o_rec;
-    s->d_Mcon = base + o_con;
+  const size_t ws_per = (size_t) npnp * npnp + (size_t) nint * nint;
+  size_t nzero = 0, o_st = 0, o_ws = 0, o_S = 0, o_f = 0;
+  auto reserve = [&] () -> int {
+    size_t n = 0, nt = 0;
+    const size_t o_rhs = take (n, nrhs * std::max (s->nmax, 1));
+    const size_t o_tb = take (n, s->tree ? nrhs * m->nsolve : 0),
+                 o_tc = take (n, s->tree ? nrhs * tree_slots (s->tree) : 0);
+    nzero = n;
+    const size_t o_par = take (n, 2 * (size_t) num_modes), o_G = take (n, nrhs * m->nglobal),
+                 o_Bm = take (n, nmc * next * nint), o_Hi = take (n, nmc * nint * nint),
+                 o_rec = take (n, nmc * nrec), o_con = take (n, nmc * ncon),
+                 o_tv = take (n, s->tree ? nrhs * m->nsolve : 0),
+                 o_ops = take (n, s->tree ? tree_ops (s->tree) * num_modes : 0);
+    o_st = take (nt, num_modes + 1);
+    o_ws = take (nt, nmc * ws_per);
+    o_S = take (nt, nmc * next * next);
+    o_f = take (nt, s->tree ? tree_scratch (s->tree, num_modes) : 0);
+    void* p = nullptr;
+    size_t bytes = 0;
+    int dev = 0, e;
+    if ((e = block_alloc (&p, sizeof (double) * n, &bytes, &dev))) return e;
+    if ((e = block_alloc ((void**) &d_ws, sizeof (double) * nt, &ws_bytes, &ws_dev))) {
+      d_ws = nullptr;
+      (void) hipFree (p);
+      return e;
+    }
+    s->block = (char*) p;
+    s->block_bytes = bytes;
+    s->block_dev = dev;
+    double* base = (double*) p;
+    s->d_rhs = base + o_rhs;
+    s->d_betak2 = base + o_par;
+    s->d_nsolve = (int*) (s->d_betak2 + num_modes);
+    s->d_G = base + o_G;
+    s->d_Bm = base + o_Bm;
+    s->d_Hinv = base + o_Hi;
+    if (tiled) {
+      s->d_Mrec = base + o_rec;
+      s->d_Mcon = base + o_con;
+    }
+    if (s->tree) {
+      s->d_tb = base + o_tb;
+      s->d_tc = base + o_tc;
+      s->d_tv = base + o_tv;
+      s->d_tops = base + o_ops;
+    }
+    return SX_OK;
+  };
+  rc = reserve ();
+  if (rc && s->tree) {
+    // the operators and the fronts do not fit the device: a band factor is a
+    // part of their size (graded meshes, many modes)
+    s->tree = nullptr;
+    rc = reserve ();
   }
-  if (s->tree) {
-    s->d_tb = base + o_tb;
-    s->d_tc = base + o_tc;
-    s->d_tv = base + o_tv;
-    s->d_tops = base + o_ops;
-  }
-  TRY (hipMemsetAsync (base, 0, sizeof (double) * nzero, st));
+  if (rc) return fail (rc);
+  TRY (hipMemsetAsync (s->block, 0, sizeof (double) * nzero, st));
   std::vector<double> par (s->betak2);
   par.resize (2 * (size_t) num_modes);
   std::memcpy (par.data () + num_modes, s->nsolve.data (), sizeof (int) * num_modes);
   TRY (hipMemcpyAsync (s->d_betak2, par.data (), sizeof (double) * par.size (),
                        hipMemcpyHostToDevice, st));
 
-  const size_t ws_per = (size_t) npnp * npnp + (size_t) nint * nint;
-  size_t nt = 0;
-  const size_t o_st = take (nt, num_modes + 1), o_ws = take (nt, nmc * ws_per),
-               o_S = take (nt, nmc * next * next),
-               o_f = take (nt, s->tree ? tree_scratch (s->tree, num_modes) : 0);
-  if ((rc = block_alloc ((void**) &d_ws, sizeof (double) * nt, &ws_bytes, &ws_dev))) return fail (rc);
   double* d_S = d_ws + o_S;
   int* d_status = (int*) (d_ws + o_st);
   TRY (hipMemsetAsync (d_status, 0, sizeof (int) * (num_modes + 1), st));
@@ -2039,8 +2061,8 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
   if (precision == SX_MIXED && s->tile_mf) {
     const TileShape R = rec_shape (m->np, true), Cs = con_shape (m->np, true);
     const size_t nr = nmc * R.KR * R.NA, nc = nmc * Cs.KR * Cs.NA;
-    TRY (hipMalloc (&s->d_Mrec32, sizeof (float) * nr));
-    TRY (hipMalloc (&s->d_Mcon32, sizeof (float) * nc));
+    TRY (dev_malloc (&s->d_Mrec32, sizeof (float) * nr));
+    TRY (dev_malloc (&s->d_Mcon32, sizeof (float) * nc));
     hipLaunchKernelGGL (k_ops32, dim3 ((unsigned) std::min<size_t> ((nr + 255) / 256, 65535)),
                         dim3 (256), 0, st, s->d_Mrec, s->d_Mrec32, nr);
     hipLaunchKernelGGL (k_ops32, dim3 ((unsigned) std::min<size_t> ((nc + 255) / 256, 65535)),
@@ -2048,8 +2070,8 @@ extern "C" int sx_msys_create_named (sx_mesh_t m, double lambda2, double beta,
     TRY (hipGetLastError ());
   }
   if (precision == SX_MIXED) {
-    TRY (hipMalloc (&s->d_Bm32, sizeof (float) * std::max<size_t> (nmc * next * nint, 1)));
-    TRY (hipMalloc (&s->d_Hinv32, sizeof (float) * std::max<size_t> (nmc * nint * nint, 1)));
+    TRY (dev_malloc (&s->d_Bm32, sizeof (float) * std::max<size_t> (nmc * next * nint, 1)));
+    TRY (dev_malloc (&s->d_Hinv32, sizeof (float) * std::max<size_t> (nmc * nint * nint, 1)));
     const size_t n1 = nmc * next * nint, n2 = nmc * nint * nint;
     if (n1) hipLaunchKernelGGL (k_to_f32, dim3 ((unsigned) ((n1 + 255) / 256)), dim3 (256), 0, st, s->d_Bm, s->d_Bm32, n1);
     if (n2) hipLaunchKernelGGL (k_to_f32, dim3 ((unsigned) ((n2 + 255) / 256)), dim3 (256), 0, st, s->d_Hinv, s->d_Hinv32, n2);
@@ -2658,12 +2680,12 @@ extern "C" int sx_field_solve_host (sx_msys_t s, int nz, int stride, const doubl
   const size_t nb = sizeof (double) * (size_t) nz * stride;
   const size_t lb = sizeof (double) * (size_t) nz * s->m->nbound * s->m->np;
   double *df = nullptr, *du = nullptr, *dl = nullptr;
-  SX_HIP (hipMalloc (&df, nb));
-  SX_HIP (hipMalloc (&du, nb));
+  SX_HIP (dev_malloc (&df, nb));
+  SX_HIP (dev_malloc (&du, nb));
   SX_HIP (hipMemcpy (df, f, nb, hipMemcpyHostToDevice));
   SX_HIP (hipMemcpy (du, u, nb, hipMemcpyHostToDevice));
   if (lines && lb) {
-    SX_HIP (hipMalloc (&dl, lb));
+    SX_HIP (dev_malloc (&dl, lb));
     SX_HIP (hipMemcpy (dl, lines, lb, hipMemcpyHostToDevice));
   }
   rc = sx_field_solve (s, nz, stride, df, du, dl, nullptr);

@@ -547,7 +547,7 @@ template <typename V> int upload (V** d, const std::vector<V>& h)
 {
   if (*d || h.empty ()) return SX_OK;
   V* p = nullptr;
-  SX_HIP (hipMalloc (&p, sizeof (V) * h.size ()));
+  SX_HIP (dev_malloc (&p, sizeof (V) * h.size ()));
   const hipError_t e = hipMemcpy (p, h.data (), sizeof (V) * h.size (), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     (void) hipFree (p);
@@ -869,7 +869,7 @@ int tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_status
       (rc = G.add (&now.tb, n * t->P.nsolve)) || (rc = G.add (&now.tv, n * t->P.nsolve)) ||
       (rc = G.add (&now.tc, n * t->P.slots)))
     return rc;
-  SX_HIP (hipMalloc (&buf.p, sizeof (double) * tree_scratch (t, s->nmodes)));
+  SX_HIP (dev_malloc (&buf.p, sizeof (double) * tree_scratch (t, s->nmodes)));
   // (the arrays are now's once installed)
   if ((rc = factor (t, s->m, s->nmodes, s->d_nsolve, Sel, G.items[0].p, (double*) buf.p, st,
                     d_status)))
@@ -896,8 +896,8 @@ int tree_sing_setup (sx_msys* s, const double* Sel, hipStream_t st, int* d_statu
     // (the scratch is the later workspace's allocation g->val: entries past
     // the matrix's are free once the factor is done)
     const size_t nb = std::max<size_t> (tree_scratch (t, 1), m->npairs);
-    SX_HIP (hipMalloc (&g->ops, sizeof (double) * std::max<size_t> (t->P.ops, 2)));
-    SX_HIP (hipMalloc (&g->val, sizeof (double) * nb));
+    SX_HIP (dev_malloc (&g->ops, sizeof (double) * std::max<size_t> (t->P.ops, 2)));
+    SX_HIP (dev_malloc (&g->val, sizeof (double) * nb));
     if (int rc = factor (t, m, 1, s->d_nsolve + md, S, g->ops, g->val, st, d_status + md)) return rc;
     if (int rc = sing_rows (m)) return rc;
     hipLaunchKernelGGL (k_tree_entries, dim3 ((m->npairs + 255) / 256), dim3 (256), 0, st,

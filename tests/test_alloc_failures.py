@@ -42,6 +42,12 @@ PRELUDE = textwrap.dedent("""
     def reserve(M, nr): return L._ZN2sx16msys_reserve_rhsEP7sx_msysi(M.handle, nr)
     def solve_nr(M, nr): return L._ZN2sx10tree_solveEPK7sx_msysiP12ihipStream_t(M.handle, nr, None)
 
+    def drain():                     # the blocks kept of earlier systems, given back
+        S.stub_fail(0, 2)
+        try: GpuMesh(rect_mesh(2, 2, 4))
+        except _lib.SxError: pass
+        S.stub_fail(-1, 0)
+
     class RawBatch:
         def __init__(self, Ms, nz=1):
             n = len(Ms)
@@ -92,6 +98,7 @@ def test_failed_reservation_keeps_the_reserved_count():
         m = rect_mesh(12, 10, 6, 0.0, 6.0, -1.0, 1.0, bc=bc, periodic_x=True)
         M = ModalMatrixSys(0.0, 1.0, 0, 4, GpuMesh(m))
         assert M.layout()["operators"] > 0
+        drain()
         k = 0
         while True:
             held = S.stub_bytes()
@@ -138,6 +145,7 @@ def test_failed_batch_leaves_its_systems_as_they_were(bc):
     total = S.stub_allocs()
     B2.destroy(); B2.free()
     del Ms2
+    drain()
     assert [w[2][4] > 0 for w in was] == [True, True] and total > 4
     assert all(w[1] == ("{bc}" == "NNNN") for w in was)
     k = 0
@@ -231,5 +239,63 @@ def test_pcg_keeps_one_set_of_pinned_flags_a_device():
     S.stub_fail(-1, 0)
     for i in (0, 1, 0, 1, 1, 0): assert pcg(i) == 0
     assert S.stub_allocs() == 0
+    print("ok")
+    """)
+
+
+def test_system_whose_dissection_does_not_fit_solves_by_band():
+    """With memory for the band but not for the operators and fronts of a mesh
+    graded both ways, the system is made and solves by band sweeps."""
+    run("""
+    t = lambda n: 0.6 * np.linspace(0, 1, n + 1) + 0.4 * np.linspace(0, 1, n + 1) ** 2
+    m = rect_mesh(16, 16, 6, 0.0, 6.0, -1.0, 1.0, bc=("D", "N", "D", "N"), periodic_x=True,
+                  xs=6 * t(16), ys=t(16))
+    g = GpuMesh(m)
+    M = ModalMatrixSys(1.0, 1.0, 0, 16, g)
+    ops = M.layout()["operators"] * 16 * 8
+    assert ops > 0
+    del M
+    drain()
+    own = S.stub_bytes()
+    hi, lo = own + 4 * ops, own
+    while hi - lo > 1 << 20:                  # the least memory a system is made in
+        mid = (lo + hi) // 2
+        S.stub_limit(mid)
+        try:
+            M = ModalMatrixSys(1.0, 1.0, 0, 16, g)
+            hi, kernel = mid, M.layout()["operators"]
+            del M
+        except _lib.SxError:
+            lo = mid
+        S.stub_limit(0)
+        drain()
+    assert kernel == 0
+    S.stub_limit(hi)
+    M = ModalMatrixSys(1.0, 1.0, 0, 16, g)
+    S.stub_limit(0)
+    assert own_solve(M, 32) == 0 and M.layout()["kernel"] in (1, 2, 3)
+    del M, g
+    assert S.stub_live() == 0 and S.stub_bad_pointers() == 0
+    print("ok")
+    """)
+
+
+def test_kept_blocks_make_room_for_any_allocation():
+    """Blocks kept of systems that went are given back when an allocation that
+    is not a system's block (a mesh, FP32 operators, a solve's workspace)
+    does not fit beside them."""
+    run("""
+    big = rect_mesh(16, 12, 8, 0.0, 6.0, -1.0, 1.0, bc=("D", "N", "D", "N"), periodic_x=True)
+    g = GpuMesh(big)
+    empty = S.stub_bytes()
+    M = ModalMatrixSys(1.0, 1.0, 0, 8, g); del M
+    kept = S.stub_bytes() - empty
+    assert kept > 1 << 20
+    S.stub_limit(S.stub_bytes() + 1000)
+    g2 = GpuMesh(rect_mesh(8, 6, 6, bc=("D", "N", "D", "N")))
+    S.stub_limit(0)
+    assert S.stub_bytes() < empty + kept
+    del g, g2
+    assert S.stub_live() == 0
     print("ok")
     """)
