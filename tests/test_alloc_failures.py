@@ -194,8 +194,8 @@ def test_held_system_keeps_its_refinement_and_builds_a_band_only_when_asked():
     B.destroy(); B.free(); del M, B
     # the band factor does not fit: the dissection, and nothing kept
     M, B = held(16, 12, 8, "NNNN", periodic_x=True)
+    drain()
     bytes_, r = S.stub_bytes(), launches("k_tree_residual")
-    k = 0
     b = [Buf(M.gmesh.plane_size) for _ in range(2)]
     S.stub_fail(0, 1 << 30)
     assert L.sx_field_solve(M.handle, 1, M.gmesh.plane_size, b[0].p, b[1].p, None, None) == 0
