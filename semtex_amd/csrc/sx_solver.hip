@@ -193,10 +193,10 @@ __global__ __launch_bounds__(256) void k_elem_sc (
 }
 
 // The same with the interior block in LDS, inverted there by blocked
-// Gauss-Jordan on FP64 MFMA tiles (spd_invert): up to N_P = 12, whose block
-// (112 x 114 doubles with its padding) is the largest that fits.  k_elem_sc
-// walks its columns through global memory, three barriers each: 184 us at
-// N_P = 8, 645 us at N_P = 10.
+// Gauss-Jordan on FP64 MFMA tiles (spd_invert): up to N_P = 12, the largest
+// measured (N_P = 13, 161 KB of the 164, would be the last that fits).
+// k_elem_sc walks its columns through global memory, three barriers each:
+// 184 us at N_P = 8, 645 us at N_P = 10.
 constexpr int ESC_NPMAX = 12;
 size_t esc_lds (int np)
 {

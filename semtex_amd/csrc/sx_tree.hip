@@ -589,9 +589,10 @@ static bool band_forced ()
 
 // The band solve stays for systems outside the dissection's bounds: bands
 // past 768 (refused as before by the band solve), a mesh tree_plan does not
-// suit, and operators of more than 24 GB.  always: also under a variable
+// suit, operators of more than 24 GB, and more classes than a grid holds.  always: also under a variable
 // that chooses a band layout.
 constexpr size_t TREE_OPS_MAX = (size_t) 3 << 30;      // doubles
+constexpr int TREE_GRID_MAX = 65535;   // classes and modes are y and z of the set-up's grids
 // More than TREE_FEW_MODES modes: also where the band solve is estimated
 // faster (up to 32 modes its twisted and split sweeps lost everywhere
 // measured; with many its chain costs little next to the fronts' many
@@ -615,8 +616,13 @@ int tree_prepare (sx_mesh* m, int nmodes, TreeDev** out, bool always, int share)
     m->trees.push_back (t);
     size_t f = 0;
     t->ok = tree_plan (m, nmodes, share, t->P);
-    for (const TreeLevel& L : t->P.lev) f = std::max (f, L.fsize);
-    t->ok = t->ok && t->P.ops * nmodes <= TREE_OPS_MAX && f * nmodes <= TREE_OPS_MAX;
+    int ncls = 0;
+    for (const TreeLevel& L : t->P.lev) {
+      f = std::max (f, L.fsize);
+      ncls = std::max (ncls, L.ncls);
+    }
+    t->ok = t->ok && t->P.ops * nmodes <= TREE_OPS_MAX && f * nmodes <= TREE_OPS_MAX &&
+            ncls <= TREE_GRID_MAX && nmodes <= TREE_GRID_MAX;
     if (!t->ok) t->P = TreePlan ();
     t->slower = nmodes > TREE_FEW_MODES && band_us (m, nmodes) < TREE_BAND * t->P.est_us;
   }
@@ -853,8 +859,9 @@ int tree_factor (sx_msys* s, const double* Sel, double* buf, hipStream_t st, int
 
 int tree_for_batch (sx_msys* s, const double* Sel, hipStream_t st, int* d_status, Held& h)
 {
-  // (64 uneven problems: 309 us at 4, 318 at 8, 359 at 32, 360 with the
-  // systems' own cuts)
+  // (64 uneven problems of one mode: 309 us at 4, 318 at 8, 359 at 32, 360
+  // with the systems' own cuts.  Systems of 4 and more modes keep their own:
+  // batches of those were not measured)
   constexpr int BATCH_SHARE = 4;
   TreeDev* t = nullptr;
   if (int rc = tree_prepare (s->m, s->nmodes, &t, true, std::max (1, BATCH_SHARE / s->nmodes)))

@@ -1,6 +1,6 @@
 """Dealiased products on k_zmat's edges -- planes whose 3/2 grid ends inside a
 16-row block or past a staging chunk of 96 k rows, and the library products
-kept past 256 planes -- against the oracle's dealiased step, velocity to the
+kept past 128 planes -- against the oracle's dealiased step, velocity to the
 FP64 DNS bar of test_gpu_dns.py (1e-11 after two steps)."""
 import numpy as np
 import pytest
