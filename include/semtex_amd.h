@@ -211,8 +211,10 @@ int sx_field_solve_pcg (sx_msys_t s, int nz, int plane_stride, double* d_f, doub
  * buffers must not overlap; problems that share a system run in order.
  * The recorded solves use no split band sweeps (they need their whole grid
  * resident at once); sx_field_solve on the same systems outside the batch
- * keeps them.  No reference counterpart: for callers that
- * solve many independent small problems (uneven batches). */
+ * keeps them where the system's band layout has them, and is the recorded
+ * solve elsewhere.  A creation that fails leaves the systems as they were.
+ * No reference counterpart: for callers that solve many independent small
+ * problems (uneven batches). */
 typedef struct sx_batch* sx_batch_t;
 int sx_batch_create (int n, const sx_msys_t* systems, const int* nz, const int* plane_stride,
                      const double* const* d_f_src, double* const* d_f_work, double* const* d_u,
