@@ -1689,13 +1689,19 @@ extern "C" int sx_msys_destroy (sx_msys_t s)
   for (void* p : ptrs) msys_free (s, p);
   if (s->block) {
     // the block may serve another system at once: wait for the device, as
-    // freeing it would
+    // freeing it would.  Where that cannot be waited for (a capture in
+    // progress, an error) it is not kept
     int dev = 0;
-    (void) hipGetDevice (&dev);
-    if (dev != s->block_dev) (void) hipSetDevice (s->block_dev);
-    (void) hipDeviceSynchronize ();
+    bool idle = hipGetDevice (&dev) == hipSuccess &&
+                (dev == s->block_dev || hipSetDevice (s->block_dev) == hipSuccess);
+    idle = idle && hipDeviceSynchronize () == hipSuccess;
     if (dev != s->block_dev) (void) hipSetDevice (dev);
-    block_free (s->block, s->block_bytes, s->block_dev);
+    if (idle) {
+      block_free (s->block, s->block_bytes, s->block_dev);
+    } else {
+      (void) hipFree (s->block);
+      (void) hipGetLastError ();
+    }
   }
   tree_sing_free (s->sing);
   delete s;

@@ -17,6 +17,7 @@ std::map<void*, size_t> live;               // device and pinned allocations
 std::map<const void*, std::string> names;   // kernel stub -> device name
 std::map<std::string, long> launched;
 long allocs = 0, fail_at = -1, fail_to = -1, device = 0, bad = 0;
+bool sync_fails = false;
 size_t limit = 0;                           // bytes on the "device" (0: no limit)
 hipError_t last = hipSuccess;
 
@@ -53,6 +54,7 @@ extern "C" {
 void stub_fail (long first, long count) { allocs = 0; fail_at = first; fail_to = first + count; }
 void stub_limit (size_t bytes) { limit = bytes; }
 void stub_device (long d) { device = d; }
+void stub_sync_fails (int on) { sync_fails = on != 0; }
 long stub_allocs () { return allocs; }
 long stub_live () { return (long) live.size (); }
 size_t stub_bytes () { size_t n = 0; for (auto& a : live) n += a.second; return n; }
@@ -74,7 +76,7 @@ hipError_t hipMemsetAsync (void* d, int v, size_t n, hipStream_t) { std::memset 
 hipError_t hipGetDevice (int* d) { *d = (int) device; return hipSuccess; }
 hipError_t hipSetDevice (int d) { device = d; return hipSuccess; }
 hipError_t hipGetDeviceCount (int* n) { *n = 2; return hipSuccess; }
-hipError_t hipDeviceSynchronize () { return hipSuccess; }
+hipError_t hipDeviceSynchronize () { return sync_fails ? ret (hipErrorStreamCaptureUnsupported) : hipSuccess; }
 hipError_t hipDeviceGetAttribute (int* v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
 hipError_t hipGetDevicePropertiesR0600 (hipDeviceProp_tR0600* p, int)
 {

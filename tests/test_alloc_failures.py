@@ -299,3 +299,23 @@ def test_kept_blocks_make_room_for_any_allocation():
     assert S.stub_live() == 0
     print("ok")
     """)
+
+
+def test_block_that_may_be_in_use_is_not_kept():
+    """A system destroyed while the device cannot be waited for (during a
+    capture) gives its block back instead of handing it to the next system."""
+    run("""
+    g = GpuMesh(rect_mesh(8, 6, 6, bc=("D", "N", "D", "N")))
+    M = ModalMatrixSys(1.0, 1.0, 0, 4, g)
+    drain()
+    held = S.stub_bytes()
+    S.stub_sync_fails(1); del M; S.stub_sync_fails(0)
+    after = S.stub_bytes()
+    drain()
+    assert after < held and S.stub_bytes() == after       # nothing of it was kept
+    M = ModalMatrixSys(1.0, 1.0, 0, 4, g)
+    assert own_solve(M, 8) == 0                           # and no error was left behind
+    del M, g
+    assert S.stub_live() == 0
+    print("ok")
+    """)
