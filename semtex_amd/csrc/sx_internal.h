@@ -179,7 +179,7 @@ constexpr int MIXED_NBLK = 256;     // workgroups of the correction-norm reducti
 size_t mixed_work_doubles (const sx_msys* s, int nz, int stride);
 int    field_solve_mixed_ws (sx_msys* s, int nz, int stride, double* d_f, double* d_u,
                              const double* d_lines, double refine_tol, int max_iter,
-                             int* iters, double* work, hipStream_t st);
+                             int* iters, double* work, hipStream_t st, bool build = true);
 int    check_mixed_solve_args (sx_msys* s, int nz, int stride, const void* f, const void* u,
                                int max_iter, const char* who);
 // The mixed solve's FP32 element passes on MFMA tiles (systems with
@@ -334,9 +334,9 @@ const int* tree_perm (const sx_msys* s);
 // a system run the split band sweeps where its band layout has them, as the
 // systems of batches always did (SX_BAND_SPLIT=0 turns split sweeps off and
 // so gives the dissection, what the batch records).  The first such solve
-// builds the band factor; under capture, or where that fails, it is the
-// dissection.
-bool by_tree (const sx_msys* s, hipStream_t st);
+// builds the band factor (build; not for a caller that may not allocate);
+// under capture, or where that fails, it is the dissection.
+bool by_tree (const sx_msys* s, hipStream_t st, bool build = true);
 struct RhsTo { double* p; int ld; const int* perm; };
 inline RhsTo rhs_in (const sx_msys* s, bool tree)
 {

@@ -335,7 +335,7 @@ __global__ void k_assemble_m (int nglobal, const int* __restrict__ gptr,
 }
 
 int inner_solve (sx_msys* s, int nz, int stride, const double* X, double* Fp,
-                 double* V, const double* lines, hipStream_t st)
+                 double* V, const double* lines, hipStream_t st, bool build = true)
 {
   const sx_mesh* m = s->m;
   const int npl = (s->base_mode == 0 && nz > 1) ? nz - 1 : nz;
@@ -346,7 +346,7 @@ int inner_solve (sx_msys* s, int nz, int stride, const double* X, double* Fp,
     hipLaunchKernelGGL (k_condense32, dim3 (m->nel, npl), dim3 (64), 0, st, m->np, m->nclass,
                         m->d_emap, m->d_cls, s->d_Bm32, X, Fp, stride, nz, s->base_mode);
   }
-  const bool tree = by_tree (s, st);
+  const bool tree = by_tree (s, st, build);
   const RhsTo to = rhs_in (s, tree);
   hipLaunchKernelGGL (k_assemble_m, dim3 ((m->nglobal + 255) / 256, npl), dim3 (256), 0, st,
                       m->nglobal, m->d_gptr, m->d_gsrc, m->d_nptr, m->d_nidx, m->d_nw, Fp,
@@ -541,7 +541,7 @@ size_t mixed_work_doubles (const sx_msys* s, int nz, int stride)
 // later, so the workspace needs no clearing.
 int field_solve_mixed_ws (sx_msys* s, int nz, int stride, double* d_f, double* d_u,
                           const double* d_lines, double refine_tol, int max_iter, int* iters,
-                          double* work, hipStream_t st)
+                          double* work, hipStream_t st, bool build)
 {
   const sx_mesh* m = s->m;
   const int npl = (s->base_mode == 0 && nz > 1) ? nz - 1 : nz;
@@ -557,7 +557,7 @@ int field_solve_mixed_ws (sx_msys* s, int nz, int stride, double* d_f, double* d
                       s->d_betak2, m->d_geo, m->d_D, m->d_emap, m->d_btog, m->d_emask, s->d_G,
                       m->nglobal, d_f, W, stride, nz, s->base_mode);
   SX_HIP (hipGetLastError ());
-  int rc = inner_solve (s, nz, stride, W, Fp, V, lines, st);
+  int rc = inner_solve (s, nz, stride, W, Fp, V, lines, st, build);
   if (rc) return rc;
   const int n_plane = m->nel * m->npnp;
   double hp[2 * MIXED_NBLK];
@@ -567,7 +567,7 @@ int field_solve_mixed_ws (sx_msys* s, int nz, int stride, double* d_f, double* d
                         s->lambda2, s->d_betak2, m->d_geo, m->d_D, W, V, X, stride, nz,
                         s->base_mode);
     SX_HIP (hipGetLastError ());
-    if ((rc = inner_solve (s, nz, stride, X, Fp, dV, lines, st))) return rc;
+    if ((rc = inner_solve (s, nz, stride, X, Fp, dV, lines, st, build))) return rc;
     hipLaunchKernelGGL (k_norms, dim3 (MIXED_NBLK), dim3 (256), 0, st, V, dV, npl, nz,
                         s->base_mode, n_plane, stride, part);
     hipLaunchKernelGGL (k_axpy_planes, dim3 ((unsigned) (((size_t) npl * n_plane + 255) / 256)),

@@ -69,5 +69,5 @@ extern "C" int sx_field_solve_mixed_noalloc (sx_msys_t s, int nz, int stride, do
   double* work = device_scratch ();
   if (!work) return SX_ERR_HIP;
   return field_solve_mixed_ws (s, nz, stride, d_f, d_u, d_lines, refine_tol, max_iter, iters,
-                               work, (hipStream_t) stream);
+                               work, (hipStream_t) stream, false);
 }

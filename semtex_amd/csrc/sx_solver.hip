@@ -1878,12 +1878,13 @@ static int own_band (sx_msys* s, hipStream_t st)
   return rc ? rc : (int) SX_ERR_FACTOR;
 }
 
-bool by_tree (const sx_msys* s, hipStream_t st)
+bool by_tree (const sx_msys* s, hipStream_t st, bool build)
 {
   if (!s->tree || !s->held || s->no_split) return s->tree != nullptr;
   const char* e = std::getenv ("SX_BAND_SPLIT");
   if (e && std::atoi (e) == 0) return true;
   if (!s->own_band) {
+    if (!build) return true;
     hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing (st, &c) != hipSuccess) { (void) hipGetLastError (); return true; }
     if (c != hipStreamCaptureStatusNone) return true;

@@ -5,6 +5,8 @@
 // runs on it.
 #include <hip/hip_runtime.h>
 
+#include "../include/semtex_amd.h"
+
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -90,7 +92,12 @@ hipError_t hipGetLastError () { hipError_t e = last; last = hipSuccess; return e
 hipError_t hipFuncSetAttribute (const void*, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipFuncGetAttributes (hipFuncAttributes* a, const void*) { std::memset (a, 0, sizeof *a); return hipSuccess; }
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor (int* n, const void*, int, size_t) { *n = 1; return hipSuccess; }
-hipError_t hipGetSymbolAddress (void** p, const void*) { *p = nullptr; return hipErrorInvalidSymbol; }
+hipError_t hipGetSymbolAddress (void** p, const void*)   // (the library has one device array)
+{
+  static void* a = std::calloc (SX_NOALLOC_DOUBLES, 8);
+  *p = a;
+  return hipSuccess;
+}
 
 hipError_t hipStreamCreate (hipStream_t* s) { *s = (hipStream_t) std::malloc (1); return hipSuccess; }
 hipError_t hipStreamDestroy (hipStream_t s) { std::free ((void*) s); return hipSuccess; }

@@ -319,3 +319,24 @@ def test_block_that_may_be_in_use_is_not_kept():
     assert S.stub_live() == 0
     print("ok")
     """)
+
+
+def test_noalloc_solve_of_a_held_system_allocates_nothing():
+    """sx_field_solve_mixed_noalloc on a system a batch holds, before any
+    other solve of it: no allocation, the dissection."""
+    run("""
+    g = GpuMesh(rect_mesh(16, 12, 8, 0.0, 6.0, -1.0, 1.0, bc=("D", "N", "D", "N"), periodic_x=True))
+    M = ModalMatrixSys(1.0, 1.0, 0, 1, g, precision=_lib.SX_MIXED)
+    B = RawBatch([M])
+    assert B.create() == 0
+    b = [Buf(M.gmesh.plane_size) for _ in range(2)]
+    S.stub_fail(0, 0)
+    it = C.c_int()
+    assert L.sx_field_solve_mixed_noalloc(M.handle, 1, M.gmesh.plane_size, b[0].p, b[1].p, None, 1e-6, 2,
+                                          C.byref(it), None) == 0
+    assert S.stub_allocs() == 0 and M.layout()["kernel"] == 4
+    assert L.sx_field_solve_mixed(M.handle, 1, M.gmesh.plane_size, b[0].p, b[1].p, None, 1e-6, 2,
+                                  C.byref(it), None) == 0
+    assert M.layout()["kernel"] == 3
+    print("ok")
+    """)
