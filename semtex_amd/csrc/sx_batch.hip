@@ -50,6 +50,14 @@ struct sx_batch {
   std::vector<std::array<int, 3>> keys;  // class keys: sw_D, sw_unit, tw
   std::vector<int> per;                // right-hand sides per sweep workgroup, per class (0: default)
   void* d_plan = nullptr;              // the merged launches' arguments and grids
+  // workspace of every mixed system, for the largest of its problems
+  std::vector<std::pair<const sx_msys*, double*>> work;
+  double* work_of (const sx_msys* s) const
+  {
+    for (auto& w : work)
+      if (w.first == s) return w.second;
+    return nullptr;
+  }
 };
 
 extern "C" int sx_batch_destroy (sx_batch_t b)
@@ -64,6 +72,7 @@ extern "C" int sx_batch_destroy (sx_batch_t b)
   if (b->fork) (void) hipEventDestroy (b->fork);
   if (b->cap) (void) hipStreamDestroy (b->cap);
   if (b->d_plan) (void) hipFree (b->d_plan);
+  for (auto& w : b->work) (void) hipFree (w.second);
   delete b;
   return SX_OK;
 }
@@ -88,7 +97,8 @@ static int record (const sx_batch* b, int n, const sx_msys_t* sys, const int* nz
     const double* li = lines ? lines[i] : nullptr;
     int rc;
     if (sys[i]->precision == SX_MIXED)
-      rc = field_solve_mixed_passes (sys[i], nz[i], stride[i], f_work[i], u[i], li, passes, ls);
+      rc = field_solve_mixed_passes (sys[i], nz[i], stride[i], f_work[i], u[i], li, passes,
+                                     b->work_of (sys[i]), ls);
     else
       rc = sx_field_solve (sys[i], nz[i], stride[i], f_work[i], u[i], li, ls);
     if (rc) return rc;
@@ -143,7 +153,7 @@ int fused_plan (const sx_batch* b, BatchPlan& P)
     P.tune = b->per[b->cls[i]];
     const int rc = s->precision == SX_MIXED
         ? plan_mixed_passes (P, b->sys[i], b->nz[i], b->stride[i], b->fwork[i], b->u[i],
-                             b->lines[i], b->passes)
+                             b->lines[i], b->passes, b->work_of (s))
         : plan_field_solve_direct (P, s, b->nz[i], b->stride[i], b->fwork[i], b->u[i],
                                    b->lines[i]);
     if (rc) return rc;
@@ -275,6 +285,17 @@ extern "C" int sx_batch_create (int n, const sx_msys_t* systems, const int* nz,
   };
   for (int i = 0; i < n; i++)
     if (int rc = msys_hold (systems[i], held[i])) return fail (rc);
+  for (int i = 0; i < n; i++) {
+    if (systems[i]->precision != SX_MIXED || b->work_of (systems[i])) continue;
+    size_t need = 0;
+    for (int j = i; j < n; j++)
+      if (systems[j] == systems[i])
+        need = std::max (need, mixed_work_doubles (systems[j], nz[j], plane_stride[j]));
+    double* w = nullptr;
+    const hipError_t e = dev_malloc (&w, sizeof (double) * need);
+    if (e != hipSuccess) return fail (hip_fail (e, "hipMalloc"));
+    b->work.emplace_back (systems[i], w);
+  }
   if (hipStreamCreate (&b->cap) != hipSuccess) return fail (hip_fail (hipErrorUnknown, "hipStreamCreate"));
   // lanes: 4, as many as the hardware queues a process gets by default
   // (measured: 4 lanes 2.9 ms FP64 / 7.4 ms mixed per 64-problem batch, 8

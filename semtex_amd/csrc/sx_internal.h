@@ -171,7 +171,8 @@ int    fourier_z_fused_batch (int nz, int S, int nb, const double* const* in,
 // Mixed-precision solve with a fixed number of refinement passes, no host
 // synchronisation (sx_mixed.hip).
 int    field_solve_mixed_passes (sx_msys* s, int nz, int stride, double* d_f, double* d_u,
-                                 const double* d_lines, int passes, hipStream_t st);
+                                 const double* d_lines, int passes, double* work,
+                                 hipStream_t st);
 // The tolerance-driven mixed solve (sx_field_solve_mixed) on a workspace of
 // at least mixed_work_doubles() doubles that the caller provides; the
 // argument check shared by its entry points.
@@ -473,7 +474,7 @@ int plan_tree_solve (BatchPlan& P, const sx_msys* s);
 int plan_sing_keep (BatchPlan& P, const sx_msys* s);
 int plan_sing_refine (BatchPlan& P, const sx_msys* s);
 int plan_mixed_passes (BatchPlan& P, sx_msys* s, int nz, int stride, double* d_f,
-                       double* d_u, const double* d_lines, int passes);
+                       double* d_u, const double* d_lines, int passes, double* work);
 int plan_condense32_tiled (BatchPlan& P, const sx_msys* s, int nz, int stride, const double* X,
                            double* Fp);
 int plan_recover32_tiled (BatchPlan& P, const sx_msys* s, int nz, int stride, const double* Fp,

@@ -427,23 +427,15 @@ int plan_inner (BatchPlan& P, sx_msys* s, int nz, int stride, const double* X, d
 
 namespace sx {
 
-// field_solve_mixed_passes, recorded for a fused batch; the system's
-// workspace is allocated here (planning is set-up, not the replayed work)
+// field_solve_mixed_passes, recorded for a fused batch (work: at least
+// mixed_work_doubles(), the batch's own)
 int plan_mixed_passes (BatchPlan& P, sx_msys* s, int nz, int stride, double* d_f, double* d_u,
-                       const double* d_lines, int passes)
+                       const double* d_lines, int passes, double* work)
 {
   const sx_mesh* m = s->m;
   const int npl = (s->base_mode == 0 && nz > 1) ? nz - 1 : nz;
   const size_t nplane = (size_t) nz * stride;
-  const size_t need = mixed_work_doubles (s, nz, stride);
-  if (s->work_doubles < need) {
-    if (s->d_work) (void) hipFree (s->d_work);
-    s->d_work = nullptr;
-    s->work_doubles = 0;
-    SX_HIP (dev_malloc (&s->d_work, sizeof (double) * need));
-    s->work_doubles = need;
-  }
-  double *W = s->d_work, *X = W + nplane, *Fp = X + nplane, *V = Fp + nplane,
+  double *W = work, *X = W + nplane, *Fp = X + nplane, *V = Fp + nplane,
          *dV = V + nplane;
   const int lstride = m->nbound * m->np;
   const double* lines = (d_lines && m->nbound) ? d_lines : (const double*) nullptr;
@@ -480,22 +472,16 @@ int plan_mixed_passes (BatchPlan& P, sx_msys* s, int nz, int stride, double* d_f
 
 // The mixed solve with a fixed number of refinement passes and no host
 // synchronisation (graph capture): the first pass is the FP32-condensed
-// solve, each further pass adds the solve of the FP64 residual.
+// solve, each further pass adds the solve of the FP64 residual.  work: at
+// least mixed_work_doubles(), the batch's own -- the system's grows with a
+// later solve of more planes, under a graph that was recorded with it.
 int field_solve_mixed_passes (sx_msys* s, int nz, int stride, double* d_f, double* d_u,
-                              const double* d_lines, int passes, hipStream_t st)
+                              const double* d_lines, int passes, double* work, hipStream_t st)
 {
   const sx_mesh* m = s->m;
   const int npl = (s->base_mode == 0 && nz > 1) ? nz - 1 : nz;
   const size_t nplane = (size_t) nz * stride;
-  const size_t need = mixed_work_doubles (s, nz, stride);
-  if (s->work_doubles < need) {
-    if (s->d_work) (void) hipFree (s->d_work);
-    s->d_work = nullptr;
-    s->work_doubles = 0;
-    SX_HIP (dev_malloc (&s->d_work, sizeof (double) * need));
-    s->work_doubles = need;
-  }
-  double *W = s->d_work, *X = W + nplane, *Fp = X + nplane, *V = Fp + nplane,
+  double *W = work, *X = W + nplane, *Fp = X + nplane, *V = Fp + nplane,
          *dV = V + nplane;
   const int lstride = m->nbound * m->np;
   const double* lines = (d_lines && m->nbound) ? d_lines : nullptr;

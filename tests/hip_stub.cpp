@@ -18,7 +18,7 @@ std::mutex mu;
 std::map<void*, size_t> live;               // device and pinned allocations
 std::map<const void*, std::string> names;   // kernel stub -> device name
 std::map<std::string, long> launched;
-long allocs = 0, fail_at = -1, fail_to = -1, device = 0, bad = 0;
+long allocs = 0, fail_at = -1, fail_to = -1, device = 0, bad = 0, freed = 0;
 bool sync_fails = false;
 size_t limit = 0;                           // bytes on the "device" (0: no limit)
 hipError_t last = hipSuccess;
@@ -45,6 +45,7 @@ hipError_t release (void* p)
   std::lock_guard<std::mutex> lock (mu);
   if (!p) return hipSuccess;
   if (!live.erase (p)) { std::abort (); }   // not an allocation, or freed twice
+  freed++;
   std::free (p);
   return hipSuccess;
 }
@@ -58,6 +59,7 @@ void stub_limit (size_t bytes) { limit = bytes; }
 void stub_device (long d) { device = d; }
 void stub_sync_fails (int on) { sync_fails = on != 0; }
 long stub_allocs () { return allocs; }
+long stub_freed () { return freed; }
 long stub_live () { return (long) live.size (); }
 size_t stub_bytes () { size_t n = 0; for (auto& a : live) n += a.second; return n; }
 long stub_launches (const char* part)

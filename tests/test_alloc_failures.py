@@ -27,7 +27,7 @@ PRELUDE = textwrap.dedent("""
     S = C.CDLL(os.environ["LD_PRELOAD"])
     S.stub_bytes.restype = C.c_size_t
     S.stub_limit.argtypes = [C.c_size_t]
-    for f in ("stub_allocs", "stub_live", "stub_launches", "stub_bad_pointers"): getattr(S, f).restype = C.c_long
+    for f in ("stub_allocs", "stub_live", "stub_launches", "stub_bad_pointers", "stub_freed"): getattr(S, f).restype = C.c_long
     S.stub_fail.argtypes = [C.c_long, C.c_long]
     S.stub_device.argtypes = [C.c_long]
     launches = lambda name: S.stub_launches(name.encode())
@@ -51,9 +51,10 @@ PRELUDE = textwrap.dedent("""
     class RawBatch:
         def __init__(self, Ms, nz=1):
             n = len(Ms)
-            self.bufs = [[Buf(nz * M.gmesh.plane_size) for _ in range(3)] for M in Ms]
+            nz = [nz] * n if isinstance(nz, int) else nz
+            self.bufs = [[Buf(z * M.gmesh.plane_size) for _ in range(3)] for M, z in zip(Ms, nz)]
             pp = lambda j: (C.c_void_p * n)(*[b[j].p for b in self.bufs])
-            self.args = (n, (C.c_void_p * n)(*[M.handle for M in Ms]), (C.c_int * n)(*[nz] * n),
+            self.args = (n, (C.c_void_p * n)(*[M.handle for M in Ms]), (C.c_int * n)(*nz),
                          (C.c_int * n)(*[M.gmesh.plane_size for M in Ms]), pp(0), pp(1), pp(2), None, 1)
             self.h = None
         def create(self):
@@ -338,5 +339,33 @@ def test_noalloc_solve_of_a_held_system_allocates_nothing():
     assert L.sx_field_solve_mixed(M.handle, 1, M.gmesh.plane_size, b[0].p, b[1].p, None, 1e-6, 2,
                                   C.byref(it), None) == 0
     assert M.layout()["kernel"] == 3
+    print("ok")
+    """)
+
+
+@pytest.mark.parametrize("fused", ["1", "0"])
+def test_mixed_batch_keeps_the_workspace_its_graph_records(fused):
+    """Problems of one mixed system with different plane counts, and a later
+    solve of more planes on it: no workspace that the graph holds is freed."""
+    run(f"""
+    os.environ["SX_BATCH_FUSED"] = "{fused}"
+    g = GpuMesh(rect_mesh(6, 4, 6, 0.0, 6.0, -1.0, 1.0, bc=("D", "N", "D", "N"), periodic_x=True))
+    freed = []
+    for nz in ([2, 8], [8, 2]):
+        M = ModalMatrixSys(1.0, 1.0, 0, 4, g, precision=_lib.SX_MIXED)
+        B = RawBatch([M, M], nz)
+        n = S.stub_freed()
+        assert B.create() == 0
+        freed.append(S.stub_freed() - n)
+        b = [Buf(8 * M.gmesh.plane_size) for _ in range(2)]
+        n = S.stub_freed()
+        assert L.sx_field_solve_mixed(M.handle, 8, M.gmesh.plane_size, b[0].p, b[1].p, None, 1e-6, 2,
+                                      None, None) == 0
+        assert S.stub_freed() == n
+        for x in b: x.free()
+        B.destroy(); B.free(); del M, B
+    assert freed[0] == freed[1], freed
+    del g
+    assert S.stub_live() == 0, S.stub_live()
     print("ok")
     """)
