@@ -1815,6 +1815,15 @@ static int condensed_again (const sx_msys* s, DevTmp& buf, double** S, int** d_s
                   d + nws + nS + nB, *d_status + s->nmodes, st);
 }
 
+// Whether a factorisation found every pivot positive (waits for it)
+static bool pivots_ok (const sx_msys* s, const int* d_status)
+{
+  std::vector<int> status (s->nmodes + 1, 1);
+  return hipMemcpy (status.data (), d_status, sizeof (int) * status.size (),
+                    hipMemcpyDeviceToHost) == hipSuccess &&
+         std::all_of (status.begin (), status.end (), [] (int e) { return e == 0; });
+}
+
 int msys_hold (sx_msys* s, Held& h)
 {
   h = Held {};
@@ -1829,6 +1838,11 @@ int msys_hold (sx_msys* s, Held& h)
     int rc = condensed_again (s, buf, &S, &d_status, nullptr);
     if (!rc) rc = tree_for_batch (s, S, nullptr, d_status, now);
     if (rc) return rc;
+    if (now.tree && !pivots_ok (s, d_status)) {
+      // (the matrix is the one the system was made with: its own cut serves)
+      for (double* p : {now.ops, now.tb, now.tv, now.tc}) (void) hipFree (p);
+      now = Held {};
+    }
     if (now.tree) {
       was.tree = s->tree;
       was.ops = s->d_tops; was.tb = s->d_tb; was.tv = s->d_tv; was.tc = s->d_tc;
@@ -1869,11 +1883,7 @@ static int own_band (sx_msys* s, hipStream_t st)
   int* d_status = nullptr;
   int rc = condensed_again (s, buf, &S, &d_status, st);
   if (!rc) rc = band_build (s, S, st, d_status);
-  std::vector<int> status (s->nmodes + 1, 1);
-  if (!rc && hipMemcpy (status.data (), d_status, sizeof (int) * status.size (),
-                        hipMemcpyDeviceToHost) == hipSuccess &&
-      std::all_of (status.begin (), status.end (), [] (int e) { return e == 0; }))
-    return SX_OK;
+  if (!rc && pivots_ok (s, d_status)) return SX_OK;
   band_drop (s);
   return rc ? rc : (int) SX_ERR_FACTOR;
 }

@@ -19,7 +19,7 @@ std::map<void*, size_t> live;               // device and pinned allocations
 std::map<const void*, std::string> names;   // kernel stub -> device name
 std::map<std::string, long> launched;
 long allocs = 0, fail_at = -1, fail_to = -1, device = 0, bad = 0, freed = 0;
-bool sync_fails = false;
+bool sync_fails = false, bad_pivots = false;
 size_t limit = 0;                           // bytes on the "device" (0: no limit)
 hipError_t last = hipSuccess;
 
@@ -57,6 +57,7 @@ extern "C" {
 void stub_fail (long first, long count) { allocs = 0; fail_at = first; fail_to = first + count; }
 void stub_limit (size_t bytes) { limit = bytes; }
 void stub_device (long d) { device = d; }
+void stub_bad_pivots (int on) { bad_pivots = on != 0; }
 void stub_sync_fails (int on) { sync_fails = on != 0; }
 long stub_allocs () { return allocs; }
 long stub_freed () { return freed; }
@@ -134,6 +135,7 @@ hipError_t hipLaunchKernel (const void* f, dim3, dim3, void** args, size_t, hipS
   std::lock_guard<std::mutex> lock (mu);
   const std::string& name = names[f];
   launched[name]++;
+  if (bad_pivots && name.find ("k_tree_panel") != std::string::npos) **(int**) args[7] = 1;
   for (auto& k : pointers)
     if (name.find (k.name) != std::string::npos)
       for (int i : k.at) {

@@ -369,3 +369,25 @@ def test_mixed_batch_keeps_the_workspace_its_graph_records(fused):
     assert S.stub_live() == 0, S.stub_live()
     print("ok")
     """)
+
+
+def test_batch_keeps_the_systems_cut_when_its_own_does_not_factor():
+    """A pivot that the batch's cut finds not positive leaves the system on the
+    cut it was made with; a new system still fails for it."""
+    run("""
+    g = GpuMesh(rect_mesh(16, 12, 6, 0.0, 6.0, -1.0, 1.0, bc=("D", "N", "D", "N"), periodic_x=True))
+    M, M2 = [ModalMatrixSys(1.0, 1.0, 0, 1, g) for _ in range(2)]
+    ops = M.layout()["operators"]
+    B, B2 = RawBatch([M]), RawBatch([M2])
+    S.stub_bad_pivots(1)
+    assert B.create() == 0 and M.layout()["operators"] == ops
+    try: ModalMatrixSys(1.0, 1.0, 0, 1, g)
+    except _lib.SxError as e: assert e.code == _lib.SX_ERR_FACTOR
+    else: assert 0
+    S.stub_bad_pivots(0)
+    assert B2.create() == 0 and M2.layout()["operators"] != ops
+    for x in (B, B2): x.destroy(); x.free()
+    del M, M2, g
+    assert S.stub_live() == 0
+    print("ok")
+    """)
