@@ -2730,7 +2730,7 @@ int band_solve (const sx_msys* s, bool tree, int nr, hipStream_t st, int moves)
 // back whose latency counts while few modes run, their panels' bytes with
 // many (past 128 modes a workgroup takes both right-hand sides).  The fit to
 // 320 traced solves (bands of 1 to 6 off-diagonal blocks, 48 to 512 modes),
-// within 20 %.  Offset-major sweeps: not worth comparing.
+// nine tenths of them within 17 %.  Offset-major sweeps: not worth comparing.
 double band_us (const sx_mesh* m, int nmodes)
 {
   if (!use_panels (m->nband, m->nsolve)) return 1e30;

@@ -216,7 +216,7 @@ void split_rows (int blocks, int pairs, long long tiles, bool batch, int* nrb, i
 // solve of these or of the band at 128 to 256 modes).  The terms, a launch
 // with one workgroup's chain, every workgroup, operators, gathers and
 // stores, are the fit to 2,400 traced launches (4x4 to 32x32 elements, N_P 4
-// to 12, uniform and graded): a solve within 15 % for nine tenths of them.
+// to 12, uniform and graded): a solve within 16 % for nine tenths of them.
 // (The fit is no better than the bytes up to 32 modes: it cut the 16x16
 // N_P=10 problem into 3 levels instead of 4, 152 us instead of 145.)
 constexpr int TREE_FEW_OPERATORS = 4096;
