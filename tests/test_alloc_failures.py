@@ -81,8 +81,8 @@ def run(body, **env):
     if not os.path.exists(STUB) or os.path.getmtime(STUB) < os.path.getmtime(SRC):
         os.makedirs(os.path.dirname(STUB), exist_ok=True)
         subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__",
-                        "-I/opt/rocm/include", SRC, "-o", STUB + ".tmp"], check=True)
-        os.replace(STUB + ".tmp", STUB)
+                        "-I/opt/rocm/include", SRC, "-o", f"{STUB}.{os.getpid()}"], check=True)
+        os.replace(f"{STUB}.{os.getpid()}", STUB)
     e = {k: v for k, v in os.environ.items() if not k.startswith("SX_")}
     e.update(LD_PRELOAD=STUB, PYTHONPATH=ROOT, **env)
     r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body)], env=e, cwd=ROOT,
